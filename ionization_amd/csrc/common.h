@@ -88,6 +88,25 @@ __device__ __forceinline__ int norm_health(const double* out_norm, int slot, dou
                                                                                           : 0;
 }
 
+// Sum over the 64 lanes of a wave in lane 63 (the other lanes hold partial sums): the row and
+// broadcast moves of the vector ALU, no LDS permutes. Every lane of the wave must take part.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    union { double d; int i[2]; } a, b;
+    a.d = v;
+    b.i[0] = __builtin_amdgcn_update_dpp(0, a.i[0], CTRL, ROWS, 0xf, true);
+    b.i[1] = __builtin_amdgcn_update_dpp(0, a.i[1], CTRL, ROWS, 0xf, true);
+    return v + b.d;
+}
+__device__ __forceinline__ double wave_sum_last(double v) {
+    v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+    v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+    v = dpp_add<0x118, 0xf>(v);  // row_shr:8: lane 15 of each row of 16 holds the row's sum
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
+
 // Sum over the 64 lanes of a wave; every lane gets the total.
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll

@@ -158,9 +158,22 @@ void free_bucket(Bucket& b) {
     b = Bucket{};
 }
 
-// l segments of at most kSegRows rows per L-phase wave, balanced in size.
-constexpr int kSegRows = kShSegRows;
-int sh_segments(int L) { return (L + kSegRows - 1) / kSegRows; }
+// Norm partials along l of one simulation (kShPartRows rows each).
+int sh_parts(int L) { return (L + kShPartRows - 1) / kShPartRows; }
+
+// Rows of an L-phase wave's l-segment: the most (up to kShSegRows) that still give the batch
+// kMinLWaves waves, about four for each SIMD. A wave walks its rows one pair after another, so a
+// small batch's L-phase takes as long as one segment: 64-row segments left one 250 x 100 mesh with
+// 8 waves (38.0 us per step, 28 us of it the L-phase; 8-row segments 19.9), one 200 x 1000 mesh with
+// 64 (51.3 -> 30.7). Long segments re-read fewer halo rows (7 per segment); on 32 simulations of
+// 15 M points 8 / 16 / 32 / 64 rows measured 270 / 260 / 267 / 267 us per step.
+// `columns` counts, for every live simulation, its 64-position columns times its partials along l.
+constexpr int64_t kMinLWaves = 4096;
+int sh_segment_rows(int64_t columns) {
+    int rows = kShSegRows;
+    while (rows > kShPartRows && columns * kShPartRows / rows < kMinLWaves) rows /= 2;
+    return rows;
+}
 
 int n_data_points(int N, int every) {
     if (every >= 1) return N / every + 1 + ((N % every) != 0 ? 1 : 0);
@@ -269,18 +282,23 @@ int rebuild_tables(tdse_ctx* ctx) {
     std::vector<int2> adw;                                      // ADI position waves (Thomas l-sweep)
     std::map<std::pair<int, int>, std::vector<int2>> alb;       // ADI position groups (partition l-sweep), (rows, 0)
     ctx->sh_norm_by_l = false;
+    int64_t columns = 0;
+    for (const ShHost& h : ctx->sh)
+        if (h.live) columns += (int64_t)(h.dev.npad / TDSE_WAVE) * sh_parts(h.dev.L);
+    const int seg_parts = sh_segment_rows(columns) / kShPartRows;
     for (int pass = 0; pass < 2; ++pass)
     for (int s = 0; s < (int)ctx->sh.size(); ++s) {
         ShHost& h = ctx->sh[s];
         if (!h.live || (int)h.vel != pass) continue;
         if (pass == 1 && ctx->n_len_waves < 0) ctx->n_len_waves = (int)waves.size();
         h.wave_first = (int)waves.size();
-        const int nseg = sh_segments(h.dev.L);
-        const int seg = (h.dev.L + nseg - 1) / nseg;
+        const int parts = sh_parts(h.dev.L);
+        const int nseg = (parts + seg_parts - 1) / seg_parts;
+        const int seg = (parts + nseg - 1) / nseg * kShPartRows;  // balanced, whole partials
         const int wpl = h.dev.npad / TDSE_WAVE;
-        for (int sg = 0; sg < nseg; ++sg) {
-            const int lo = sg * seg, hi = std::min(h.dev.L, lo + seg);
-            for (int w = 0; w < wpl; ++w) waves.push_back(ShWave{s, w * TDSE_WAVE, lo, hi, sg * wpl + w});
+        for (int lo = 0; lo < h.dev.L; lo += seg) {
+            const int hi = std::min(h.dev.L, lo + seg);
+            for (int w = 0; w < wpl; ++w) waves.push_back(ShWave{s, w * TDSE_WAVE, lo, hi});
         }
         h.wave_count = (int)waves.size() - h.wave_first;
         jobs.push_back(make_int2(s, -1));
@@ -1112,7 +1130,7 @@ int tdse_sh_add(tdse_ctx* ctx, const tdse_sh_desc* desc, const double* tables, c
     S.store_every = D.store_every;
     S.LB = D.lb;
     S.n_basis = D.n_basis;
-    S.nwaves = (S.npad / TDSE_WAVE) * sh_segments(S.L);
+    S.n_part = (S.npad / TDSE_WAVE) * sh_parts(S.L);
     S.norm_by_l = D.norm_by_l ? 1 : 0;
     S.corr0 = D.corr0;
     S.delta_r = D.delta_r;
@@ -1136,14 +1154,14 @@ int tdse_sh_add(tdse_ctx* ctx, const tdse_sh_desc* desc, const double* tables, c
         (H.adi && (rc = copy_to_device(ctx, H.blocks, fs, (size_t)S.N, &dfa))) ||
         (rc = copy_to_device(ctx, H.blocks, ts, (size_t)S.N, &dts)) ||
         (rc = copy_to_device<double2>(ctx, H.blocks, nullptr, (size_t)S.LB * npad, &snap)) ||
-        (rc = copy_to_device<double>(ctx, H.blocks, nullptr, 2 * (size_t)S.nwaves, &part)) ||
+        (rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)S.n_part + S.npad / TDSE_WAVE, &part)) ||
         (rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)H.n_data, &on)) ||
         (rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)H.n_data, &oln)) ||
         (rc = copy_to_device<double2>(ctx, H.blocks, nullptr, (size_t)H.n_data * std::max(1, S.n_basis), &oip)) ||
         (S.n_basis > 0 && ((rc = copy_to_device(ctx, H.blocks, basis, (size_t)S.n_basis * npad, &bas)) ||
                            (rc = copy_to_device(ctx, H.blocks, basis_l, (size_t)S.n_basis, &bl)))) ||
         (S.norm_by_l &&
-         ((rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)S.nwaves * kShSegRows, &pl)) ||
+         ((rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)S.L * (S.npad / TDSE_WAVE), &pl)) ||
           (rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)H.n_data * S.L, &onl))))) {
         (void)hipStreamSynchronize(ctx->stream);
         free_blocks(ctx, H.blocks);

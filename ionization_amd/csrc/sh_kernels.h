@@ -34,11 +34,11 @@ struct ShSim {
     const double* fs;      // [N] field times tau ratio per step: E(t_{n+1}+dt/2) * tau_n / tau0
     const double* ts;      // [N] tau_n / tau0
     double2* snap;         // [LB][npad] rows l < LB captured at data steps
-    double* part;          // [2][nwaves] per-wave partial |g|^2 sums (all l, largest l); nwaves counts L-phase waves
+    double* part;          // [n_part] |g|^2 sums of kShPartRows l-rows x 64 positions, then [npad / 64] of the largest l
     double* out_norm;      // [n_data]
     double* out_lnorm;     // [n_data]
     double2* out_ip;       // [n_data][n_basis]
-    double* part_l;        // [nwaves][kShSegRows] per-wave |g|^2 sums of each row (norm by l), or null
+    double* part_l;        // [L][npad / 64] |g|^2 sums of each row over 64 positions (norm by l), or null
     double* out_nl;        // [n_data][L] norm in each l, or null
     const double* basis;   // [n_basis][npad] radial g of each test state, position order
     const int* basis_l;    // [n_basis]
@@ -46,7 +46,7 @@ struct ShSim {
     double corr0;          // tau0 * (-2 P_r) * dr (1 + dr) / 8, added at l = 0, j = 0
     double delta_r;
     double cu;             // tau0 hbar^2 / (2 mu): U_j = cu / r_j^2, r_j = (j + 1/2) delta_r
-    int n, L, P, m, npad, N, store_every, LB, n_basis, nwaves;
+    int n, L, P, m, npad, N, store_every, LB, n_basis, n_part;
     int step;              // steps already advanced; device-updated
     int active;
     int phase;             // 0: g is mid-step (after the R-phase); 1: g is the reference g after `step` steps
@@ -59,6 +59,9 @@ struct ShSim {
 };
 
 constexpr int kShSegRows = 64;  // most rows of one L-phase wave (its l-segment)
+// Rows of one norm partial. Segments are whole numbers of these, so the partials, and with them
+// the stored norms, do not depend on how many rows the L-phase gives a wave in a given batch.
+constexpr int kShPartRows = 8;
 
 enum { SH_T = 0, SH_U = 1, SH_AP = 2, SH_AN = 3, SH_RQ = 4, SH_MASK = 5, SH_NTAB = 6 };
 // velocity-gauge simulations carry one more row: tau0 hbar q / (2 m dr) alpha_j, zero for j >= n - 1
@@ -117,27 +120,30 @@ __device__ __forceinline__ void sh_rotate(double a, double2& x0, double2& x1) {
 // ------------------------------------------------------------------ L-phase
 //
 // A wave covers 64 consecutive positions of one simulation and one segment
-// [lo, hi) of its l range (wave table entry: sim, first position, lo, hi).
-// Each lane streams over l carrying a three-stage pipeline: virtual row
-// v = l + q (q = parity of j*L) puts the E-pairs on even v and the O-pairs on
-// odd v for every lane, so iteration it consumes rows (2it, 2it+1) and
-// finishes rows (2it-3, 2it-2). A finished row depends on input rows within
+// [lo, hi) of its l range (wave table entry: sim, first position, lo, hi; lo a
+// multiple of kShPartRows, hi too unless it is L). Each lane streams over l
+// carrying a three-stage pipeline: virtual row v = l + q (q = parity of j*L)
+// puts the E-pairs on even v and the O-pairs on odd v for every lane, so
+// iteration it consumes rows (2it, 2it+1) and finishes rows (2it-3, 2it-2). A finished row depends on input rows within
 // distance 3 (O, E, O pair chains), so a segment starts its pipeline 4 rows
 // below lo and stores only rows in [lo, hi); segments let short and long l
 // ranges spread evenly over the GPU. Row loads are issued PF iterations ahead.
+// The host picks the segment length by the size of the batch (sh_segment_rows).
 //
 // Mode per simulation, from its step counter n (N = total steps) and phase:
 //   start      E_n, O_n                          (n < N)
 //   end        O_{n-1}, E_{n-1}, mask            (n > 0 and g is mid-step)
 // At data times the reference g after n steps (between "end" and "start")
-// is observed: per-wave |g|^2 partials and the rows l < LB. Elsewhere the two
+// is observed: |g|^2 partials of kShPartRows rows and the rows l < LB. A pair
+// that straddles two segments is observed by the wave that holds its first row,
+// so every pair takes the same arithmetic whatever the segments. Elsewhere the two
 // E rotations of a pair, which share the generator sigma_x and commute with
 // the mask (a function of r only), are applied as one rotation by the sum of
 // their angles. end_only != 0 materialises the reference g after n steps for
 // the listed waves without starting step n and without observing; it too
 // writes sh_state(S, n + 1) (the host then swaps the two buffers).
 struct ShWave {
-    int sim, p0, lo, hi, part;  // part: index of this wave's norm partial within the simulation
+    int sim, p0, lo, hi;
 };
 
 // BY_L: the instance that can also reduce the norm in every l (launched only
@@ -173,10 +179,12 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
     const int LB = S.LB;
     double2* __restrict__ const snap = S.snap;
     double* __restrict__ const part_l = S.part_l;
+    double* __restrict__ const part = S.part;
     const int p = wt.p0 + lane;
     const int j = (p % P) * m + p / P;
     const bool live = j < S.n;
-    const int q = (j & 1) & (L & 1);  // parity of j*L
+    // parity of j*L, the same in every lane: m is even and a wave lies in one row-block of positions
+    const int q = __builtin_amdgcn_readfirstlane((j & 1) & (L & 1));
     const double rq = ld1(S.tab, SH_RQ * npad + p);
     const double mk = ld1(S.tab, SH_MASK * npad + p);
     const double f_end = do_end ? ld1(S.fs, n - 1) * rq : 0.0;
@@ -201,19 +209,14 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
     };
 
     // first iteration: rows below lo - 4 do not influence rows >= lo
-    // Rows of one lane's iteration depend on its parity q, so with odd L the
-    // lanes of a wave may have different bounds. Reducing the norm of every
-    // row across the wave (norm by l) needs the same bounds for all lanes: the
-    // union is used then (an earlier start or later end only adds pipeline
-    // warm-up / run-out on rows that are not stored).
     const bool by_l = BY_L && observe && S.norm_by_l;
-    const int it0 = (lo <= 4) ? 0 : ((lo + (by_l ? 0 : q) - 4) >> 1);
-    const int it_end = (hi - 1 + (by_l ? 1 : q) + 3) >> 1;  // last iteration stores row hi-1
+    const int it0 = (lo <= 4) ? 0 : ((lo + q - 4) >> 1);
+    const int it_end = (hi - 1 + q + 3) >> 1;  // last iteration stores row hi-1
+    const int wpl = npad / TDSE_WAVE, wcol = wt.p0 / TDSE_WAVE;
     const double2 zero = make_double2(0.0, 0.0);
     double2 carry_u = zero, carry_s1 = zero, carry_s3 = zero;
     double c_m3 = load_c(2 * it0 - 3), c_m2 = load_c(2 * it0 - 2), c_m1 = load_c(2 * it0 - 1);
     double acc_norm = 0.0, acc_lnorm = 0.0;
-    double pend = 0.0;  // norm by l: the q = 0 lanes' share of odd row v0 - 1, completed next iteration
     double2 ring0[PF], ring1[PF];
     double ringc0[PF], ringc1[PF];
 #pragma unroll
@@ -254,11 +257,9 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
         } else {
             // At a data time the stored rows are the same as elsewhere (one rotation when both halves
             // apply), and the pair's norm is that of the rotated rows (E_start keeps it). Rows observed
-            // on their own -- below LB (snapshots for the inner products), the largest l, rows outside
-            // [lo, hi) (counted by the neighbouring segment), every row for the norm by l -- take E_end
-            // and the mask once more by themselves.
-            // decided for the whole wave (lanes differ only by the parity q): no divergent rotations
-            const bool per_row = __any(!both || le < LB || le < lo || le + 1 >= hi || le + 1 >= L - 1);
+            // on their own -- below LB (snapshots for the inner products), the largest l, every row for
+            // the norm by l -- take E_end and the mask once more by themselves.
+            const bool per_row = !both || le < LB || le + 1 >= L - 1;
             double2 oa = s2a, ob = s2b;  // the observed rows: g after step n
             if (both) {
                 if (by_l || per_row) {
@@ -276,36 +277,38 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
                 oa = s2a;
                 ob = s2b;
             }
-            if (observe && live) {
-                if (!per_row) {
-                    acc_norm += cabs2(s2a) + cabs2(s2b);
-                } else {
-                    if (le >= lo && le < hi) {
-                        acc_norm += cabs2(oa);
-                        if (le == L - 1) acc_lnorm += cabs2(oa);
-                        if (le < LB) st2(snap, (size_t)le * npad + p, oa);
-                    }
-                    if (le + 1 >= lo && le + 1 < hi) {
-                        acc_norm += cabs2(ob);
-                        if (le + 1 == L - 1) acc_lnorm += cabs2(ob);
+            // the wave that holds the pair's first row observes it (row 0 alone, le = -1, is the first wave's)
+            const int first = max(le, 0);
+            if (observe && le >= -1 && first >= lo && first < hi && le < L) {
+                if (live) {
+                    if (!per_row) {
+                        acc_norm += cabs2(s2a) + cabs2(s2b);
+                    } else {
+                        // rows -1 and L are zero
+                        acc_norm += cabs2(oa) + cabs2(ob);
+                        if (le == L - 1) acc_lnorm = cabs2(oa);
+                        if (le + 1 == L - 1) acc_lnorm = cabs2(ob);
+                        if (le >= 0 && le < LB) st2(snap, (size_t)le * npad + p, oa);
                         if (le + 1 < LB) st2(snap, (size_t)(le + 1) * npad + p, ob);
                     }
                 }
+                const bool last = le + 2 >= L;
+                if (last || (le + 2) / kShPartRows != first / kShPartRows) {
+                    const double sum = wave_sum_last(acc_norm);
+                    if (lane == TDSE_WAVE - 1) part[(first / kShPartRows) * wpl + wcol] = sum;
+                    acc_norm = 0.0;
+                }
+                if (last) {
+                    const double sum = wave_sum_last(acc_lnorm);
+                    if (lane == TDSE_WAVE - 1) part[S.n_part + wcol] = sum;
+                }
             }
             if (by_l) {
-                // this iteration finishes rows v0-2 (all lanes), v0-1 (q = 0 lanes)
-                // and v0-3 (q = 1 lanes); sums in a fixed order per wave
-                const bool ok_a = live && le >= lo && le < hi, ok_b = live && le + 1 >= lo && le + 1 < hi;
-                const double na = ok_a ? cabs2(oa) : 0.0, nb = ok_b ? cabs2(ob) : 0.0;
-                const double r3 = wave_sum(q ? na : 0.0);  // row v0-3
-                const double r2 = wave_sum(q ? nb : na);   // row v0-2
-                const double r1 = wave_sum(q ? 0.0 : nb);  // row v0-1
-                if (lane == 0) {
-                    double* pl = part_l + (size_t)wt.part * kShSegRows;
-                    if (v0 - 3 >= lo && v0 - 3 < hi) pl[v0 - 3 - lo] = pend + r3;
-                    if (v0 - 2 >= lo && v0 - 2 < hi) pl[v0 - 2 - lo] = r2;
+                const double ra = wave_sum_last(live ? cabs2(oa) : 0.0), rb = wave_sum_last(live ? cabs2(ob) : 0.0);
+                if (lane == TDSE_WAVE - 1) {
+                    if (le >= lo && le < hi) part_l[(size_t)le * wpl + wcol] = ra;
+                    if (le + 1 >= lo && le + 1 < hi) part_l[(size_t)(le + 1) * wpl + wcol] = rb;
                 }
-                pend = r1;
             }
             if (!both && do_start) sh_rotate<VEL>(f_start * c_m2, s2a, s2b);
         }
@@ -323,15 +326,6 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
         c_m3 = c_m1;
         c_m2 = c0;
         c_m1 = c1;
-    }
-
-    if (observe) {
-        acc_norm = wave_sum(acc_norm);
-        acc_lnorm = wave_sum(acc_lnorm);
-        if (lane == 0) {
-            S.part[wt.part] = acc_norm;
-            S.part[S.nwaves + wt.part] = acc_lnorm;
-        }
     }
 }
 
@@ -355,25 +349,18 @@ __global__ void __launch_bounds__(256) k_sh_observe(ShSim* __restrict__ sims, co
     const int t = threadIdx.x;
     double re = 0.0, im = 0.0;
     if (jb.y == -2) {
-        // norm in every l: rows of l-segment sg sit in the partials of its waves
-        // sg * wpl .. sg * wpl + wpl - 1 (wave table order), summed in that order
-        const int L = S.L;
-        const int nseg = S.nwaves / (S.npad / TDSE_WAVE);
-        const int seg = (L + nseg - 1) / nseg;
-        const int wpl = S.npad / TDSE_WAVE;
+        // norm in every l: the row's partials in position order
+        const int L = S.L, wpl = S.npad / TDSE_WAVE;
         for (int l = t; l < L; l += blockDim.x) {
-            const int sg = l / seg, row = l - sg * seg;
             double acc = 0.0;
-            for (int w = 0; w < wpl; ++w) acc += ld1(S.part_l, (size_t)(sg * wpl + w) * kShSegRows + row);
+            for (int w = 0; w < wpl; ++w) acc += ld1(S.part_l, (size_t)l * wpl + w);
             S.out_nl[(size_t)slot * L + l] = acc * S.delta_r;
         }
         return;
     }
     if (jb.y < 0) {
-        for (int w = t; w < S.nwaves; w += blockDim.x) {
-            re += ld1(S.part, w);
-            im += ld1(S.part, S.nwaves + w);
-        }
+        for (int w = t; w < S.n_part; w += blockDim.x) re += ld1(S.part, w);
+        for (int w = t; w < S.npad / TDSE_WAVE; w += blockDim.x) im += ld1(S.part, S.n_part + w);
     } else {
         const double* phi = S.basis + (size_t)jb.y * S.npad;
         const double2* row = S.snap + (size_t)S.basis_l[jb.y] * S.npad;
