@@ -53,7 +53,9 @@ struct CylSim {
     int m_roots;  // smoothness = 2^m_roots: the root is m_roots square roots; -1 otherwise
     int nz, nr, Pz, Mz, npz, Cr, Mr, nrpad, lanes, n_groups;
     int N, store_every, n_basis;
-    int step;   // steps already advanced; device-updated
+    int step;   // steps already advanced; read by the z-sweep and the host, written by the rho-sweep
+    int rstep;  // the step under way: written by the z-sweep, read by the rho-sweep
+    int obs;    // time index whose observation partials are in `part`, or -1
     int active;
     int phase;  // 1: g is the reference g after `step` steps; 0: the explicit rho half of step `step` is applied
     int hold;   // 1: end every step at an exact state (phase 1)
@@ -108,6 +110,78 @@ __device__ __forceinline__ double cyl_mask_r(const CylSim& S, double r) {
     return pow(fabs(cs), S.m_inv_s);
 }
 
+// Job table entry (sim, b): b == -1 reduces the rho-sweep partials of a data time to the norm, b >= 0
+// to the inner product with test state b. One wave per job, sums in a fixed order. The partials of a
+// step are reduced by job waves in the leading workgroups of the next step's z-sweep launch (CylJobs), or
+// after the run's last step by a launch of their own. Job -3 rides with both sweeps and counts: the
+// z-sweep reads S.step, its job copies it to S.rstep; the rho-sweep reads S.rstep, its job sets S.step
+// for the next z-sweep. The two launches per step that this replaces took 8 us of the 23 us step of one
+// 250 x 100 mesh.
+struct CylJobs {
+    CylSim* sims;  // as ShObs
+    const int2* jobs;
+    int n_jobs;
+    int blocks;  // leading workgroups of the launch that take jobs, blockDim.x / 64 each
+};
+
+__device__ __forceinline__ void cyl_observe_job(CylSim& S, const int b, const int n, const int lane) {
+    const int slot = sh_data_slot(n, S.N, S.store_every);
+    const int stride = 1 + 2 * S.n_basis;
+    const int off = b < 0 ? 0 : 1 + 2 * b;
+    const double* __restrict__ part = S.part;
+    const int n_groups = S.n_groups;
+    double re = 0.0, im = 0.0;
+#pragma unroll 4
+    for (int g = lane; g < n_groups; g += TDSE_WAVE) {
+        re += ld1(part, (size_t)g * stride + off);
+        if (b >= 0) im += ld1(part, (size_t)g * stride + off + 1);
+    }
+    re = wave_sum_last(re);
+    im = wave_sum_last(im);
+    if (lane != TDSE_WAVE - 1) return;
+    if (b < 0) {
+        const double nrm = re * S.delta;
+        const int health = norm_health(S.out_norm, slot, nrm);
+        S.out_norm[slot] = nrm;
+        if (health) S.flags |= health;
+    } else {
+        S.out_ip[(size_t)slot * S.n_basis + b] = cmk(re * S.delta, im * S.delta);
+    }
+}
+
+// Time index observed by the step that ends at n + 1 (MAIN) or by the pre-sweep (n = 0), or -1.
+__device__ __forceinline__ int cyl_observed(const CylSim& S, int n) {
+    return sh_is_data_step(n, S.N, S.store_every) ? n : -1;
+}
+
+// AFTER_RHO false: with the z-sweep, or after the last step. A simulation's pending partials are those of
+// the g it now holds: reduced once per data time (again with the same result if it stays at that step).
+template <bool AFTER_RHO>
+__device__ __forceinline__ void cyl_job_block(const CylJobs& jobs) {
+    const int job = blockIdx.x * (blockDim.x / TDSE_WAVE) + threadIdx.x / TDSE_WAVE;
+    if (job >= jobs.n_jobs) return;
+    const int2 jb = jobs.jobs[job];
+    CylSim& S = jobs.sims[jb.x];
+    const int lane = threadIdx.x % TDSE_WAVE;
+    if (!S.active) return;
+    if (AFTER_RHO) {
+        const int n = S.rstep;
+        if (jb.y != -3 || lane != 0 || n >= S.N) return;
+        S.obs = cyl_observed(S, n + 1);
+        S.phase = (n + 1 < S.N && !S.hold) ? 0 : 1;  // whether g is exact
+        S.step = n + 1;
+    } else {
+        const int n = S.step;
+        if (jb.y == -3) {
+            if (lane == 0) S.rstep = n;
+        } else if (S.obs == n) {
+            cyl_observe_job(S, jb.y, n, lane);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256) k_cyl_observe(CylJobs jobs) { cyl_job_block<false>(jobs); }
+
 // ------------------------------------------------------------------ z-sweep
 //
 // One workgroup of 2 Pz threads per (simulation, pair of rho-lines 2 q, 2 q + 1);
@@ -120,9 +194,13 @@ __device__ __forceinline__ double cyl_mask_r(const CylSim& S, double r) {
 // padding line (r = nr for odd nr): it holds zeros and stays zero.
 template <int M, int MAXT, int WPE, int FORM>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
-k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs) {
+k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, CylJobs jobs) {
     extern __shared__ double2 lds[];  // 3 * Pz * 2, then M * Pz * 2 for CN_CAYLEY_LDS
-    const int job = blockIdx.x;
+    if ((int)blockIdx.x < jobs.blocks) {
+        cyl_job_block<false>(jobs);
+        return;
+    }
+    const int job = blockIdx.x - jobs.blocks;
     if (job >= n_pairs) return;
     const int2 lt = pairs[job];
     CylSim& S = sims[lt.x];
@@ -193,13 +271,16 @@ __device__ __forceinline__ double cyl_block_sum(double v, double* red, int t, in
 
 template <int M, int LANES, int MODE, int MAXT, int WPE>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_cyl_rho(CylSim* __restrict__ sims, const int2* __restrict__ groups,
-                                                  int n_groups) {
+                                                  int n_groups, CylJobs jobs) {
     extern __shared__ double2 lds[];  // 3 * Cr * LANES double2, then 16 doubles for reductions
-    if ((int)blockIdx.x >= n_groups) return;
+    if ((int)blockIdx.x < jobs.blocks) {
+        if (MODE == CYL_MAIN) cyl_job_block<true>(jobs);
+        return;
+    }
     // neighbouring position groups share 128 B lines: keep them on one XCD
-    const int2 gt = groups[xcd_remap(blockIdx.x, n_groups)];
+    const int2 gt = groups[xcd_remap(blockIdx.x - jobs.blocks, n_groups)];
     CylSim& S = sims[gt.x];
-    const int n = S.step;
+    const int n = (MODE == CYL_PRE) ? S.step : S.rstep;
     if (!S.active || n >= S.N) return;
     if (MODE == CYL_PRE && S.phase != 1) return;
     const int t = threadIdx.x;
@@ -299,7 +380,9 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
 
     // observables of the exact g after n + 1 (MAIN) or 0 (PRE) steps
     const int obs = (MODE == CYL_MAIN) ? n + 1 : 0;
-    if ((MODE == CYL_MAIN || n == 0) && sh_is_data_step(obs, S.N, S.store_every)) {
+    if (MODE == CYL_PRE && n == 0 && gt.y == 0 && t == 0) jobs.sims[gt.x].obs = cyl_observed(S, 0);
+    const bool observe = (MODE == CYL_MAIN || n == 0) && sh_is_data_step(obs, S.N, S.store_every);
+    if (observe) {
         const int nb = S.n_basis;
         double* part = S.part + (size_t)gt.y * (1 + 2 * nb);
         double acc = 0.0;
@@ -346,66 +429,4 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
     }
 #pragma unroll
     for (int i = 0; i < M; ++i) st2(gl, cyl_at(i, 0, npz), x[i]);
-}
-
-// Reduce the rho-sweep partials of every simulation at a data time: job
-// (sim, -1) gives the norm, (sim, b) the inner product with test state b.
-// PRE: after the pre-sweep (data time 0); MAIN: after the main sweep (n + 1).
-__global__ void __launch_bounds__(256) k_cyl_observe(CylSim* __restrict__ sims, const int2* __restrict__ jobs,
-                                                     int n_jobs, int after_main) {
-    const int job = blockIdx.x;
-    if (job >= n_jobs) return;
-    const int2 jb = jobs[job];
-    CylSim& S = sims[jb.x];
-    const int n = S.step;
-    if (!S.active || n >= S.N) return;
-    int obs;
-    if (after_main) {
-        obs = n + 1;
-    } else {
-        if (n != 0 || S.phase != 1) return;
-        obs = 0;
-    }
-    if (!sh_is_data_step(obs, S.N, S.store_every)) return;
-    const int slot = sh_data_slot(obs, S.N, S.store_every);
-    const int stride = 1 + 2 * S.n_basis;
-    const int off = jb.y < 0 ? 0 : 1 + 2 * jb.y;
-    __shared__ double red_re[256];
-    __shared__ double red_im[256];
-    const int t = threadIdx.x;
-    double re = 0.0, im = 0.0;
-    for (int g = t; g < S.n_groups; g += blockDim.x) {
-        re += ld1(S.part, (size_t)g * stride + off);
-        if (jb.y >= 0) im += ld1(S.part, (size_t)g * stride + off + 1);
-    }
-    red_re[t] = re;
-    red_im[t] = im;
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (t < s) {
-            red_re[t] += red_re[t + s];
-            red_im[t] += red_im[t + s];
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        if (jb.y < 0) {
-            const double nrm = red_re[0] * S.delta;
-            const int health = norm_health(S.out_norm, slot, nrm);
-            S.out_norm[slot] = nrm;
-            if (health) S.flags |= health;
-        } else {
-            S.out_ip[(size_t)slot * S.n_basis + jb.y] = cmk(red_re[0] * S.delta, red_im[0] * S.delta);
-        }
-    }
-}
-
-// After a full step: advance the step counter and record whether g is exact.
-__global__ void k_cyl_advance(CylSim* sims, int n_sims) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n_sims && sims[s].active && sims[s].step < sims[s].N) {
-        const int next = sims[s].step + 1;
-        sims[s].phase = (next < sims[s].N && !sims[s].hold) ? 0 : 1;
-        sims[s].step = next;
-    }
 }

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstddef>
 #include <cstdio>
@@ -31,7 +32,9 @@ constexpr int kGraphSteps = 8;
 constexpr int kMaxL = 4096;          // largest l_bound accepted (c_l table size)
 constexpr int kSlotCapacity = 8192;  // simulations of each kind per context
 constexpr int kSideStreams = 3;      // extra streams for concurrent R-phase buckets (default priority)
+constexpr int kMaxRidingJobs = 1024;  // observation jobs (one wave each) that ride in an R-phase launch
 constexpr int kMaxPairThreads = 512; // largest workgroup of the two-line (velocity odd l-pair) R-phase
+constexpr int kNoObs = -1;           // no observation partials of a freshly uploaded cylindrical state
 constexpr int kNoFlags = 0;          // health flags of a freshly uploaded state
 static_assert(TDSE_FLAG_NONFINITE == TDSE_HEALTH_NONFINITE && TDSE_FLAG_NORM_GROWTH == TDSE_HEALTH_NORM_GROWTH,
               "health flag values of the ABI and the kernels differ");
@@ -144,14 +147,16 @@ struct Bucket {
     int P = 0;
     bool imag = false;  // Line: complex time steps (imaginary-time relaxation)
     int method = 0;     // Line: LINE_ADI, LINE_SIO_LEN or LINE_SIO_VEL
-    int lanes = 1;      // cylindrical rho-sweep: lines per workgroup
-    DevVec<int2> lines;  // SH: (slot, l); Line: (slot, 0); Cyl z: (slot, rho); Cyl rho: (slot, position group)
+    int Mr = 0, Cr = 0, lanes = 1;  // cylindrical rho-sweep: rows per thread, chunks, lines per workgroup
+    DevVec<int2> lines;   // SH: (slot, l); Line: (slot, 0); Cyl z-sweep: (slot, pair of rho-lines)
+    DevVec<int2> rlines;  // Cyl rho-sweep: (slot, position group)
     DevVec<int2> vpairs[2];  // SH: the velocity-gauge l-pairs (slot, l) of even / odd l among these simulations
     DevVec<int2> fpairs;     // SH: velocity-gauge odd l-pairs solved with their h2 factors (k_sh_rphase_vpair)
 };
 
 void free_bucket(Bucket& b) {
     if (b.lines.ptr) (void)hipFree(b.lines.ptr);
+    if (b.rlines.ptr) (void)hipFree(b.rlines.ptr);
     for (auto& v : b.vpairs)
         if (v.ptr) (void)hipFree(v.ptr);
     if (b.fpairs.ptr) (void)hipFree(b.fpairs.ptr);
@@ -193,15 +198,15 @@ struct tdse_ctx {
     ShSim* d_sh = nullptr;
     LineSim* d_line = nullptr;
     CylSim* d_cyl = nullptr;
-    DevVec<int2> cyl_jobs;
-    std::vector<Bucket> cyl_z_buckets;
-    std::vector<Bucket> cyl_r_buckets;
+    DevVec<int2> cyl_jobs, cyl_count_jobs;
+    std::vector<Bucket> cyl_buckets;  // by (z and rho layout)
     double* d_cl = nullptr;
     double* d_clv = nullptr;  // c_l (l + 1): the velocity gauge's h1 coupling per l
     int* d_ctl = nullptr;     // [1] nonzero while the next replay of the current run follows (ADI run-ahead)
     DevVec<ShWave> waves;     // length-gauge simulations' waves first, then velocity-gauge ones
     int n_len_waves = 0;
-    DevVec<int2> jobs;
+    DevVec<int2> jobs;      // SH observations, and the step counts of all but the ADI simulations
+    DevVec<int2> adi_jobs;  // the ADI simulations' step counts
     std::vector<Bucket> sh_buckets;
     std::vector<int> sh_order;  // sh_buckets by decreasing work
     std::vector<Bucket> sh_adi_buckets;  // AlternatingDirectionImplicit l-lines (slot, l) by (rows, chunks)
@@ -273,7 +278,7 @@ void drop_graph(tdse_ctx* ctx) {
 // Rebuild the ragged work tables from the live simulations.
 int rebuild_tables(tdse_ctx* ctx) {
     std::vector<ShWave> waves;
-    std::vector<int2> jobs;
+    std::vector<int2> jobs, ajobs;
     ctx->n_len_waves = -1;
     std::map<std::pair<int, int>, std::vector<int2>> shb, lnb;  // (rows, chunks [+ 4096 if complex steps])
     std::map<std::pair<int, int>, std::vector<int2>> vpb[2];    // velocity l-pairs by parity, (rows, chunks)
@@ -301,6 +306,7 @@ int rebuild_tables(tdse_ctx* ctx) {
             for (int w = 0; w < wpl; ++w) waves.push_back(ShWave{s, w * TDSE_WAVE, lo, hi});
         }
         h.wave_count = (int)waves.size() - h.wave_first;
+        (h.adi ? ajobs : jobs).push_back(make_int2(s, -3));
         jobs.push_back(make_int2(s, -1));
         if (h.dev.norm_by_l) {
             jobs.push_back(make_int2(s, -2));
@@ -338,24 +344,26 @@ int rebuild_tables(tdse_ctx* ctx) {
         if (!h.live) continue;
         lnb[{h.dev.m, h.dev.P + (h.complex_steps ? 4096 : 0) + 8192 * h.dev.method}].push_back(make_int2(s, 0));
     }
-    std::vector<int2> cjobs;
-    std::map<std::pair<int, int>, std::vector<int2>> czb;             // (rows, chunks)
-    std::map<std::pair<int, int>, std::vector<int2>> crb;             // (rows + 64 * lanes, chunks)
+    std::vector<int2> cjobs, ccount;
+    std::map<std::array<int, 5>, std::pair<std::vector<int2>, std::vector<int2>>> cyb;  // (Mz, Pz, Mr, Cr, lanes)
     for (int s = 0; s < (int)ctx->cyl.size(); ++s) {
         const CylHost& h = ctx->cyl[s];
         if (!h.live) continue;
         const CylSim& C = h.dev;
         cjobs.push_back(make_int2(s, -1));
+        cjobs.push_back(make_int2(s, -3));
+        ccount.push_back(make_int2(s, -3));
         for (int b = 0; b < C.n_basis; ++b) cjobs.push_back(make_int2(s, b));
-        auto& vz = czb[{C.Mz, C.Pz}];
-        for (int q = 0; 2 * q < C.nr; ++q) vz.push_back(make_int2(s, q));  // pairs of rho-lines
-        auto& vr = crb[{C.Mr + 64 * C.lanes, C.Cr}];
-        for (int g = 0; g < C.n_groups; ++g) vr.push_back(make_int2(s, g));
+        auto& v = cyb[{C.Mz, C.Pz, C.Mr, C.Cr, C.lanes}];
+        for (int q = 0; 2 * q < C.nr; ++q) v.first.push_back(make_int2(s, q));  // pairs of rho-lines
+        for (int g = 0; g < C.n_groups; ++g) v.second.push_back(make_int2(s, g));
     }
     int rc;
     if ((rc = devvec_upload(ctx, ctx->waves, waves))) return rc;
     if ((rc = devvec_upload(ctx, ctx->jobs, jobs))) return rc;
+    if ((rc = devvec_upload(ctx, ctx->adi_jobs, ajobs))) return rc;
     if ((rc = devvec_upload(ctx, ctx->cyl_jobs, cjobs))) return rc;
+    if ((rc = devvec_upload(ctx, ctx->cyl_count_jobs, ccount))) return rc;
     auto fill = [&](std::vector<Bucket>& dst, std::map<std::pair<int, int>, std::vector<int2>>& src) -> int {
         for (auto& b : dst) free_bucket(b);
         dst.clear();
@@ -385,8 +393,19 @@ int rebuild_tables(tdse_ctx* ctx) {
         if (it != fpb.end() && (rc = devvec_upload(ctx, b.fpairs, it->second))) return rc;
     }
     if ((rc = fill(ctx->line_buckets, lnb))) return rc;
-    if ((rc = fill(ctx->cyl_z_buckets, czb))) return rc;
-    if ((rc = fill(ctx->cyl_r_buckets, crb))) return rc;
+    for (auto& b : ctx->cyl_buckets) free_bucket(b);
+    ctx->cyl_buckets.clear();
+    for (auto& kv : cyb) {
+        ctx->cyl_buckets.emplace_back();
+        Bucket& b = ctx->cyl_buckets.back();
+        b.M = kv.first[0];
+        b.P = kv.first[1];
+        b.Mr = kv.first[2];
+        b.Cr = kv.first[3];
+        b.lanes = kv.first[4];
+        if ((rc = devvec_upload(ctx, b.lines, kv.second.first)) || (rc = devvec_upload(ctx, b.rlines, kv.second.second)))
+            return rc;
+    }
     {
         std::vector<std::pair<double, int>> w;
         for (size_t i = 0; i < ctx->sh_buckets.size(); ++i) {
@@ -400,10 +419,6 @@ int rebuild_tables(tdse_ctx* ctx) {
         std::sort(w.begin(), w.end());
         ctx->sh_order.clear();
         for (auto& pr : w) ctx->sh_order.push_back(pr.second);
-    }
-    for (auto& b : ctx->cyl_r_buckets) {  // key first = rows + 64 * lanes
-        b.lanes = b.M / 64;
-        b.M %= 64;
     }
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     drop_graph(ctx);
@@ -442,56 +457,64 @@ size_t cn_lds_bytes(int M, int P, int form) {
     return (size_t)(form == CN_CAYLEY_LDS ? 3 + M : 3) * P * sizeof(double2);
 }
 
-// Launch shapes per rows-per-thread M (block size, minimum waves per EU).
-template <int M, int MAXT, int WPE>
-void launch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
-    const int form = cn_form(M, b.P);
-    const size_t lds = cn_lds_bytes(M, b.P, form);
-    const dim3 grid((unsigned)b.lines.count), block(b.P);
-    if (form == CN_EXPLICIT)
-        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
-                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count);
-    else if (form == CN_CAYLEY_LDS)
-        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS)>), grid, block, lds,
-                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count);
-    else
-        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
-                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count);
+// A job list as leading workgroups of a launch of `threads` per workgroup (none: no jobs ride there).
+ShObs obs_of(const tdse_ctx* ctx, const DevVec<int2>& list, int threads, bool ride) {
+    const int per = threads / TDSE_WAVE, nj = ride ? (int)list.count : 0;
+    return ShObs{ctx->d_sh, list.ptr, nj, (nj + per - 1) / per, ctx->d_ctl};
 }
 
-void dispatch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
+// Launch shapes per rows-per-thread M (block size, minimum waves per EU).
+template <int M, int MAXT, int WPE>
+void launch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
+    const int form = cn_form(M, b.P);
+    const size_t lds = cn_lds_bytes(M, b.P, form);
+    const ShObs obs = obs_of(ctx, ctx->jobs, b.P, ride);
+    const dim3 grid((unsigned)(b.lines.count + obs.blocks)), block(b.P);
+    if (form == CN_EXPLICIT)
+        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
+                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
+    else if (form == CN_CAYLEY_LDS)
+        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS)>), grid, block, lds,
+                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
+    else
+        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
+                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
+}
+
+void dispatch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
     switch (b.M) {
-        case 2: launch_rphase<2, 512, 4>(ctx, b, st); break;
-        case 4: launch_rphase<4, 512, 4>(ctx, b, st); break;
-        case 6: launch_rphase<6, 512, 4>(ctx, b, st); break;
-        case 8: launch_rphase<8, 512, 4>(ctx, b, st); break;
+        case 2: launch_rphase<2, 512, 4>(ctx, b, st, ride); break;
+        case 4: launch_rphase<4, 512, 4>(ctx, b, st, ride); break;
+        case 6: launch_rphase<6, 512, 4>(ctx, b, st, ride); break;
+        case 8: launch_rphase<8, 512, 4>(ctx, b, st, ride); break;
         // radial lines past 4096 points: 512-thread workgroups of deep tiles
-        case 10: b.P > 256 ? launch_rphase<10, 512, 1>(ctx, b, st) : launch_rphase<10, 256, 3>(ctx, b, st); break;
-        case 12: b.P > 256 ? launch_rphase<12, 512, 1>(ctx, b, st) : launch_rphase<12, 256, 2>(ctx, b, st); break;
-        case 14: b.P > 256 ? launch_rphase<14, 512, 1>(ctx, b, st) : launch_rphase<14, 256, 2>(ctx, b, st); break;
-        default: b.P > 256 ? launch_rphase<16, 512, 1>(ctx, b, st) : launch_rphase<16, 256, 1>(ctx, b, st); break;
+        case 10: b.P > 256 ? launch_rphase<10, 512, 1>(ctx, b, st, ride) : launch_rphase<10, 256, 3>(ctx, b, st, ride); break;
+        case 12: b.P > 256 ? launch_rphase<12, 512, 1>(ctx, b, st, ride) : launch_rphase<12, 256, 2>(ctx, b, st, ride); break;
+        case 14: b.P > 256 ? launch_rphase<14, 512, 1>(ctx, b, st, ride) : launch_rphase<14, 256, 2>(ctx, b, st, ride); break;
+        default: b.P > 256 ? launch_rphase<16, 512, 1>(ctx, b, st, ride) : launch_rphase<16, 256, 1>(ctx, b, st, ride); break;
     }
 }
 
 template <int M, int MAXT, int WPE, bool EXPL>
-void launch_adi_r(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
+void launch_adi_r(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
     const size_t lds = 3 * (size_t)b.P * sizeof(double2);
-    hipLaunchKernelGGL((k_sh_adi_r<M, MAXT, WPE, EXPL>), dim3((unsigned)b.lines.count), dim3(b.P), lds, st,
-                       ctx->d_sh, b.lines.ptr, (int)b.lines.count, ctx->d_ctl);
+    const ShObs obs = obs_of(ctx, EXPL ? ctx->jobs : ctx->adi_jobs, b.P, ride);
+    hipLaunchKernelGGL((k_sh_adi_r<M, MAXT, WPE, EXPL>), dim3((unsigned)(b.lines.count + obs.blocks)), dim3(b.P), lds,
+                       st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, ctx->d_ctl, obs);
 }
 
 // the R-phase's launch shapes
 template <bool EXPL>
-void dispatch_adi_r(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
+void dispatch_adi_r(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
     switch (b.M) {
-        case 2: launch_adi_r<2, 512, 4, EXPL>(ctx, b, st); break;
-        case 4: launch_adi_r<4, 512, 4, EXPL>(ctx, b, st); break;
-        case 6: launch_adi_r<6, 512, 4, EXPL>(ctx, b, st); break;
-        case 8: launch_adi_r<8, 512, EXPL ? 4 : 3, EXPL>(ctx, b, st); break;  // the run-ahead's registers
-        case 10: b.P > 256 ? launch_adi_r<10, 512, 1, EXPL>(ctx, b, st) : launch_adi_r<10, 256, 3, EXPL>(ctx, b, st); break;
-        case 12: b.P > 256 ? launch_adi_r<12, 512, 1, EXPL>(ctx, b, st) : launch_adi_r<12, 256, 2, EXPL>(ctx, b, st); break;
-        case 14: b.P > 256 ? launch_adi_r<14, 512, 1, EXPL>(ctx, b, st) : launch_adi_r<14, 256, 2, EXPL>(ctx, b, st); break;
-        default: b.P > 256 ? launch_adi_r<16, 512, 1, EXPL>(ctx, b, st) : launch_adi_r<16, 256, 2, EXPL>(ctx, b, st); break;
+        case 2: launch_adi_r<2, 512, 4, EXPL>(ctx, b, st, ride); break;
+        case 4: launch_adi_r<4, 512, 4, EXPL>(ctx, b, st, ride); break;
+        case 6: launch_adi_r<6, 512, 4, EXPL>(ctx, b, st, ride); break;
+        case 8: launch_adi_r<8, 512, EXPL ? 4 : 3, EXPL>(ctx, b, st, ride); break;  // the run-ahead's registers
+        case 10: b.P > 256 ? launch_adi_r<10, 512, 1, EXPL>(ctx, b, st, ride) : launch_adi_r<10, 256, 3, EXPL>(ctx, b, st, ride); break;
+        case 12: b.P > 256 ? launch_adi_r<12, 512, 1, EXPL>(ctx, b, st, ride) : launch_adi_r<12, 256, 2, EXPL>(ctx, b, st, ride); break;
+        case 14: b.P > 256 ? launch_adi_r<14, 512, 1, EXPL>(ctx, b, st, ride) : launch_adi_r<14, 256, 2, EXPL>(ctx, b, st, ride); break;
+        default: b.P > 256 ? launch_adi_r<16, 512, 1, EXPL>(ctx, b, st, ride) : launch_adi_r<16, 256, 2, EXPL>(ctx, b, st, ride); break;
     }
 }
 
@@ -589,49 +612,63 @@ void dispatch_line(tdse_ctx* ctx, const Bucket& b, int n_steps) {
     else dispatch_line_m<true, LINE_ADI>(ctx, b, n_steps);
 }
 
+// The cylindrical observation jobs as leading workgroups of a launch of `threads` per workgroup.
+CylJobs cyl_jobs_of(const tdse_ctx* ctx, const DevVec<int2>& list, int threads, bool ride) {
+    const int per = threads / TDSE_WAVE, nj = ride ? (int)list.count : 0;
+    return CylJobs{ctx->d_cyl, list.ptr, nj, (nj + per - 1) / per};
+}
+
 // The z-sweep solves two rho-lines per workgroup (2 Pz threads), explicit form
 // (with two lines per workgroup the Cayley forms measured slower: re-reading the
 // rows 0.44 ms, keeping them in LDS 0.64 ms per sweep against 0.40 ms).
 template <int M, int MAXT, int WPE>
-void launch_cyl_z(tdse_ctx* ctx, const Bucket& b) {
+void launch_cyl_z(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
     const size_t lds = 2 * cn_lds_bytes(M, b.P, CN_EXPLICIT);
-    hipLaunchKernelGGL((k_cyl_z<M, MAXT, WPE, CN_EXPLICIT>), dim3((unsigned)b.lines.count), dim3(2 * b.P), lds,
-                       ctx->stream, ctx->d_cyl, b.lines.ptr, (int)b.lines.count);
+    const CylJobs jobs = cyl_jobs_of(ctx, ctx->cyl_jobs, 2 * b.P, ride);
+    hipLaunchKernelGGL((k_cyl_z<M, MAXT, WPE, CN_EXPLICIT>), dim3((unsigned)(b.lines.count + jobs.blocks)),
+                       dim3(2 * b.P), lds, st, ctx->d_cyl, b.lines.ptr, (int)b.lines.count, jobs);
 }
 
-void dispatch_cyl_z(tdse_ctx* ctx, const Bucket& b) {
+void dispatch_cyl_z(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
     switch (b.M) {
-        case 2: launch_cyl_z<2, 1024, 4>(ctx, b); break;
-        case 4: launch_cyl_z<4, 1024, 4>(ctx, b); break;
-        case 6: launch_cyl_z<6, 1024, 4>(ctx, b); break;
-        case 8: launch_cyl_z<8, 1024, 4>(ctx, b); break;
-        case 10: launch_cyl_z<10, 512, 3>(ctx, b); break;
-        case 12: launch_cyl_z<12, 512, 2>(ctx, b); break;
-        case 14: launch_cyl_z<14, 512, 2>(ctx, b); break;
-        default: launch_cyl_z<16, 512, 2>(ctx, b); break;
+        case 2: launch_cyl_z<2, 1024, 4>(ctx, b, st, ride); break;
+        case 4: launch_cyl_z<4, 1024, 4>(ctx, b, st, ride); break;
+        case 6: launch_cyl_z<6, 1024, 4>(ctx, b, st, ride); break;
+        case 8: launch_cyl_z<8, 1024, 4>(ctx, b, st, ride); break;
+        case 10: launch_cyl_z<10, 512, 3>(ctx, b, st, ride); break;
+        case 12: launch_cyl_z<12, 512, 2>(ctx, b, st, ride); break;
+        case 14: launch_cyl_z<14, 512, 2>(ctx, b, st, ride); break;
+        default: launch_cyl_z<16, 512, 2>(ctx, b, st, ride); break;
     }
 }
 
 template <int M, int LANES, int MAXT, int WPE>
-void launch_cyl_rho(tdse_ctx* ctx, const Bucket& b, int mode) {
-    const size_t lds = 3 * (size_t)b.P * LANES * sizeof(double2) + 16 * sizeof(double);
-    const dim3 grid((unsigned)b.lines.count), block((unsigned)(b.P * LANES));
+void launch_cyl_rho(tdse_ctx* ctx, const Bucket& b, hipStream_t st, int mode, bool ride) {
+    const CylJobs jobs = cyl_jobs_of(ctx, ctx->cyl_count_jobs, b.Cr * LANES, ride);
+    const size_t lds = 3 * (size_t)b.Cr * LANES * sizeof(double2) + 16 * sizeof(double);
+    const dim3 grid((unsigned)(b.rlines.count + jobs.blocks)), block((unsigned)(b.Cr * LANES));
     if (mode == CYL_PRE)
-        hipLaunchKernelGGL((k_cyl_rho<M, LANES, CYL_PRE, MAXT, WPE>), grid, block, lds, ctx->stream, ctx->d_cyl,
-                           b.lines.ptr, (int)b.lines.count);
+        hipLaunchKernelGGL((k_cyl_rho<M, LANES, CYL_PRE, MAXT, WPE>), grid, block, lds, st, ctx->d_cyl,
+                           b.rlines.ptr, (int)b.rlines.count, jobs);
     else
-        hipLaunchKernelGGL((k_cyl_rho<M, LANES, CYL_MAIN, MAXT, WPE>), grid, block, lds, ctx->stream, ctx->d_cyl,
-                           b.lines.ptr, (int)b.lines.count);
+        hipLaunchKernelGGL((k_cyl_rho<M, LANES, CYL_MAIN, MAXT, WPE>), grid, block, lds, st, ctx->d_cyl,
+                           b.rlines.ptr, (int)b.rlines.count, jobs);
 }
 
 // rho-sweep shapes (rows, lines per workgroup, block limit, minimum waves per
 // EU); the layout chooser of the host package picks one of these.
-void dispatch_cyl_rho(tdse_ctx* ctx, const Bucket& b, int mode) {
-    if (b.M == 4 && b.lanes == 4) launch_cyl_rho<4, 4, 1024, 4>(ctx, b, mode);
-    else if (b.M == 8 && b.lanes == 4) launch_cyl_rho<8, 4, 512, 4>(ctx, b, mode);
-    else if (b.M == 4 && b.lanes == 8) launch_cyl_rho<4, 8, 1024, 4>(ctx, b, mode);
-    else if (b.M == 8 && b.lanes == 8) launch_cyl_rho<8, 8, 1024, 4>(ctx, b, mode);
-    else launch_cyl_rho<16, 4, 512, 2>(ctx, b, mode);
+void dispatch_cyl_rho(tdse_ctx* ctx, const Bucket& b, hipStream_t st, int mode, bool ride) {
+    if (b.Mr == 4 && b.lanes == 4) launch_cyl_rho<4, 4, 1024, 4>(ctx, b, st, mode, ride);
+    else if (b.Mr == 8 && b.lanes == 4) launch_cyl_rho<8, 4, 512, 4>(ctx, b, st, mode, ride);
+    else if (b.Mr == 4 && b.lanes == 8) launch_cyl_rho<4, 8, 1024, 4>(ctx, b, st, mode, ride);
+    else if (b.Mr == 8 && b.lanes == 8) launch_cyl_rho<8, 8, 1024, 4>(ctx, b, st, mode, ride);
+    else launch_cyl_rho<16, 4, 512, 2>(ctx, b, st, mode, ride);
+}
+
+// Reduce the pending observations of the cylindrical simulations.
+void cyl_observe(tdse_ctx* ctx) {
+    const CylJobs jobs = cyl_jobs_of(ctx, ctx->cyl_jobs, 256, true);
+    hipLaunchKernelGGL(k_cyl_observe, dim3(jobs.blocks), dim3(256), 0, ctx->stream, jobs);
 }
 
 // Launch one full step of every simulation kind onto the context stream.
@@ -646,20 +683,25 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
         if (nl > 0) {
             auto lphase = ctx->sh_norm_by_l ? k_sh_lphase<true, false> : k_sh_lphase<false, false>;
             hipLaunchKernelGGL(lphase, dim3((nl * TDSE_WAVE + 255) / 256), dim3(256), 0, ctx->stream, ctx->d_sh,
-                               ctx->waves.ptr, nl, ctx->d_cl, 0);
+                               ctx->waves.ptr, nl, ctx->d_cl, 0, ctx->d_sh);
         }
         if (nv > 0) {
             auto lphase = ctx->sh_norm_by_l ? k_sh_lphase<true, true> : k_sh_lphase<false, true>;
             hipLaunchKernelGGL(lphase, dim3((nv * TDSE_WAVE + 255) / 256), dim3(256), 0, ctx->stream, ctx->d_sh,
-                               ctx->waves.ptr + nl, nv, ctx->d_clv, 0);
+                               ctx->waves.ptr + nl, nv, ctx->d_clv, 0, ctx->d_sh);
         }
         prof_end(ctx);
-        // The observables read only what the L-phase wrote (per-wave partials, snapshot rows), which
-        // nothing else touches before the next replay: they can run beside the R-phase.
+        // The observables read only what the L-phase wrote (partials, snapshot rows), which nothing
+        // else touches before the next replay: a few of them ride in the next launch (the smallest
+        // R-phase bucket, or the first explicit ADI sweep), many get a launch beside the R-phase.
         const int nj = (int)ctx->jobs.count;
+        const bool ride = nj <= kMaxRidingJobs;
         auto observe = [&](hipStream_t st) {
-            hipLaunchKernelGGL(k_sh_observe, dim3(nj), dim3(256), 0, st, ctx->d_sh, ctx->jobs.ptr, nj);
+            if (ride) return;
+            const ShObs obs = obs_of(ctx, ctx->jobs, 256, true);
+            hipLaunchKernelGGL(k_sh_observe, dim3(obs.blocks), dim3(256), 0, st, obs);
         };
+        const Bucket* rider = ctx->sh_order.empty() ? nullptr : &ctx->sh_buckets[ctx->sh_order.back()];
         // One bucket's chain: velocity-gauge h2 factors of its even, then odd l-pairs
         // (before the CN solve), the R-phase, the factors in reverse (after it). The
         // chains of different buckets touch different simulations.
@@ -672,7 +714,7 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
                 }
             if (b.lines.count) {
                 prof_begin(ctx, 1);
-                dispatch_rphase(ctx, b, st);
+                dispatch_rphase(ctx, b, st, ride && &b == rider);
                 prof_end(ctx);
             }
             if (b.fpairs.count) {
@@ -730,7 +772,10 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
         };
         if (!ctx->sh_adi_buckets.empty()) {
             int rc;
-            if ((rc = fan(ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) { dispatch_adi_r<true>(ctx, b, st); })))
+            const Bucket* first = rider ? nullptr : &ctx->sh_adi_buckets[0];
+            if ((rc = fan(ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) {
+                    dispatch_adi_r<true>(ctx, b, st, ride && &b == first);
+                })))
                 return rc;
             if ((rc = fan(ctx->sh_adi_lbuckets, [&](const Bucket& b, hipStream_t st) { dispatch_adi_lp(ctx, b, st); })))
                 return rc;
@@ -738,33 +783,29 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
             if (na > 0)
                 hipLaunchKernelGGL(k_sh_adi_l, dim3((na * TDSE_WAVE + 255) / 256), dim3(256), 0, ctx->stream,
                                    ctx->d_sh, ctx->adi_waves.ptr, na, ctx->d_cl);
-            if ((rc = fan(ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) { dispatch_adi_r<false>(ctx, b, st); })))
+            if ((rc = fan(ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) {
+                    dispatch_adi_r<false>(ctx, b, st, &b == &ctx->sh_adi_buckets[0]);
+                })))
                 return rc;
         }
-        const int ns = (int)ctx->sh.size();
-        hipLaunchKernelGGL(k_sh_advance, dim3((ns + 255) / 256), dim3(256), 0, ctx->stream, ctx->d_sh, ns, ctx->d_ctl);
     }
     for (auto& b : ctx->line_buckets) dispatch_line(ctx, b, 1);
-    if (!ctx->cyl_r_buckets.empty()) {
-        const int nj = (int)ctx->cyl_jobs.count;
+    if (!ctx->cyl_buckets.empty()) {
         if (cyl_pre) {
-            for (auto& b : ctx->cyl_r_buckets) dispatch_cyl_rho(ctx, b, CYL_PRE);
-            hipLaunchKernelGGL(k_cyl_observe, dim3(nj), dim3(256), 0, ctx->stream, ctx->d_cyl, ctx->cyl_jobs.ptr, nj,
-                               0);
+            for (auto& b : ctx->cyl_buckets) dispatch_cyl_rho(ctx, b, ctx->stream, CYL_PRE, false);
+            cyl_observe(ctx);
         }
-        for (auto& b : ctx->cyl_z_buckets) {
+        // one bucket's chain; the buckets hold different simulations. The jobs of all of them ride with the
+        // first z-sweep (S.step is then still the same for every sweep) and the last rho-sweep.
+        auto chain = [&](const Bucket& b, hipStream_t st) {
             prof_begin(ctx, 2);
-            dispatch_cyl_z(ctx, b);
+            dispatch_cyl_z(ctx, b, st, &b == &ctx->cyl_buckets[0]);
             prof_end(ctx);
-        }
-        for (auto& b : ctx->cyl_r_buckets) {
             prof_begin(ctx, 3);
-            dispatch_cyl_rho(ctx, b, CYL_MAIN);
+            dispatch_cyl_rho(ctx, b, st, CYL_MAIN, &b == &ctx->cyl_buckets.back());
             prof_end(ctx);
-        }
-        hipLaunchKernelGGL(k_cyl_observe, dim3(nj), dim3(256), 0, ctx->stream, ctx->d_cyl, ctx->cyl_jobs.ptr, nj, 1);
-        const int nc = (int)ctx->cyl.size();
-        hipLaunchKernelGGL(k_cyl_advance, dim3((nc + 255) / 256), dim3(256), 0, ctx->stream, ctx->d_cyl, nc);
+        };
+        for (auto& b : ctx->cyl_buckets) chain(b, ctx->stream);
     }
     HIP_TRY(ctx, hipGetLastError());
     return TDSE_OK;
@@ -926,10 +967,12 @@ int tdse_ctx_destroy(tdse_ctx* ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     drop_graph(ctx);
     for (auto* v : {&ctx->sh_buckets, &ctx->sh_adi_buckets, &ctx->sh_adi_lbuckets, &ctx->line_buckets,
-                    &ctx->cyl_z_buckets, &ctx->cyl_r_buckets})
+                    &ctx->cyl_buckets})
         for (auto& b : *v) free_bucket(b);
     if (ctx->adi_waves.ptr) (void)hipFree(ctx->adi_waves.ptr);
     if (ctx->cyl_jobs.ptr) (void)hipFree(ctx->cyl_jobs.ptr);
+    if (ctx->cyl_count_jobs.ptr) (void)hipFree(ctx->cyl_count_jobs.ptr);
+    if (ctx->adi_jobs.ptr) (void)hipFree(ctx->adi_jobs.ptr);
     if (ctx->d_cyl) (void)hipFree(ctx->d_cyl);
     if (ctx->waves.ptr) (void)hipFree(ctx->waves.ptr);
     if (ctx->jobs.ptr) (void)hipFree(ctx->jobs.ptr);
@@ -1345,6 +1388,7 @@ int tdse_cyl_add(tdse_ctx* ctx, const tdse_cyl_desc* desc, const double* zt, con
     S.rho0 = D.rho_first;
     S.drho = D.rho_step;
     S.step = 0;
+    S.obs = -1;
     S.active = 1;
     S.phase = 1;
     S.hold = 0;
@@ -1441,6 +1485,10 @@ int tdse_run(tdse_ctx* ctx, int32_t n_steps, int32_t use_graph) {
         }
         ctx->cyl_pending = false;
         i += done;
+    }
+    if (n_steps > 0 && !ctx->cyl_buckets.empty()) {  // the last step's observations
+        cyl_observe(ctx);
+        HIP_TRY(ctx, hipGetLastError());
     }
     HIP_TRY(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
     HIP_TRY(ctx, hipEventSynchronize(ctx->ev_stop));
@@ -1592,6 +1640,7 @@ int tdse_upload_state(tdse_ctx* ctx, int32_t kind, int32_t slot, const double* g
         HIP_TRY(ctx, hipMemcpy(base + offsetof(CylSim, step), &st[0], sizeof(int), hipMemcpyHostToDevice));
         HIP_TRY(ctx, hipMemcpy(base + offsetof(CylSim, phase), &st[1], sizeof(int), hipMemcpyHostToDevice));
         HIP_TRY(ctx, hipMemcpy(base + offsetof(CylSim, flags), &kNoFlags, sizeof(int), hipMemcpyHostToDevice));
+        HIP_TRY(ctx, hipMemcpy(base + offsetof(CylSim, obs), &kNoObs, sizeof(int), hipMemcpyHostToDevice));
         ctx->cyl_pending = true;
     } else {
         return fail(ctx, TDSE_ERR_ARG, "unknown simulation kind");
@@ -1689,10 +1738,10 @@ int tdse_materialize(tdse_ctx* ctx, int32_t kind, int32_t slot) {
     const int nw = H.wave_count;
     if (H.vel)
         hipLaunchKernelGGL((k_sh_lphase<false, true>), dim3((nw * TDSE_WAVE + 255) / 256), dim3(256), 0, ctx->stream,
-                           ctx->d_sh, ctx->waves.ptr + H.wave_first, nw, ctx->d_clv, 1);
+                           ctx->d_sh, ctx->waves.ptr + H.wave_first, nw, ctx->d_clv, 1, ctx->d_sh);
     else
         hipLaunchKernelGGL((k_sh_lphase<false, false>), dim3((nw * TDSE_WAVE + 255) / 256), dim3(256), 0,
-                           ctx->stream, ctx->d_sh, ctx->waves.ptr + H.wave_first, nw, ctx->d_cl, 1);
+                           ctx->stream, ctx->d_sh, ctx->waves.ptr + H.wave_first, nw, ctx->d_cl, 1, ctx->d_sh);
     HIP_TRY(ctx, hipGetLastError());
     // the end-only L-phase wrote sh_state(n + 1): swap the buffers so the exact
     // state is sh_state(n) for the unchanged step counter

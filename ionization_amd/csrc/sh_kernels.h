@@ -47,7 +47,8 @@ struct ShSim {
     double delta_r;
     double cu;             // tau0 hbar^2 / (2 mu): U_j = cu / r_j^2, r_j = (j + 1/2) delta_r
     int n, L, P, m, npad, N, store_every, LB, n_basis, n_part;
-    int step;              // steps already advanced; device-updated
+    int step;              // steps already advanced; read by the L-phase and the host, written after it (sh_advance)
+    int rstep;             // the step under way: written by the L-phase, read by every kernel after it
     int active;
     int phase;             // 0: g is mid-step (after the R-phase); 1: g is the reference g after `step` steps
     int norm_by_l;         // 1: also reduce the norm of every l at data times
@@ -89,6 +90,20 @@ __device__ __forceinline__ int sh_data_slot(int n, int N, int every) {
 // after n + 1 steps is not observed.
 __device__ __forceinline__ bool sh_adi_ahead(const ShSim& S, int n, int ok) {
     return ok && n + 1 < S.N && !sh_is_data_step(n + 1, S.N, S.store_every);
+}
+
+// The step counters. The L-phase reads S.step and copies it to S.rstep (its first wave, at its end);
+// the kernels of the rest of the step read S.rstep only, so a job wave beside them (job -3) may set
+// S.step for the next L-phase: a step needs no launch of its own to count, which cost 4.4 us of a small
+// mesh's 20. The job of an ADI simulation rides with the implicit sweep, the step's last kernel, since
+// the explicit one reads S.ahead. A finished simulation has step N + 1.
+__device__ __forceinline__ void sh_count_step(ShSim& S, int ctl) {
+    const int n = S.rstep;
+    if (!S.active || n > S.N) return;
+    // the same decision as this replay's implicit ADI r-sweep
+    S.ahead = (S.adi && n < S.N && sh_adi_ahead(S, n, ctl)) ? 1 : 0;
+    S.phase = 0;
+    S.step = n + 1;
 }
 
 // Length gauge (VEL = false): exp(-i a sigma_x) applied to (x0, x1),
@@ -153,9 +168,11 @@ struct ShWave {
 // mesh_operators.py:1201-1250): the host supplies the angle factors (RQ row:
 // tau0 hbar (q / m) / r_j; fs: the vector potential; cl: c_l (l + 1)) and the
 // rotation is the real one.
+// counters: the simulations again, for the step counter's store (a pointer of its own as in ShObs).
 template <bool BY_L, bool VEL>
 __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, const ShWave* __restrict__ waves,
-                                                   int n_waves, const double* __restrict__ cl, int end_only) {
+                                                   int n_waves, const double* __restrict__ cl, int end_only,
+                                                   ShSim* counters) {
     constexpr int PF = 4;  // prefetch depth in iterations (2 rows each)
     const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / TDSE_WAVE;
     const int lane = threadIdx.x % TDSE_WAVE;
@@ -164,8 +181,13 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
     ShSim& S = sims[wt.sim];
     const int n = S.step;
     const int N = S.N;
-    if (!S.active || n > N) return;
-    if (S.ahead) return;  // ADI: the previous replay already masked g and started this step in place of it
+    if (!S.active) return;
+    const bool begins = !end_only && wt.p0 == 0 && wt.lo == 0 && lane == 0;
+    // ADI run-ahead: the previous replay already masked g and started this step in place of this one
+    if (n > N || S.ahead) {
+        if (begins) counters[wt.sim].rstep = n;
+        return;
+    }
     const bool do_end = n > 0 && S.phase == 0;
     const bool do_start = n < N && !end_only;
     const bool observe = !end_only && sh_is_data_step(n, N, S.store_every);
@@ -327,72 +349,85 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
         c_m2 = c0;
         c_m1 = c1;
     }
+    if (begins) counters[wt.sim].rstep = n;
 }
 
 // ------------------------------------------------------------------ observables
 //
-// Job table entry (sim, b): b == -1 reduces the norm partials, b >= 0 forms
-// the inner product of test state b with the captured row l_b:
+// Job table entry (sim, b): b == -1 reduces the norm partials, b == -2 the norms by l, b == -3 counts
+// the step (sh_count_step), b >= 0 forms the inner product of test state b with the captured row l_b:
 //     <phi_b | g> = sum_j phi_b(j) g(l_b, j) dr        (meshes.py:1117-1129)
-// Sums run in a fixed order per simulation, independent of the batch.
-__global__ void __launch_bounds__(256) k_sh_observe(ShSim* __restrict__ sims, const int2* __restrict__ jobs,
-                                                    int n_jobs) {
-    const int job = blockIdx.x;
-    if (job >= n_jobs) return;
-    const int2 jb = jobs[job];
-    ShSim& S = sims[jb.x];
-    const int n = S.step;
+// One wave per job; sums run in a fixed order per simulation, independent of the batch and of the
+// launch. The observations read only what the L-phase wrote, so in a small batch they ride in the first
+// workgroups of the launch that follows it (ShObs; 4.5 us of a small mesh's 20 us step as a launch of
+// their own); a large batch's run beside the R-phase on a side stream.
+struct ShObs {
+    ShSim* sims;  // the launch's simulations, by a pointer of its own: what the jobs store must not look to the
+                  // compiler like a store to the fields that the launch's other workgroups read (sims, restrict),
+                  // which it would then load through the vector memory path (R-phase 6 to 12 more VGPRs)
+    const int2* jobs;
+    int n_jobs;
+    int blocks;  // leading workgroups of the launch that take jobs, blockDim.x / 64 each
+    const int* ctl;
+};
+
+__device__ __forceinline__ void sh_observe_job(ShSim& S, const int b, const int lane) {
+    const int n = S.rstep;
     if (!S.active || n > S.N || !sh_is_data_step(n, S.N, S.store_every)) return;
     const int slot = sh_data_slot(n, S.N, S.store_every);
-    __shared__ double red_re[256];
-    __shared__ double red_im[256];
-    const int t = threadIdx.x;
-    double re = 0.0, im = 0.0;
-    if (jb.y == -2) {
+    if (b == -2) {
         // norm in every l: the row's partials in position order
         const int L = S.L, wpl = S.npad / TDSE_WAVE;
-        for (int l = t; l < L; l += blockDim.x) {
+        for (int l = lane; l < L; l += TDSE_WAVE) {
             double acc = 0.0;
             for (int w = 0; w < wpl; ++w) acc += ld1(S.part_l, (size_t)l * wpl + w);
             S.out_nl[(size_t)slot * L + l] = acc * S.delta_r;
         }
         return;
     }
-    if (jb.y < 0) {
-        for (int w = t; w < S.n_part; w += blockDim.x) re += ld1(S.part, w);
-        for (int w = t; w < S.npad / TDSE_WAVE; w += blockDim.x) im += ld1(S.part, S.n_part + w);
+    double re = 0.0, im = 0.0;
+    if (b < 0) {
+        const double* __restrict__ part = S.part;
+        const int n_part = S.n_part, wpl = S.npad / TDSE_WAVE;
+#pragma unroll 4
+        for (int w = lane; w < n_part; w += TDSE_WAVE) re += ld1(part, w);
+        for (int w = lane; w < wpl; w += TDSE_WAVE) im += ld1(part, n_part + w);
     } else {
-        const double* phi = S.basis + (size_t)jb.y * S.npad;
-        const double2* row = S.snap + (size_t)S.basis_l[jb.y] * S.npad;
-        for (int p = t; p < S.npad; p += blockDim.x) {
+        const int npad = S.npad;
+        const double* __restrict__ phi = S.basis + (size_t)b * npad;
+        const double2* __restrict__ row = S.snap + (size_t)S.basis_l[b] * npad;
+#pragma unroll 4
+        for (int p = lane; p < npad; p += TDSE_WAVE) {
             const double f = ld1(phi, p);
             const double2 z = ld2(row, p);
             re = fma(f, z.x, re);
             im = fma(f, z.y, im);
         }
     }
-    red_re[t] = re;
-    red_im[t] = im;
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (t < s) {
-            red_re[t] += red_re[t + s];
-            red_im[t] += red_im[t + s];
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        if (jb.y < 0) {
-            const double nrm = red_re[0] * S.delta_r;
-            const int health = norm_health(S.out_norm, slot, nrm);
-            S.out_norm[slot] = nrm;
-            S.out_lnorm[slot] = red_im[0] * S.delta_r;
-            if (health) S.flags |= health;
-        } else {
-            S.out_ip[(size_t)slot * S.n_basis + jb.y] = cmk(red_re[0] * S.delta_r, red_im[0] * S.delta_r);
-        }
+    re = wave_sum_last(re);
+    im = wave_sum_last(im);
+    if (lane != TDSE_WAVE - 1) return;
+    if (b < 0) {
+        const double nrm = re * S.delta_r;
+        const int health = norm_health(S.out_norm, slot, nrm);
+        S.out_norm[slot] = nrm;
+        S.out_lnorm[slot] = im * S.delta_r;
+        if (health) S.flags |= health;
+    } else {
+        S.out_ip[(size_t)slot * S.n_basis + b] = cmk(re * S.delta_r, im * S.delta_r);
     }
 }
+
+__device__ __forceinline__ void sh_observe_block(const ShObs& obs) {
+    const int job = blockIdx.x * (blockDim.x / TDSE_WAVE) + threadIdx.x / TDSE_WAVE;
+    if (job >= obs.n_jobs) return;
+    const int2 jb = obs.jobs[job];
+    const int lane = threadIdx.x % TDSE_WAVE;
+    if (jb.y != -3) sh_observe_job(obs.sims[jb.x], jb.y, lane);
+    else if (lane == 0) sh_count_step(obs.sims[jb.x], *obs.ctl);
+}
+
+__global__ void __launch_bounds__(256) k_sh_observe(ShObs obs) { sh_observe_block(obs); }
 
 // ------------------------------------------------------------------ R-phase
 
@@ -452,14 +487,18 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 
 template <int M, int MAXT, int WPE, int FORM>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
-k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines) {
+k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, ShObs obs) {
     extern __shared__ double2 lds[];  // 3 * P, then M * P for CN_CAYLEY_LDS
+    if ((int)blockIdx.x < obs.blocks) {
+        sh_observe_block(obs);
+        return;
+    }
     // consecutive l-lines of a simulation (which share its coefficient rows) on one XCD
-    const int line = xcd_remap(blockIdx.x, gridDim.x);
+    const int line = xcd_remap(blockIdx.x - obs.blocks, gridDim.x - obs.blocks);
     if (line >= n_lines) return;
     const int2 lt = lines[line];
     ShSim& S = sims[lt.x];
-    const int n = S.step;
+    const int n = S.rstep;
     if (!S.active || n >= S.N) return;  // uniform across the block
     const int l = lt.y;
     const int P = S.P, npad = S.npad;
@@ -488,8 +527,8 @@ k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_line
 #pragma unroll
         for (int i = 0; i < M; ++i) x[i] = (FORM == CN_CAYLEY_MEM) ? ld2(gl, (size_t)i * P) : ld2s(gl, (size_t)i * P);
     }
-    auto diag = [&](int i, double T) {
-        const int j = k * M + i;
+    auto diag = [&](int i, double T, int kk) {
+        const int j = kk * M + i;
         const double r = fma((double)j, dr, 0.5 * dr);
         const double U = (j < nr) ? cu * tdse_rcp(r * r) : 0.0;
         return sn * (fma(ll1, U, T) + (i == 0 ? c0 : 0.0));
@@ -497,20 +536,22 @@ k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_line
     double carry = a_left;  // A_{j-1} of the next row (pass 1 visits rows in order)
     auto coef = [&](int i, double& hm, double& h, double& hp) {
         const double2 tv = ld2(TA, (size_t)i * P);
-        h = diag(i, tv.x);
+        h = diag(i, tv.x, k);
         hm = sn * carry;
         hp = sn * tv.y;
         carry = tv.y;
     };
     // Second read of the same coefficients (pass 2, rows in order). The empty
-    // asm makes the pointer opaque so the compiler reloads instead of keeping
-    // the first pass's values live across the solver's barriers.
+    // asm makes the pointer and the chunk opaque so the compiler reloads (and forms
+    // r_j again) instead of keeping the first pass's values live across the
+    // solver's barriers.
     double carry2 = a_left;
     auto coef2 = [&](int i, double& hm, double& h) {
         const double2* TA2 = TA;
-        asm volatile("" : "+v"(TA2));
+        int k2 = k;
+        asm volatile("" : "+v"(TA2), "+v"(k2));
         const double2 tv = ld2(TA2, (size_t)i * P);
-        h = diag(i, tv.x);
+        h = diag(i, tv.x, k2);
         hm = sn * carry2;
         carry2 = tv.y;
     };
@@ -613,7 +654,7 @@ __global__ void __launch_bounds__(512) k_sh_vphase(ShSim* __restrict__ sims, con
     if (pair >= n_pairs) return;
     const int2 pt = pairs[pair];
     ShSim& S = sims[pt.x];
-    const int n = S.step;
+    const int n = S.rstep;
     if (!S.active || n >= S.N) return;  // uniform across the block
     const double fn = ld1(S.fs, n);
     if (fn == 0.0) return;  // every angle is zero: the factor is the identity
@@ -748,7 +789,7 @@ k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int 
     if (job >= n_pairs) return;
     const int2 pt = pairs[job];
     ShSim& S = sims[pt.x];
-    const int n = S.step;
+    const int n = S.rstep;
     if (!S.active || n >= S.N) return;  // uniform across the block
     const int P = S.P, npad = S.npad;
     const int ln = threadIdx.x & 1, k = threadIdx.x >> 1;
@@ -833,13 +874,18 @@ k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int 
 // products are the ones those two sweeps would form.
 template <int M, int MAXT, int WPE, bool EXPL>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
-k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const int* __restrict__ ctl) {
+k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const int* __restrict__ ctl,
+           ShObs obs) {
     extern __shared__ double2 lds[];  // 3 * P
-    const int line = xcd_remap(blockIdx.x, gridDim.x);
+    if ((int)blockIdx.x < obs.blocks) {
+        sh_observe_block(obs);
+        return;
+    }
+    const int line = xcd_remap(blockIdx.x - obs.blocks, gridDim.x - obs.blocks);
     if (line >= n_lines) return;
     const int2 lt = lines[line];
     ShSim& S = sims[lt.x];
-    const int n = S.step;
+    const int n = S.rstep;
     if (!S.active || n >= S.N) return;  // uniform across the block
     if (EXPL && S.ahead) return;         // applied by the previous replay's implicit sweep
     const int l = lt.y;
@@ -949,7 +995,7 @@ __global__ void __launch_bounds__(256) k_sh_adi_l(ShSim* __restrict__ sims, cons
     if (wave >= n_waves) return;
     const int2 wt = waves[wave];
     ShSim& S = sims[wt.x];
-    const int n = S.step;
+    const int n = S.rstep;
     if (!S.active || n >= S.N) return;
     const int L = S.L, P = S.P, m = S.m, npad = S.npad;
     const int p = wt.y + lane;
@@ -1006,7 +1052,7 @@ __global__ void __launch_bounds__(kAdiLanes * kAdiChunks) k_sh_adi_lp(ShSim* __r
     if (job >= n_groups) return;
     const int2 gt = groups[job];
     ShSim& S = sims[gt.x];
-    const int n = S.step;
+    const int n = S.rstep;
     if (!S.active || n >= S.N) return;  // uniform across the block
     const int t = threadIdx.x;
     const int ln = t % LANES, c = t / LANES;
@@ -1040,17 +1086,5 @@ __global__ void __launch_bounds__(kAdiLanes * kAdiChunks) k_sh_adi_lp(ShSim* __r
     for (int i = 0; i < M; ++i) {
         const int l = c * M + i;
         if (l < L) st2s(g, (size_t)l * npad, x[i]);
-    }
-}
-
-// Advance every active simulation's step counter after a full graph step.
-__global__ void k_sh_advance(ShSim* sims, int n_sims, const int* __restrict__ ctl) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < n_sims && sims[s].active && sims[s].step <= sims[s].N) {
-        ShSim& S = sims[s];
-        // the same decision as this replay's implicit ADI r-sweep
-        S.ahead = (S.adi && S.step < S.N && sh_adi_ahead(S, S.step, *ctl)) ? 1 : 0;
-        S.step += 1;
-        S.phase = 0;
     }
 }
