@@ -147,6 +147,7 @@ struct Bucket {
     int P = 0;
     bool imag = false;  // Line: complex time steps (imaginary-time relaxation)
     int method = 0;     // Line: LINE_ADI, LINE_SIO_LEN or LINE_SIO_VEL
+    size_t lds = 0;     // Line, M == 0 (any layouts): dynamic LDS of the launch
     int Mr = 0, Cr = 0, lanes = 1;  // cylindrical rho-sweep: rows per thread, chunks, lines per workgroup
     DevVec<int2> lines;   // SH: (slot, l); Line: (slot, 0); Cyl z-sweep: (slot, pair of rho-lines)
     DevVec<int2> rlines;  // Cyl rho-sweep: (slot, position group)
@@ -189,6 +190,7 @@ int n_data_points(int N, int every) {
 
 struct tdse_ctx {
     int device = 0;
+    int cus = 0;  // compute units
     hipStream_t stream = nullptr;
     Arena arena;
     std::string err;
@@ -202,7 +204,8 @@ struct tdse_ctx {
     std::vector<Bucket> cyl_buckets;  // by (z and rho layout)
     double* d_cl = nullptr;
     double* d_clv = nullptr;  // c_l (l + 1): the velocity gauge's h1 coupling per l
-    int* d_ctl = nullptr;     // [1] nonzero while the next replay of the current run follows (ADI run-ahead)
+    int* d_ctl = nullptr;     // [0] nonzero while the next replay of the current run follows (ADI run-ahead);
+                              // [1] a tridiagonal line that was split has to be solved as one run
     DevVec<ShWave> waves;     // length-gauge simulations' waves first, then velocity-gauge ones
     int n_len_waves = 0;
     DevVec<int2> jobs;      // SH observations, and the step counts of all but the ADI simulations
@@ -275,12 +278,15 @@ void drop_graph(tdse_ctx* ctx) {
     ctx->graph_k = nullptr;
 }
 
+size_t line_lds_bytes(int M, int P, bool real_steps);
+
 // Rebuild the ragged work tables from the live simulations.
 int rebuild_tables(tdse_ctx* ctx) {
     std::vector<ShWave> waves;
     std::vector<int2> jobs, ajobs;
     ctx->n_len_waves = -1;
     std::map<std::pair<int, int>, std::vector<int2>> shb, lnb;  // (rows, chunks [+ 4096 if complex steps])
+    std::map<std::pair<bool, int>, std::vector<int>> lna;       // lines of any layout, (complex steps, method)
     std::map<std::pair<int, int>, std::vector<int2>> vpb[2];    // velocity l-pairs by parity, (rows, chunks)
     std::map<std::pair<int, int>, std::vector<int2>> fpb;       // velocity odd l-pairs solved in one workgroup
     std::map<std::pair<int, int>, std::vector<int2>> adb;       // ADI l-lines, (rows, chunks)
@@ -339,10 +345,15 @@ int rebuild_tables(tdse_ctx* ctx) {
             }
     }
     if (ctx->n_len_waves < 0) ctx->n_len_waves = (int)waves.size();
+    int n_lines = 0;
+    for (const LineHost& h : ctx->line) n_lines += h.live;
+    // at most one line per CU: one launch for all layouts of a method (bucket M == 0)
+    const bool any_layout = n_lines <= ctx->cus;
     for (int s = 0; s < (int)ctx->line.size(); ++s) {
         const LineHost& h = ctx->line[s];
         if (!h.live) continue;
-        lnb[{h.dev.m, h.dev.P + (h.complex_steps ? 4096 : 0) + 8192 * h.dev.method}].push_back(make_int2(s, 0));
+        if (any_layout) lna[{h.complex_steps, h.dev.method}].push_back(s);
+        else lnb[{h.dev.m, h.dev.P + (h.complex_steps ? 4096 : 0) + 8192 * h.dev.method}].push_back(make_int2(s, 0));
     }
     std::vector<int2> cjobs, ccount;
     std::map<std::array<int, 5>, std::pair<std::vector<int2>, std::vector<int2>>> cyb;  // (Mz, Pz, Mr, Cr, lanes)
@@ -393,6 +404,27 @@ int rebuild_tables(tdse_ctx* ctx) {
         if (it != fpb.end() && (rc = devvec_upload(ctx, b.fpairs, it->second))) return rc;
     }
     if ((rc = fill(ctx->line_buckets, lnb))) return rc;
+    for (auto& kv : lna) {
+        ctx->line_buckets.emplace_back();
+        Bucket& b = ctx->line_buckets.back();
+        b.imag = kv.first.first;
+        b.method = kv.first.second;
+        // longest lines first; one layout keeps its own instance (fewer registers, exact block size)
+        std::stable_sort(kv.second.begin(), kv.second.end(),
+                         [&](int x, int y) { return ctx->line[x].dev.npad > ctx->line[y].dev.npad; });
+        std::vector<int2> ids;
+        bool one_layout = true;
+        const LineSim& first = ctx->line[kv.second[0]].dev;
+        for (int s : kv.second) {
+            const LineSim& S = ctx->line[s].dev;
+            ids.push_back(make_int2(s, 0));
+            one_layout = one_layout && S.m == first.m && S.P == first.P;
+            b.P = std::max(b.P, S.P);
+            b.lds = std::max(b.lds, line_lds_bytes(S.m, S.P, !b.imag));
+        }
+        b.M = one_layout ? first.m : 0;
+        if ((rc = devvec_upload(ctx, b.lines, ids))) return rc;
+    }
     for (auto& b : ctx->cyl_buckets) free_bucket(b);
     ctx->cyl_buckets.clear();
     for (auto& kv : cyb) {
@@ -582,34 +614,63 @@ void dispatch_vphase(tdse_ctx* ctx, const Bucket& b, int par, hipStream_t st) {
     }
 }
 
-template <int M, bool IMAG, int METHOD>
-void launch_line(tdse_ctx* ctx, const Bucket& b, int n_steps) {
-    const size_t lds = (size_t)line_lds_rows(M, IMAG) * b.P * sizeof(double2) + 64 * sizeof(double);
-    hipLaunchKernelGGL((k_line_steps<M, 512, IMAG, METHOD>), dim3((unsigned)b.lines.count), dim3(b.P), lds,
-                       ctx->stream, ctx->d_line, b.lines.ptr, (int)b.lines.count, n_steps);
+size_t line_lds_bytes(int M, int P, bool real_steps) {
+    return (size_t)line_lds_rows(M, real_steps) * P * sizeof(double2) + 64 * sizeof(double);
 }
 
+template <int M, bool IMAG, int METHOD>
+void launch_line(tdse_ctx* ctx, const Bucket& b, int n_steps, hipStream_t st) {
+    hipLaunchKernelGGL((k_line_steps<M, 512, IMAG, METHOD>), dim3((unsigned)b.lines.count), dim3(b.P),
+                       line_lds_bytes(M, b.P, IMAG), st, ctx->d_line, b.lines.ptr, (int)b.lines.count, n_steps);
+}
+
+// b.M == 0: lines of any layouts (k_line_steps_any), b.P the most threads and b.lds the most LDS of any of them
 template <bool IMAG, int METHOD>
-void dispatch_line_m(tdse_ctx* ctx, const Bucket& b, int n_steps) {
+void dispatch_line_m(tdse_ctx* ctx, const Bucket& b, int n_steps, hipStream_t st) {
     switch (b.M) {
-        case 2: launch_line<2, IMAG, METHOD>(ctx, b, n_steps); break;
-        case 4: launch_line<4, IMAG, METHOD>(ctx, b, n_steps); break;
-        case 6: launch_line<6, IMAG, METHOD>(ctx, b, n_steps); break;
-        case 8: launch_line<8, IMAG, METHOD>(ctx, b, n_steps); break;
-        case 10: launch_line<10, IMAG, METHOD>(ctx, b, n_steps); break;
-        case 12: launch_line<12, IMAG, METHOD>(ctx, b, n_steps); break;
-        case 14: launch_line<14, IMAG, METHOD>(ctx, b, n_steps); break;
-        default: launch_line<16, IMAG, METHOD>(ctx, b, n_steps); break;
+        case 0:
+            hipLaunchKernelGGL((k_line_steps_any<512, IMAG, METHOD>), dim3((unsigned)b.lines.count), dim3(b.P), b.lds,
+                               st, ctx->d_line, b.lines.ptr, (int)b.lines.count, n_steps);
+            break;
+        case 2: launch_line<2, IMAG, METHOD>(ctx, b, n_steps, st); break;
+        case 4: launch_line<4, IMAG, METHOD>(ctx, b, n_steps, st); break;
+        case 6: launch_line<6, IMAG, METHOD>(ctx, b, n_steps, st); break;
+        case 8: launch_line<8, IMAG, METHOD>(ctx, b, n_steps, st); break;
+        case 10: launch_line<10, IMAG, METHOD>(ctx, b, n_steps, st); break;
+        case 12: launch_line<12, IMAG, METHOD>(ctx, b, n_steps, st); break;
+        case 14: launch_line<14, IMAG, METHOD>(ctx, b, n_steps, st); break;
+        default: launch_line<16, IMAG, METHOD>(ctx, b, n_steps, st); break;
     }
 }
 
 // complex time steps take the general instance (ADI only: the host rejects the
 // split operator with complex steps)
-void dispatch_line(tdse_ctx* ctx, const Bucket& b, int n_steps) {
-    if (b.imag) dispatch_line_m<false, LINE_ADI>(ctx, b, n_steps);
-    else if (b.method == LINE_SIO_LEN) dispatch_line_m<true, LINE_SIO_LEN>(ctx, b, n_steps);
-    else if (b.method == LINE_SIO_VEL) dispatch_line_m<true, LINE_SIO_VEL>(ctx, b, n_steps);
-    else dispatch_line_m<true, LINE_ADI>(ctx, b, n_steps);
+void dispatch_line(tdse_ctx* ctx, const Bucket& b, int n_steps, hipStream_t st) {
+    if (b.imag) dispatch_line_m<false, LINE_ADI>(ctx, b, n_steps, st);
+    else if (b.method == LINE_SIO_LEN) dispatch_line_m<true, LINE_SIO_LEN>(ctx, b, n_steps, st);
+    else if (b.method == LINE_SIO_VEL) dispatch_line_m<true, LINE_SIO_VEL>(ctx, b, n_steps, st);
+    else dispatch_line_m<true, LINE_ADI>(ctx, b, n_steps, st);
+}
+
+// Run `launch(bucket, stream)` for every bucket over the context stream and the side streams (round robin),
+// forked and joined by events: the buckets hold different simulations.
+template <class F>
+int fan_out(tdse_ctx* ctx, const std::vector<Bucket>& bs, F&& launch) {
+    if (ctx->profiling || bs.size() < 2) {
+        for (auto& b : bs) launch(b, ctx->stream);
+        return TDSE_OK;
+    }
+    HIP_TRY(ctx, hipEventRecord(ctx->ev_fork, ctx->stream));
+    for (int j = 0; j < kSideStreams; ++j) HIP_TRY(ctx, hipStreamWaitEvent(ctx->side[j], ctx->ev_fork, 0));
+    for (size_t i = 0; i < bs.size(); ++i) {
+        const int j = (int)(i % (kSideStreams + 1));
+        launch(bs[i], j == 0 ? ctx->stream : ctx->side[j - 1]);
+    }
+    for (int j = 0; j < kSideStreams; ++j) {
+        HIP_TRY(ctx, hipEventRecord(ctx->ev_join[j], ctx->side[j]));
+        HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, ctx->ev_join[j], 0));
+    }
+    return TDSE_OK;
 }
 
 // The cylindrical observation jobs as leading workgroups of a launch of `threads` per workgroup.
@@ -753,43 +814,27 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
         // Within each of the three sweeps the buckets are independent: they run concurrently
         // over the context stream and the side streams (fork and join by events), and each
         // sweep starts after the whole previous one.
-        auto fan = [&](std::vector<Bucket>& bs, auto&& launch) -> int {
-            if (ctx->profiling || bs.size() < 2) {
-                for (auto& b : bs) launch(b, ctx->stream);
-                return TDSE_OK;
-            }
-            HIP_TRY(ctx, hipEventRecord(ctx->ev_fork, ctx->stream));
-            for (int j = 0; j < kSideStreams; ++j) HIP_TRY(ctx, hipStreamWaitEvent(ctx->side[j], ctx->ev_fork, 0));
-            for (size_t i = 0; i < bs.size(); ++i) {
-                const int j = (int)(i % (kSideStreams + 1));
-                launch(bs[i], j == 0 ? ctx->stream : ctx->side[j - 1]);
-            }
-            for (int j = 0; j < kSideStreams; ++j) {
-                HIP_TRY(ctx, hipEventRecord(ctx->ev_join[j], ctx->side[j]));
-                HIP_TRY(ctx, hipStreamWaitEvent(ctx->stream, ctx->ev_join[j], 0));
-            }
-            return TDSE_OK;
-        };
         if (!ctx->sh_adi_buckets.empty()) {
             int rc;
             const Bucket* first = rider ? nullptr : &ctx->sh_adi_buckets[0];
-            if ((rc = fan(ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) {
+            if ((rc = fan_out(ctx, ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) {
                     dispatch_adi_r<true>(ctx, b, st, ride && &b == first);
                 })))
                 return rc;
-            if ((rc = fan(ctx->sh_adi_lbuckets, [&](const Bucket& b, hipStream_t st) { dispatch_adi_lp(ctx, b, st); })))
+            if ((rc = fan_out(ctx, ctx->sh_adi_lbuckets, [&](const Bucket& b, hipStream_t st) { dispatch_adi_lp(ctx, b, st); })))
                 return rc;
             const int na = (int)ctx->adi_waves.count;
             if (na > 0)
                 hipLaunchKernelGGL(k_sh_adi_l, dim3((na * TDSE_WAVE + 255) / 256), dim3(256), 0, ctx->stream,
                                    ctx->d_sh, ctx->adi_waves.ptr, na, ctx->d_cl);
-            if ((rc = fan(ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) {
+            if ((rc = fan_out(ctx, ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) {
                     dispatch_adi_r<false>(ctx, b, st, &b == &ctx->sh_adi_buckets[0]);
                 })))
                 return rc;
         }
     }
-    for (auto& b : ctx->line_buckets) dispatch_line(ctx, b, 1);
+    if (int rc = fan_out(ctx, ctx->line_buckets, [&](const Bucket& b, hipStream_t st) { dispatch_line(ctx, b, 1, st); }))
+        return rc;
     if (!ctx->cyl_buckets.empty()) {
         if (cyl_pre) {
             for (auto& b : ctx->cyl_buckets) dispatch_cyl_rho(ctx, b, ctx->stream, CYL_PRE, false);
@@ -892,6 +937,32 @@ double2* device_scratch(int device, hipError_t* err) {
     return g_scratch_ptr[device];
 }
 
+// Thomas solves of n_systems lines (lengths on the host and, as len, on the device). A line gets one wave for
+// every kTdmaSpan rows, of which those find work whose rows hold a restart (k_tdma_lines); the span
+// grows where that would be more than kTdmaWaves workgroups. A second launch redoes every line as one run if
+// a split line met a value that is not finite.
+constexpr int64_t kTdmaSpan = 64, kTdmaWaves = int64_t(1) << 20;
+hipError_t launch_tdma(tdse_ctx* ctx, const double2* a, const double2* b, const double2* c, const double2* d,
+                       double2* x, double2* cp, const int64_t* off, const int64_t* len, const int64_t* lengths,
+                       int64_t n_systems) {
+    int64_t longest = 1;
+    for (int64_t i = 0; i < n_systems; ++i) longest = std::max(longest, lengths[i]);
+    const int64_t most = std::max<int64_t>(1, kTdmaWaves / n_systems);  // waves per line
+    const int64_t span = std::max(kTdmaSpan, (longest + most - 1) / most);
+    const int64_t per_line = (longest + span - 1) / span;
+    int* redo = ctx->d_ctl + 1;
+    hipError_t e = hipSuccess;
+    if (per_line > 1) e = hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(redo), 0, 1, ctx->stream);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_tdma_lines, dim3((unsigned)(n_systems * per_line)), dim3(TDSE_WAVE), 0, ctx->stream, a, b, c, d,
+                       x, cp, off, len, n_systems, span, per_line, 0, redo);
+    e = hipGetLastError();
+    if (e != hipSuccess || per_line == 1) return e;
+    hipLaunchKernelGGL(k_tdma_lines, dim3((unsigned)n_systems), dim3(TDSE_WAVE), 0, ctx->stream, a, b, c, d, x, cp, off,
+                       len, n_systems, longest, int64_t(1), 1, redo);
+    return hipGetLastError();
+}
+
 void free_blocks(tdse_ctx* ctx, std::vector<void*>& blocks) {
     for (void* p : blocks) ctx->arena.dealloc(p);
     blocks.clear();
@@ -917,6 +988,7 @@ int tdse_ctx_create(int device, size_t pool_bytes, tdse_ctx** out) {
     if (hipSetDevice(device) != hipSuccess) return fail(nullptr, TDSE_ERR_HIP, "hipSetDevice failed");
     tdse_ctx* ctx = new tdse_ctx();
     ctx->device = device;
+    if (hipDeviceGetAttribute(&ctx->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) ctx->cus = 0;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
         delete ctx;
         return fail(nullptr, TDSE_ERR_HIP, "hipStreamCreate failed");
@@ -936,7 +1008,7 @@ int tdse_ctx_create(int device, size_t pool_bytes, tdse_ctx** out) {
               hipMalloc(&ctx->d_clv, kMaxL * sizeof(double)) == hipSuccess &&
               hipMemcpy(ctx->d_clv, clv.data(), kMaxL * sizeof(double), hipMemcpyHostToDevice) == hipSuccess &&
               hipMalloc(&ctx->d_sh, kSlotCapacity * sizeof(ShSim)) == hipSuccess &&
-              hipMalloc(&ctx->d_ctl, sizeof(int)) == hipSuccess && hipMemset(ctx->d_ctl, 0, sizeof(int)) == hipSuccess &&
+              hipMalloc(&ctx->d_ctl, 2 * sizeof(int)) == hipSuccess && hipMemset(ctx->d_ctl, 0, 2 * sizeof(int)) == hipSuccess &&
               hipMalloc(&ctx->d_line, kSlotCapacity * sizeof(LineSim)) == hipSuccess &&
               hipMalloc(&ctx->d_cyl, kSlotCapacity * sizeof(CylSim)) == hipSuccess &&
               hipMemset(ctx->d_sh, 0, kSlotCapacity * sizeof(ShSim)) == hipSuccess &&
@@ -1065,11 +1137,7 @@ int tdse_tdma_batched(tdse_ctx* ctx, const double* sub, const double* diag, cons
         free_blocks(ctx, blocks);
         return rc;
     }
-    const int threads = 64;
-    const int64_t grid = (n_systems + threads - 1) / threads;
-    hipLaunchKernelGGL(k_tdma_lines, dim3((unsigned)grid), dim3(threads), 0, ctx->stream, da, db, dc, dd, dx, dcp, doff,
-                       dlen, n_systems);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_tdma(ctx, da, db, dc, dd, dx, dcp, doff, dlen, lengths, n_systems);
     if (e == hipSuccess) e = hipMemcpyAsync(x, dx, n * sizeof(double2), hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->stream);
@@ -1112,13 +1180,9 @@ int tdse_tdma_batched_noalloc(tdse_ctx* ctx, const double* sub, const double* di
     const size_t nb = (size_t)n_systems * sizeof(int64_t);
     HIP_TRY(ctx, hipMemcpyAsync(doff, offsets, nb, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(dlen, lengths, nb, hipMemcpyHostToDevice, ctx->stream));
-    const int threads = 64;
-    const int64_t grid = (n_systems + threads - 1) / threads;
-    hipLaunchKernelGGL(k_tdma_lines, dim3((unsigned)grid), dim3(threads), 0, ctx->stream,
-                       reinterpret_cast<const double2*>(sub), reinterpret_cast<const double2*>(diag),
-                       reinterpret_cast<const double2*>(sup), reinterpret_cast<const double2*>(d),
-                       reinterpret_cast<double2*>(x), cp, doff, dlen, n_systems);
-    HIP_TRY(ctx, hipGetLastError());
+    HIP_TRY(ctx, launch_tdma(ctx, reinterpret_cast<const double2*>(sub), reinterpret_cast<const double2*>(diag),
+                             reinterpret_cast<const double2*>(sup), reinterpret_cast<const double2*>(d),
+                             reinterpret_cast<double2*>(x), cp, doff, dlen, lengths, n_systems));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return TDSE_OK;
 }
@@ -1513,7 +1577,9 @@ int tdse_line_run(tdse_ctx* ctx, int32_t n_steps) {
     int rc;
     if (ctx->dirty && (rc = rebuild_tables(ctx))) return rc;
     HIP_TRY(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
-    for (auto& b : ctx->line_buckets) dispatch_line(ctx, b, n_steps);
+    if ((rc = fan_out(ctx, ctx->line_buckets,
+                      [&](const Bucket& b, hipStream_t st) { dispatch_line(ctx, b, n_steps, st); })))
+        return rc;
     HIP_TRY(ctx, hipGetLastError());
     HIP_TRY(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
     HIP_TRY(ctx, hipEventSynchronize(ctx->ev_stop));

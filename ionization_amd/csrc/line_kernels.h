@@ -122,15 +122,15 @@ __device__ __forceinline__ int line_data_slot(int n, int N, int every) {
     return n == 0 ? 0 : 1;
 }
 
-// Block-wide sum in a fixed order (deterministic for a given block size).
-__device__ __forceinline__ double block_sum(double v, double* red) {
+// Sum over the line's P threads in a fixed order.
+__device__ __forceinline__ double block_sum(double v, double* red, const int P) {
     const int t = threadIdx.x;
     v = wave_sum(v);
     __syncthreads();
     if ((t % TDSE_WAVE) == 0) red[t / TDSE_WAVE] = v;
     __syncthreads();
     double tot = 0.0;
-    const int nw = (blockDim.x + TDSE_WAVE - 1) / TDSE_WAVE;
+    const int nw = P / TDSE_WAVE;
     for (int w = 0; w < nw; ++w) tot += red[w];
     return tot;
 }
@@ -141,7 +141,7 @@ __device__ __forceinline__ void line_observe(LineSim& S, const double2 (&x)[M], 
     double acc = 0.0;
 #pragma unroll
     for (int i = 0; i < M; ++i) acc += cabs2(x[i]);
-    const double nrm = block_sum(acc, red);
+    const double nrm = block_sum(acc, red, P);
     if (threadIdx.x == 0) {
         const int health = norm_health(S.out_norm, slot, nrm * S.delta_z);
         S.out_norm[slot] = nrm * S.delta_z;
@@ -157,8 +157,8 @@ __device__ __forceinline__ void line_observe(LineSim& S, const double2 (&x)[M], 
             re += f.x * x[i].x + f.y * x[i].y;
             im += f.x * x[i].y - f.y * x[i].x;
         }
-        const double sre = block_sum(re, red);
-        const double sim = block_sum(im, red);
+        const double sre = block_sum(re, red, P);
+        const double sim = block_sum(im, red, P);
         if (threadIdx.x == 0) S.out_ip[(size_t)slot * S.n_basis + b] = cmk(sre * S.delta_z, sim * S.delta_z);
     }
 }
@@ -169,17 +169,14 @@ constexpr bool line_alpha_lds(int M) { return M >= 10; }
 // LDS rows of P double2 that the solver uses (the reduction scratch follows them)
 constexpr int line_lds_rows(int M, bool IMAG) { return (IMAG && line_alpha_lds(M)) ? 3 + M - 2 : 3; }
 
-// blockDim.x == P and m == M for every simulation launched together; one block per simulation.
+// m == M; the P threads of the line call this together, one line per workgroup.
 // IMAG: every w_n is purely imaginary (real time steps), which halves the
 // coefficient arithmetic; imaginary-time relaxation uses the general path.
 // METHOD: the step of every simulation of the launch (LINE_ADI, LINE_SIO_LEN,
 // LINE_SIO_VEL; the split operator only with IMAG).
-template <int M, int MAXT, bool IMAG, int METHOD>
-__global__ void __launch_bounds__(MAXT) k_line_steps(LineSim* __restrict__ sims, const int2* __restrict__ ids,
-                                                     int n_ids, int n_steps) {
-    extern __shared__ double2 lds[];  // the solver's line_lds_rows(M, IMAG) * P double2, then reduction scratch
-    if ((int)blockIdx.x >= n_ids) return;
-    LineSim& S = sims[ids[blockIdx.x].x];
+// lds: the solver's line_lds_rows(M, IMAG) * P double2, then 64 doubles of reduction scratch.
+template <int M, bool IMAG, int METHOD>
+__device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double2* __restrict__ lds) {
     if (!S.active) return;
     int n = S.step;
     const int N = S.N;
@@ -270,7 +267,7 @@ __global__ void __launch_bounds__(MAXT) k_line_steps(LineSim* __restrict__ sims,
             double acc = 0.0;
 #pragma unroll
             for (int i = 0; i < M; ++i) acc += cabs2(x[i]);
-            const double inv = 1.0 / sqrt(block_sum(acc, red) * S.delta_z);
+            const double inv = 1.0 / sqrt(block_sum(acc, red, P) * S.delta_z);
 #pragma unroll
             for (int i = 0; i < M; ++i) x[i] = cscale(inv, x[i]);
         }
@@ -285,4 +282,37 @@ __global__ void __launch_bounds__(MAXT) k_line_steps(LineSim* __restrict__ sims,
     for (int i = 0; i < M; ++i) st2(gs, (size_t)i * P, x[i]);
     __syncthreads();
     if (k == 0) S.step = (n == N) ? N + 1 : n;
+}
+
+// Lines of one layout: blockDim.x == P and m == M for every simulation launched together.
+template <int M, int MAXT, bool IMAG, int METHOD>
+__global__ void __launch_bounds__(MAXT) k_line_steps(LineSim* __restrict__ sims, const int2* __restrict__ ids,
+                                                     int n_ids, int n_steps) {
+    extern __shared__ double2 lds[];
+    if ((int)blockIdx.x >= n_ids) return;
+    line_steps<M, IMAG, METHOD>(sims[ids[blockIdx.x].x], n_steps, lds);
+}
+
+// Lines of any layouts in one launch, for batches of at most one line per CU: a line is bound by the
+// latency of its own chain of steps, so lines of different layouts gain nothing from launches of their
+// own, one after another. The workgroup has the longest line's threads; the whole waves past a line's P leave
+// before any barrier (s_barrier waits for the surviving waves only). 24 lines of 800 to 8192 points, velocity
+// gauge: 108.9 us per step as a launch for each layout, 16.3 with this one.
+template <int MAXT, bool IMAG, int METHOD>
+__global__ void __launch_bounds__(MAXT) k_line_steps_any(LineSim* __restrict__ sims, const int2* __restrict__ ids,
+                                                         int n_ids, int n_steps) {
+    extern __shared__ double2 lds[];
+    if ((int)blockIdx.x >= n_ids) return;
+    LineSim& S = sims[ids[blockIdx.x].x];
+    if ((int)threadIdx.x >= S.P) return;
+    switch (S.m) {
+        case 2: line_steps<2, IMAG, METHOD>(S, n_steps, lds); break;
+        case 4: line_steps<4, IMAG, METHOD>(S, n_steps, lds); break;
+        case 6: line_steps<6, IMAG, METHOD>(S, n_steps, lds); break;
+        case 8: line_steps<8, IMAG, METHOD>(S, n_steps, lds); break;
+        case 10: line_steps<10, IMAG, METHOD>(S, n_steps, lds); break;
+        case 12: line_steps<12, IMAG, METHOD>(S, n_steps, lds); break;
+        case 14: line_steps<14, IMAG, METHOD>(S, n_steps, lds); break;
+        default: line_steps<16, IMAG, METHOD>(S, n_steps, lds); break;
+    }
 }
