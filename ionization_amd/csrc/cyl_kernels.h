@@ -195,7 +195,7 @@ __global__ void __launch_bounds__(256) k_cyl_observe(CylJobs jobs) { cyl_job_blo
 template <int M, int MAXT, int WPE, int FORM>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, CylJobs jobs) {
-    extern __shared__ double2 lds[];  // 3 * Pz * 2, then M * Pz * 2 for CN_CAYLEY_LDS
+    extern __shared__ double2 lds[];  // 3 * Pz * 2 + kRedScratch
     if ((int)blockIdx.x < jobs.blocks) {
         cyl_job_block<false>(jobs);
         return;
@@ -272,7 +272,7 @@ __device__ __forceinline__ double cyl_block_sum(double v, double* red, int t, in
 template <int M, int LANES, int MODE, int MAXT, int WPE>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_cyl_rho(CylSim* __restrict__ sims, const int2* __restrict__ groups,
                                                   int n_groups, CylJobs jobs) {
-    extern __shared__ double2 lds[];  // 3 * Cr * LANES double2, then 16 doubles for reductions
+    extern __shared__ double2 lds[];  // 3 * Cr * LANES + kRedScratch double2, then 16 doubles for reductions
     if ((int)blockIdx.x < jobs.blocks) {
         if (MODE == CYL_MAIN) cyl_job_block<true>(jobs);
         return;
@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
     // rows c M .. c M + M - 1 (M even): row c M + i at gl[cyl_at(i, 0, npz)]; with the two
     // rows of a pair adjacent, LANES = 4 neighbouring positions read whole 128 B lines
     double2* __restrict__ gl = S.g + cyl_at(c * M, p, npz);
-    double* red = reinterpret_cast<double*>(lds + 3 * P * LANES);
+    double* red = reinterpret_cast<double*>(lds + 3 * P * LANES + kRedScratch);
 
     double2 x[M];
 #pragma unroll

@@ -483,10 +483,10 @@ void prof_end(tdse_ctx* ctx) {
 // default, else re-reading them. Chosen from kernel-trace timings.
 int cn_form(int M, int P) {
     if (M >= 10) return CN_EXPLICIT;
-    return (3 + M) * (size_t)P * sizeof(double2) <= 65536 ? CN_CAYLEY_LDS : CN_CAYLEY_MEM;
+    return ((3 + M) * (size_t)P + kRedScratch) * sizeof(double2) <= 65536 ? CN_CAYLEY_LDS : CN_CAYLEY_MEM;
 }
 size_t cn_lds_bytes(int M, int P, int form) {
-    return (size_t)(form == CN_CAYLEY_LDS ? 3 + M : 3) * P * sizeof(double2);
+    return ((size_t)(form == CN_CAYLEY_LDS ? 3 + M : 3) * P + kRedScratch) * sizeof(double2);
 }
 
 // A job list as leading workgroups of a launch of `threads` per workgroup (none: no jobs ride there).
@@ -529,7 +529,7 @@ void dispatch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) 
 
 template <int M, int MAXT, int WPE, bool EXPL>
 void launch_adi_r(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
-    const size_t lds = 3 * (size_t)b.P * sizeof(double2);
+    const size_t lds = (3 * (size_t)b.P + kRedScratch) * sizeof(double2);
     const ShObs obs = obs_of(ctx, EXPL ? ctx->jobs : ctx->adi_jobs, b.P, ride);
     hipLaunchKernelGGL((k_sh_adi_r<M, MAXT, WPE, EXPL>), dim3((unsigned)(b.lines.count + obs.blocks)), dim3(b.P), lds,
                        st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, ctx->d_ctl, obs);
@@ -552,7 +552,7 @@ void dispatch_adi_r(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
 
 template <int M>
 void launch_adi_lp(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
-    const size_t lds = 3 * (size_t)kAdiChunks * kAdiLanes * sizeof(double2);
+    const size_t lds = (3 * (size_t)kAdiChunks * kAdiLanes + kRedScratch) * sizeof(double2);
     hipLaunchKernelGGL(k_sh_adi_lp<M>, dim3((unsigned)b.lines.count), dim3(kAdiChunks * kAdiLanes), lds, st,
                        ctx->d_sh, b.lines.ptr, (int)b.lines.count, ctx->d_cl);
 }
@@ -573,7 +573,7 @@ void dispatch_adi_lp(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
 template <int M, int WPE>
 void launch_rphase_vpair(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
     // the reduced system (3 P) and alpha_i of rows 0 .. M - 3 (M - 2 P) per line, two lines
-    const size_t lds = (size_t)(3 + M - 2) * b.P * 2 * sizeof(double2);
+    const size_t lds = ((size_t)(3 + M - 2) * b.P * 2 + kRedScratch) * sizeof(double2);
     hipLaunchKernelGGL((k_sh_rphase_vpair<M, kMaxPairThreads, WPE>), dim3((unsigned)b.fpairs.count), dim3(2 * b.P),
                        lds, st, ctx->d_sh, b.fpairs.ptr, (int)b.fpairs.count, ctx->d_cl);
 }
@@ -615,7 +615,7 @@ void dispatch_vphase(tdse_ctx* ctx, const Bucket& b, int par, hipStream_t st) {
 }
 
 size_t line_lds_bytes(int M, int P, bool real_steps) {
-    return (size_t)line_lds_rows(M, real_steps) * P * sizeof(double2) + 64 * sizeof(double);
+    return ((size_t)line_lds_rows(M, real_steps) * P + kRedScratch) * sizeof(double2) + 64 * sizeof(double);
 }
 
 template <int M, bool IMAG, int METHOD>
@@ -684,7 +684,7 @@ CylJobs cyl_jobs_of(const tdse_ctx* ctx, const DevVec<int2>& list, int threads, 
 // rows 0.44 ms, keeping them in LDS 0.64 ms per sweep against 0.40 ms).
 template <int M, int MAXT, int WPE>
 void launch_cyl_z(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
-    const size_t lds = 2 * cn_lds_bytes(M, b.P, CN_EXPLICIT);
+    const size_t lds = cn_lds_bytes(M, 2 * b.P, CN_EXPLICIT);
     const CylJobs jobs = cyl_jobs_of(ctx, ctx->cyl_jobs, 2 * b.P, ride);
     hipLaunchKernelGGL((k_cyl_z<M, MAXT, WPE, CN_EXPLICIT>), dim3((unsigned)(b.lines.count + jobs.blocks)),
                        dim3(2 * b.P), lds, st, ctx->d_cyl, b.lines.ptr, (int)b.lines.count, jobs);
@@ -706,7 +706,7 @@ void dispatch_cyl_z(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
 template <int M, int LANES, int MAXT, int WPE>
 void launch_cyl_rho(tdse_ctx* ctx, const Bucket& b, hipStream_t st, int mode, bool ride) {
     const CylJobs jobs = cyl_jobs_of(ctx, ctx->cyl_count_jobs, b.Cr * LANES, ride);
-    const size_t lds = 3 * (size_t)b.Cr * LANES * sizeof(double2) + 16 * sizeof(double);
+    const size_t lds = (3 * (size_t)b.Cr * LANES + kRedScratch) * sizeof(double2) + 16 * sizeof(double);
     const dim3 grid((unsigned)(b.rlines.count + jobs.blocks)), block((unsigned)(b.Cr * LANES));
     if (mode == CYL_PRE)
         hipLaunchKernelGGL((k_cyl_rho<M, LANES, CYL_PRE, MAXT, WPE>), grid, block, lds, st, ctx->d_cyl,

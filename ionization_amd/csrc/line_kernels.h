@@ -174,7 +174,7 @@ constexpr int line_lds_rows(int M, bool IMAG) { return (IMAG && line_alpha_lds(M
 // coefficient arithmetic; imaginary-time relaxation uses the general path.
 // METHOD: the step of every simulation of the launch (LINE_ADI, LINE_SIO_LEN,
 // LINE_SIO_VEL; the split operator only with IMAG).
-// lds: the solver's line_lds_rows(M, IMAG) * P double2, then 64 doubles of reduction scratch.
+// lds: the solver's line_lds_rows(M, IMAG) * P + kRedScratch double2, then 64 doubles of reduction scratch.
 template <int M, bool IMAG, int METHOD>
 __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double2* __restrict__ lds) {
     if (!S.active) return;
@@ -183,7 +183,7 @@ __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double
     if (n > N) return;
     const int P = S.P, npad = S.npad;
     const int k = threadIdx.x;
-    double* red = reinterpret_cast<double*>(lds + line_lds_rows(M, IMAG) * P);
+    double* red = reinterpret_cast<double*>(lds + line_lds_rows(M, IMAG) * P + kRedScratch);
     double2* __restrict__ g = S.g + k;
     const double* __restrict__ H = S.tab + LN_H * npad + k;
     const double* __restrict__ AP = S.tab + LN_AP * npad + k;

@@ -15,13 +15,12 @@
 //    Y_k = y_{k m + m - 1}; the chunk's last row then gives one equation in
 //    (Y_{k-1}, Y_k, Y_{k+1}).
 //  * The P-unknown reduced system (every equation normalised to a unit
-//    diagonal) is solved in LDS by cyclic reduction (reduced_cr) or parallel
-//    cyclic reduction (reduced_pcr).
+//    diagonal) is solved in LDS (reduced_cr).
 //  * Each thread back-substitutes its rows.
 //
 // M is the exact number of rows per chunk (a compile-time constant, 2 <= M).
 // Requirements: all P threads of the line call this together
-// (block-wide barriers), lds holds 3 P double2 for this line. Rows beyond the
+// (block-wide barriers), lds holds 3 P double2 for this line and kRedScratch more. Rows beyond the
 // physical line are padding rows with H = 0 and x = 0 (they stay 0).
 #pragma once
 
@@ -38,58 +37,28 @@ __device__ __forceinline__ double2 wmul(double2 w, double2 v) {
 // coef(i, hm, h, hp): H_{j,j-1}, H_{j,j}, H_{j,j+1} of the thread's row i.
 // xl / xr: x_{km-1} and x_{km+m} (zero at the line ends).
 // The reduced system  a_k Y_{k-1} + Y_k + c_k Y_{k+1} = d_k,  k < P  (one equation
-// per thread, unit diagonal, a_0 = c_{P-1} = 0). Both solvers return Y_k and Y_{k-1}.
+// per thread, unit diagonal, a_0 = c_{P-1} = 0): returns Y_k and Y_{k-1}.
 //
-// Parallel cyclic reduction: ceil(log2 P) levels, every equation updated at every level.
-__device__ __forceinline__ void reduced_pcr(double2 A, double2 C, double2 D, const int k, const int P,
-                                            double2* __restrict__ lds, double2& Yk, double2& Ykm1) {
-    double2* pa = lds;
-    double2* pc = lds + P;
-    double2* pd = lds + 2 * P;
-    for (int s = 1; s < P; s <<= 1) {
-        __syncthreads();
-        pa[k] = A;
-        pc[k] = C;
-        pd[k] = D;
-        __syncthreads();
-        double2 am = cmk(0.0, 0.0), cm = cmk(0.0, 0.0), dm = cmk(0.0, 0.0);
-        double2 apl = cmk(0.0, 0.0), cpl = cmk(0.0, 0.0), dpl = cmk(0.0, 0.0);
-        if (k - s >= 0) {
-            am = pa[k - s];
-            cm = pc[k - s];
-            dm = pd[k - s];
-        }
-        if (k + s < P) {
-            apl = pa[k + s];
-            cpl = pc[k + s];
-            dpl = pd[k + s];
-        }
-        const double2 bn = csub(csub(cmk(1.0, 0.0), cmul(A, cm)), cmul(C, apl));
-        const double2 an2 = cneg(cmul(A, am));
-        const double2 cn2 = cneg(cmul(C, cpl));
-        const double2 dn2 = csub(csub(D, cmul(A, dm)), cmul(C, dpl));
-        const double2 ib = crecip(bn);
-        A = cmul(an2, ib);
-        C = cmul(cn2, ib);
-        D = cmul(dn2, ib);
-    }
-    __syncthreads();
-    pd[k] = D;
-    __syncthreads();
-    Yk = D;
-    Ykm1 = (k > 0) ? pd[k - 1] : cmk(0.0, 0.0);
-}
+// Cyclic reduction with compacted threads down to what one wave holds, parallel
+// cyclic reduction there, and the back substitution. At stride s the surviving
+// equations kk = 2 s (t + 1) - 1 are updated by threads t = 0, 1, ... (so whole waves
+// drop out as the system shrinks), eliminating kk - s and kk + s. Once the survivors
+// of the block's lines fit 64 lanes, the first wave finishes them without barriers:
+// log2 levels in which every lane updates its own equation, where cyclic reduction
+// would take as many levels up and again down at the same issue cost (a wave's
+// instruction costs the same with one lane active), each behind a block barrier. The
+// eliminated equations s (2 t + 1) - 1 then follow from their solved neighbours.
+// Against cyclic reduction throughout, us per step: one 8192-point line (P = 512) 12.2 ->
+// 10.5, 250 x 100 SH (P = 64) 17.2 -> 16.1, 250 x 100 cylinder 20.2 -> 18.4; R-phase of
+// the 256-simulation scan 0.98 -> 0.92 ms (serial).
+//
+// LANES > 1: LANES independent lines share the block, thread k LANES + ln on equation
+// k of line ln, which sits at LDS index k * LANES + ln (each array of 3 holds P * LANES
+// entries); all lines have the same P and step through the levels together. The
+// wave's own part takes kRedScratch more entries after them, contiguous so that
+// neighbouring lanes do not conflict.
+constexpr int kRedScratch = 3 * TDSE_WAVE;
 
-// Cyclic reduction with compacted threads: at stride s the surviving equations
-// kk = 2 s (t + 1) - 1 are updated by threads t = 0, 1, ... (so whole waves drop
-// out as the system shrinks), eliminating kk - s and kk + s; the back
-// substitution then solves the eliminated equations s (2 t + 1) - 1 from their
-// already solved neighbours. About 2 P equation updates in total instead of
-// P log2 P, at the same number of barriers.
-//
-// LANES > 1: LANES independent lines share the block, equation k of line ln at
-// LDS index k * LANES + ln (each array of 3 holds P * LANES entries); all lines
-// have the same P and step through the levels together.
 template <int LANES = 1>
 __device__ __forceinline__ void reduced_cr(double2 A, double2 C, double2 D, const int k, const int P,
                                            double2* __restrict__ lds, double2& Yk, double2& Ykm1,
@@ -97,35 +66,77 @@ __device__ __forceinline__ void reduced_cr(double2 A, double2 C, double2 D, cons
     double2* pa = lds + ln;
     double2* pc = lds + P * LANES + ln;
     double2* pd = lds + 2 * P * LANES + ln;
+    // a0 Y_- + Y + c0 Y_+ = d0 without its neighbours (am, cm, dm) and (apl, cpl, dpl)
+    auto eliminate = [](double2& a0, double2& c0, double2& d0, double2 am, double2 cm, double2 dm, double2 apl,
+                        double2 cpl, double2 dpl) {
+        const double2 bn = csub(csub(cmk(1.0, 0.0), cmul(a0, cm)), cmul(c0, apl));
+        const double2 an2 = cneg(cmul(a0, am));
+        const double2 cn2 = cneg(cmul(c0, cpl));
+        const double2 dn2 = csub(csub(d0, cmul(a0, dm)), cmul(c0, dpl));
+        const double2 ib = crecip(bn);
+        a0 = cmul(an2, ib);
+        c0 = cmul(cn2, ib);
+        d0 = cmul(dn2, ib);
+    };
     __syncthreads();
     pa[k * LANES] = A;
     pc[k * LANES] = C;
     pd[k * LANES] = D;
-    int s = 1;
-    for (; s < P; s <<= 1) {
+    int s = 1, left = P;  // equations s (t + 1) - 1, t < left, survive
+    for (; left * LANES > TDSE_WAVE; s <<= 1, left = P / s) {
         __syncthreads();
         const int kk = 2 * s * (k + 1) - 1;
         if (kk < P) {
             const int e = kk * LANES, em = (kk - s) * LANES, ep = (kk + s) * LANES;
-            const double2 a0 = pa[e], c0 = pc[e], d0 = pd[e];
-            const double2 am = pa[em], cm = pc[em], dm = pd[em];
+            double2 a0 = pa[e], c0 = pc[e], d0 = pd[e];
             double2 apl = cmk(0.0, 0.0), cpl = cmk(0.0, 0.0), dpl = cmk(0.0, 0.0);
             if (kk + s < P) {
                 apl = pa[ep];
                 cpl = pc[ep];
                 dpl = pd[ep];
             }
-            const double2 bn = csub(csub(cmk(1.0, 0.0), cmul(a0, cm)), cmul(c0, apl));
-            const double2 an2 = cneg(cmul(a0, am));
-            const double2 cn2 = cneg(cmul(c0, cpl));
-            const double2 dn2 = csub(csub(d0, cmul(a0, dm)), cmul(c0, dpl));
-            const double2 ib = crecip(bn);
-            pa[e] = cmul(an2, ib);
-            pc[e] = cmul(cn2, ib);
-            pd[e] = cmul(dn2, ib);
+            eliminate(a0, c0, d0, pa[em], pc[em], pd[em], apl, cpl, dpl);
+            pa[e] = a0;
+            pc[e] = c0;
+            pd[e] = d0;
         }
     }
-    // equations still standing have no neighbours in range: their d is their solution
+    __syncthreads();
+    const int t = k * LANES + ln;
+    if (t < TDSE_WAVE) {
+        double2* __restrict__ w = lds + 3 * P * LANES + t;
+        const double2 zero = cmk(0.0, 0.0);
+        const bool on = k < left;
+        const int e = (s * (k + 1) - 1) * LANES;
+        double2 a0 = zero, c0 = zero, d0 = zero;
+        if (on) {
+            a0 = pa[e];
+            c0 = pc[e];
+            d0 = pd[e];
+        }
+        for (int q = 1; q < left; q <<= 1) {
+            w[0] = a0;
+            w[TDSE_WAVE] = c0;
+            w[2 * TDSE_WAVE] = d0;
+            // one wave: its LDS operations complete in order, only the compiler has to keep it
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            double2 am = zero, cm = zero, dm = zero, apl = zero, cpl = zero, dpl = zero;
+            if (k >= q) {
+                am = w[-q * LANES];
+                cm = w[TDSE_WAVE - q * LANES];
+                dm = w[2 * TDSE_WAVE - q * LANES];
+            }
+            if (k + q < left) {
+                apl = w[q * LANES];
+                cpl = w[TDSE_WAVE + q * LANES];
+                dpl = w[2 * TDSE_WAVE + q * LANES];
+            }
+            __builtin_amdgcn_wave_barrier();
+            eliminate(a0, c0, d0, am, cm, dm, apl, cpl, dpl);
+        }
+        if (on) pd[e] = d0;  // no neighbours left: its d is its solution
+    }
     for (s >>= 1; s >= 1; s >>= 1) {
         __syncthreads();
         const int kk = s * (2 * k + 1) - 1;
@@ -165,7 +176,7 @@ struct OffDiag<true> {
 
 // RHS_IS_X: the right-hand side is x itself (implicit solve only, no explicit
 // half); xl / xr are then unused.
-template <int M, bool IMAG, class Coef, bool RHS_IS_X = false, bool REDUCED_CR = true>
+template <int M, bool IMAG, class Coef, bool RHS_IS_X = false>
 __device__ __forceinline__ void cn_partition(double2 (&x)[M], const int k, const int P,
                                              const double2 xl, const double2 xr, const double2 w,
                                              Coef coef, double2* __restrict__ lds, const bool sync_first) {
@@ -246,8 +257,7 @@ __device__ __forceinline__ void cn_partition(double2 (&x)[M], const int k, const
         D = cmul(D, ib);
     }
     double2 Lk, Yk;
-    if constexpr (REDUCED_CR) reduced_cr(A, C, D, k, P, lds, Yk, Lk);
-    else reduced_pcr(A, C, D, k, P, lds, Yk, Lk);
+    reduced_cr(A, C, D, k, P, lds, Yk, Lk);
     D = Yk;
     double2 y = D;
 #pragma unroll
@@ -255,18 +265,6 @@ __device__ __forceinline__ void cn_partition(double2 (&x)[M], const int k, const
         if (i < M - 1) y = csub(csub(de[i], cmul(al[i], Lk)), cmul(ga[i], y));
         x[i] = y;
     }
-}
-
-// Real-time form through the Cayley identity
-//     (1 + i H)^-1 (1 - i H) x = 2 (1 + i H)^-1 x - x,
-// which needs no explicit stencil (and no neighbour exchange): solve
-// (1 + i H) z = x in place with cn_partition's elimination (d = x); the
-// caller forms y = 2 z - x, re-reading x from memory (a cache hit) rather than
-// keeping a second copy live in registers.
-template <int M, class Coef>
-__device__ __forceinline__ void cn_cayley_solve(double2 (&x)[M], const int k, const int P, Coef coef,
-                                                double2* __restrict__ lds) {
-    cn_partition<M, true, Coef, true>(x, k, P, cmk(0.0, 0.0), cmk(0.0, 0.0), cmk(0.0, 1.0), coef, lds, false);
 }
 
 // Implicit solve (1 + i H) z = x for real H with a smaller register footprint
@@ -299,7 +297,7 @@ __device__ __forceinline__ void cn_cayley_solve(double2 (&x)[M], const int k, co
 // would otherwise spill):
 //  * pass 1 forms the pivots from the chunk's leading principal minors (no
 //    division in the recurrence) and stores alpha_i, i < m - 2, in LDS after
-//    the reduced system's 3 P LANES entries, at (3 P + i P + k) LANES + ln
+//    the reduced system's entries, at 3 P LANES + kRedScratch + (i P + k) LANES + ln
 //    (M - 2 more P LANES double2; alpha_{m-2} stays in its register);
 //  * the row-0 coefficients through (L_k, Y_k) come from a backward sweep over
 //    the stored alpha_i instead of the running forward sums;
@@ -315,7 +313,7 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
                                                    const double2 xl = make_double2(0.0, 0.0),
                                                    const double2 xr = make_double2(0.0, 0.0), const int ln = 0,
                                                    Ratio ratio = Ratio{}, const int ib = -1) {
-    double2* __restrict__ alds = lds + (3 * P + k) * LANES + ln;  // alpha_i at alds[i P LANES]
+    double2* __restrict__ alds = lds + (3 * P + k) * LANES + kRedScratch + ln;  // alpha_i at alds[i P LANES]
     double2 ga[M - 1], de[M - 1];
     double2 al = cmk(0.0, 0.0), pi = cmk(1.0, 0.0), sa = cmk(0.0, 0.0), sd = cmk(0.0, 0.0);
     double2 gprev = cmk(0.0, 0.0), dprev = cmk(0.0, 0.0);

@@ -453,7 +453,7 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
             for (int i = 0; i < M; ++i) st2s(gl, (size_t)i * st, x[i]);
         }
     } else {
-        double2* keep = lds + 3 * P * LANES;  // CN_CAYLEY_LDS: this thread's own rows only
+        double2* keep = lds + 3 * P * LANES + kRedScratch;  // CN_CAYLEY_LDS: this thread's own rows only
         if constexpr (FORM == CN_CAYLEY_LDS) {
 #pragma unroll
             for (int i = 0; i < M; ++i) keep[(i * P + k) * LANES + ln] = x[i];
@@ -488,7 +488,7 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 template <int M, int MAXT, int WPE, int FORM>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, ShObs obs) {
-    extern __shared__ double2 lds[];  // 3 * P, then M * P for CN_CAYLEY_LDS
+    extern __shared__ double2 lds[];  // 3 * P + kRedScratch, then M * P for CN_CAYLEY_LDS
     if ((int)blockIdx.x < obs.blocks) {
         sh_observe_block(obs);
         return;
@@ -784,7 +784,7 @@ template <int M, int MAXT, int WPE>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs,
                   const double* __restrict__ cl) {
-    extern __shared__ double2 lds[];  // (3 + M - 2) * P * 2: the solver's rows and alpha_i of both lines, interleaved
+    extern __shared__ double2 lds[];  // (3 + M - 2) * P * 2 + kRedScratch: the solver's rows and alpha_i of both lines, interleaved
     const int job = xcd_remap(blockIdx.x, gridDim.x);
     if (job >= n_pairs) return;
     const int2 pt = pairs[job];
@@ -876,7 +876,7 @@ template <int M, int MAXT, int WPE, bool EXPL>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const int* __restrict__ ctl,
            ShObs obs) {
-    extern __shared__ double2 lds[];  // 3 * P
+    extern __shared__ double2 lds[];  // 3 * P + kRedScratch
     if ((int)blockIdx.x < obs.blocks) {
         sh_observe_block(obs);
         return;
@@ -1046,7 +1046,7 @@ template <int M>
 __global__ void __launch_bounds__(kAdiLanes * kAdiChunks) k_sh_adi_lp(ShSim* __restrict__ sims,
                                                                       const int2* __restrict__ groups, int n_groups,
                                                                       const double* __restrict__ cl) {
-    extern __shared__ double2 lds[];  // 3 * kAdiChunks * kAdiLanes
+    extern __shared__ double2 lds[];  // 3 * kAdiChunks * kAdiLanes + kRedScratch
     constexpr int LANES = kAdiLanes;
     const int job = xcd_remap(blockIdx.x, gridDim.x);
     if (job >= n_groups) return;
