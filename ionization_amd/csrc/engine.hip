@@ -217,6 +217,12 @@ struct tdse_ctx {
     std::vector<Bucket> sh_adi_lbuckets;  // ADI position groups (slot, group) of the partition l-sweep, by rows
     hipStream_t side[3] = {nullptr, nullptr, nullptr};
     hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
+    // every layout in one launch for each sweep (any_layouts): the buckets' lines, longest first
+    bool any_sh = false, any_adi = false;
+    DevVec<int2> any_lines, any_pairs, any_adi_lines, any_adi_groups;
+    int any_threads = 0, any_pair_threads = 0, any_adi_threads = 0;
+    size_t any_lds = 0, any_adi_lds = 0;
+    bool any_has_pairs = false;  // some entries of any_lines are velocity odd l-pairs
     std::vector<Bucket> line_buckets;
     bool dirty = true;
     bool sh_norm_by_l = false;   // some live SH simulation reduces the norm in every l (L-phase instance)
@@ -279,6 +285,75 @@ void drop_graph(tdse_ctx* ctx) {
 }
 
 size_t line_lds_bytes(int M, int P, bool real_steps);
+size_t cn_lds_bytes(int M, int P, int form);
+int cn_form(int M, int P);
+size_t vpair_lds_bytes(int M, int P);
+size_t adi_lds_bytes(int P);
+
+// Whether the layouts of a set of lines share one launch per sweep: more than one of them, none past kAnyP threads,
+// and a batch small enough that the launches and their forks and joins cost more than the deepest tile's
+// occupancy does. Measured (us per step, one launch / a launch for each layout): 32 length-gauge simulations of 15 M
+// points 228 / 239, the 256 of 111 M 1689 / 1579; velocity gauge 4.7 M 194 / 275, 111 M 4334 / 3500; ADI 4.2 M
+// 104 / 143, 111 M 2441 / 2024. Between them the gain falls linearly with the points: the lines below are near zero.
+using Layouts = std::map<std::pair<int, int>, std::vector<int2>>;  // (rows, chunks) -> lines
+constexpr int64_t kAnyPoints = int64_t(24) << 20;       // single lines only
+constexpr int64_t kAnyPointsMore = int64_t(12) << 20;   // with velocity-gauge pairs, or ADI's three sweeps
+bool any_layouts(const Layouts& lines, const Layouts& pairs, int64_t limit) {
+    int64_t points = 0;
+    for (const Layouts* m : {&lines, &pairs})
+        for (auto& kv : *m) {
+            if (kv.first.second > kAnyP) return false;
+            points += (int64_t)kv.second.size() * kv.first.first * kv.first.second;
+        }
+    return lines.size() + pairs.size() > 1 && points <= limit;
+}
+
+// The single-launch tables of the split-operator and ADI simulations (longest lines first).
+int build_any(tdse_ctx* ctx, const Layouts& lines, const Layouts (&vpairs)[2], const Layouts& fpairs,
+              const Layouts& adi, const Layouts& adi_groups) {
+    std::vector<int2> solve, pairs, al, ag;
+    int rc;
+    // pairs count half their points (one entry for two rows)
+    ctx->any_sh = any_layouts(lines, fpairs, fpairs.empty() ? kAnyPoints : kAnyPointsMore / 2);
+    ctx->any_adi = any_layouts(adi, adi_groups, kAnyPointsMore) && ctx->adi_waves.count == 0;
+    ctx->any_threads = ctx->any_pair_threads = ctx->any_adi_threads = 0;
+    ctx->any_lds = ctx->any_adi_lds = 0;
+    ctx->any_has_pairs = false;
+    if (ctx->any_sh) {
+        for (auto it = fpairs.rbegin(); it != fpairs.rend(); ++it) {
+            const int M = it->first.first, P = it->first.second;
+            for (const int2& e : it->second) solve.push_back(make_int2(e.x, e.y | kAnyPair));
+            ctx->any_has_pairs = true;
+            ctx->any_threads = std::max(ctx->any_threads, 2 * P);
+            ctx->any_lds = std::max(ctx->any_lds, vpair_lds_bytes(M, P));
+        }
+        for (auto it = lines.rbegin(); it != lines.rend(); ++it) {
+            const int M = it->first.first, P = it->first.second;
+            solve.insert(solve.end(), it->second.begin(), it->second.end());
+            ctx->any_threads = std::max(ctx->any_threads, P);
+            ctx->any_lds = std::max(ctx->any_lds, cn_lds_bytes(M, P, cn_form(M, P)));
+        }
+        // up to kAnyP threads the odd l-pairs are solved with the lines: only the even ones are left
+        for (auto it = vpairs[0].rbegin(); it != vpairs[0].rend(); ++it) {
+            pairs.insert(pairs.end(), it->second.begin(), it->second.end());
+            ctx->any_pair_threads = std::max(ctx->any_pair_threads, sh_vel_split(it->first.first) * it->first.second);
+        }
+    }
+    if (ctx->any_adi) {
+        for (auto it = adi.rbegin(); it != adi.rend(); ++it) {
+            al.insert(al.end(), it->second.begin(), it->second.end());
+            ctx->any_adi_threads = std::max(ctx->any_adi_threads, it->first.second);
+            ctx->any_adi_lds = std::max(ctx->any_adi_lds, adi_lds_bytes(it->first.second));
+        }
+        for (auto it = adi_groups.rbegin(); it != adi_groups.rend(); ++it)
+            ag.insert(ag.end(), it->second.begin(), it->second.end());
+    }
+    if ((rc = devvec_upload(ctx, ctx->any_lines, solve)) || (rc = devvec_upload(ctx, ctx->any_pairs, pairs)) ||
+        (rc = devvec_upload(ctx, ctx->any_adi_lines, al)) || (rc = devvec_upload(ctx, ctx->any_adi_groups, ag)))
+        return rc;
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // the host vectors end here
+    return TDSE_OK;
+}
 
 // Rebuild the ragged work tables from the live simulations.
 int rebuild_tables(tdse_ctx* ctx) {
@@ -322,9 +397,9 @@ int rebuild_tables(tdse_ctx* ctx) {
         if (h.adi) {
             for (int l = 0; l < h.dev.L; ++l) adb[{h.dev.m, h.dev.P}].push_back(make_int2(s, l));
             // l-direction: the partition solver where kAdiChunks chunks of at most 16 rows cover l_bound
-            const int ml = 2 * ((h.dev.L + 2 * kAdiChunks - 1) / (2 * kAdiChunks));
+            const int ml = sh_adi_lp_rows(h.dev.L);
             if (ml <= 16) {
-                for (int gq = 0; gq < h.dev.npad / kAdiLanes; ++gq) alb[{std::max(ml, 2), 0}].push_back(make_int2(s, gq));
+                for (int gq = 0; gq < h.dev.npad / kAdiLanes; ++gq) alb[{ml, 0}].push_back(make_int2(s, gq));
             } else {
                 for (int w = 0; w < wpl; ++w) adw.push_back(make_int2(s, w * TDSE_WAVE));
             }
@@ -403,6 +478,7 @@ int rebuild_tables(tdse_ctx* ctx) {
         auto it = fpb.find({b.M, b.P});
         if (it != fpb.end() && (rc = devvec_upload(ctx, b.fpairs, it->second))) return rc;
     }
+    if ((rc = build_any(ctx, shb, vpb, fpb, adb, alb))) return rc;
     if ((rc = fill(ctx->line_buckets, lnb))) return rc;
     for (auto& kv : lna) {
         ctx->line_buckets.emplace_back();
@@ -527,9 +603,11 @@ void dispatch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) 
     }
 }
 
+size_t adi_lds_bytes(int P) { return (3 * (size_t)P + kRedScratch) * sizeof(double2); }
+
 template <int M, int MAXT, int WPE, bool EXPL>
 void launch_adi_r(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
-    const size_t lds = (3 * (size_t)b.P + kRedScratch) * sizeof(double2);
+    const size_t lds = adi_lds_bytes(b.P);
     const ShObs obs = obs_of(ctx, EXPL ? ctx->jobs : ctx->adi_jobs, b.P, ride);
     hipLaunchKernelGGL((k_sh_adi_r<M, MAXT, WPE, EXPL>), dim3((unsigned)(b.lines.count + obs.blocks)), dim3(b.P), lds,
                        st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, ctx->d_ctl, obs);
@@ -570,10 +648,12 @@ void dispatch_adi_lp(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
     }
 }
 
+size_t vpair_lds_bytes(int M, int P) { return ((size_t)(3 + M - 2) * P * 2 + kRedScratch) * sizeof(double2); }
+
 template <int M, int WPE>
 void launch_rphase_vpair(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
     // the reduced system (3 P) and alpha_i of rows 0 .. M - 3 (M - 2 P) per line, two lines
-    const size_t lds = ((size_t)(3 + M - 2) * b.P * 2 + kRedScratch) * sizeof(double2);
+    const size_t lds = vpair_lds_bytes(M, b.P);
     hipLaunchKernelGGL((k_sh_rphase_vpair<M, kMaxPairThreads, WPE>), dim3((unsigned)b.fpairs.count), dim3(2 * b.P),
                        lds, st, ctx->d_sh, b.fpairs.ptr, (int)b.fpairs.count, ctx->d_cl);
 }
@@ -597,7 +677,7 @@ void dispatch_rphase_vpair(tdse_ctx* ctx, const Bucket& b, hipStream_t st) {
 template <bool REV>
 void dispatch_vphase(tdse_ctx* ctx, const Bucket& b, int par, hipStream_t st) {
     const DevVec<int2>& pairs = b.vpairs[par];
-    const bool split = (b.M == 8 || b.M == 12 || b.M == 16) && 2 * b.P <= 512;
+    const bool split = sh_vel_split(b.M) == 2 && 2 * b.P <= 512;
     const dim3 grid((unsigned)pairs.count), block((unsigned)(split ? 2 * b.P : b.P));
     auto args = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, block, 0, st, ctx->d_sh, pairs.ptr, (int)pairs.count, ctx->d_cl);
@@ -790,7 +870,24 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
                     prof_end(ctx);
                 }
         };
-        if (ctx->profiling || ctx->sh_buckets.size() < 2) {
+        if (ctx->any_sh && !ctx->profiling) {
+            observe(ctx->stream);
+            auto vphase = [&](auto kernel) {
+                if (!ctx->any_pairs.count) return;
+                hipLaunchKernelGGL(kernel, dim3((unsigned)ctx->any_pairs.count), dim3(ctx->any_pair_threads), 0,
+                                   ctx->stream, ctx->d_sh, ctx->any_pairs.ptr, (int)ctx->any_pairs.count, ctx->d_cl);
+            };
+            const ShObs obs = obs_of(ctx, ctx->jobs, ctx->any_threads, ride);
+            auto solve = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(ctx->any_lines.count + obs.blocks)), dim3(ctx->any_threads),
+                                   ctx->any_lds, ctx->stream, ctx->d_sh, ctx->any_lines.ptr,
+                                   (int)ctx->any_lines.count, ctx->d_cl, obs);
+            };
+            vphase(k_sh_vphase_any<false>);
+            if (ctx->any_has_pairs) solve(k_sh_solve_any<true>);
+            else solve(k_sh_solve_any<false>);
+            vphase(k_sh_vphase_any<true>);
+        } else if (ctx->profiling || ctx->sh_buckets.size() < 2) {
             observe(ctx->stream);
             for (auto& b : ctx->sh_buckets) chain(b, ctx->stream);
         } else {
@@ -814,7 +911,20 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
         // Within each of the three sweeps the buckets are independent: they run concurrently
         // over the context stream and the side streams (fork and join by events), and each
         // sweep starts after the whole previous one.
-        if (!ctx->sh_adi_buckets.empty()) {
+        if (ctx->any_adi && !ctx->profiling) {
+            const int nl = (int)ctx->any_adi_lines.count, ng = (int)ctx->any_adi_groups.count;
+            const dim3 threads(ctx->any_adi_threads);
+            const ShObs obs = obs_of(ctx, ctx->jobs, ctx->any_adi_threads, ride && !rider);
+            const ShObs counts = obs_of(ctx, ctx->adi_jobs, ctx->any_adi_threads, true);
+            hipLaunchKernelGGL(k_sh_adi_r_any<true>, dim3(nl + obs.blocks), threads,
+                               ctx->any_adi_lds, ctx->stream,
+                               ctx->d_sh, ctx->any_adi_lines.ptr, nl, ctx->d_ctl, obs);
+            hipLaunchKernelGGL(k_sh_adi_lp_any, dim3(ng), dim3(kAdiChunks * kAdiLanes),
+                               (3 * (size_t)kAdiChunks * kAdiLanes + kRedScratch) * sizeof(double2), ctx->stream,
+                               ctx->d_sh, ctx->any_adi_groups.ptr, ng, ctx->d_cl);
+            hipLaunchKernelGGL(k_sh_adi_r_any<false>, dim3(nl + counts.blocks), threads, ctx->any_adi_lds, ctx->stream,
+                               ctx->d_sh, ctx->any_adi_lines.ptr, nl, ctx->d_ctl, counts);
+        } else if (!ctx->sh_adi_buckets.empty()) {
             int rc;
             const Bucket* first = rider ? nullptr : &ctx->sh_adi_buckets[0];
             if ((rc = fan_out(ctx, ctx->sh_adi_buckets, [&](const Bucket& b, hipStream_t st) {
@@ -1044,7 +1154,8 @@ int tdse_ctx_destroy(tdse_ctx* ctx) {
     if (ctx->adi_waves.ptr) (void)hipFree(ctx->adi_waves.ptr);
     if (ctx->cyl_jobs.ptr) (void)hipFree(ctx->cyl_jobs.ptr);
     if (ctx->cyl_count_jobs.ptr) (void)hipFree(ctx->cyl_count_jobs.ptr);
-    if (ctx->adi_jobs.ptr) (void)hipFree(ctx->adi_jobs.ptr);
+    for (auto* v : {&ctx->adi_jobs, &ctx->any_lines, &ctx->any_pairs, &ctx->any_adi_lines, &ctx->any_adi_groups})
+        if (v->ptr) (void)hipFree(v->ptr);
     if (ctx->d_cyl) (void)hipFree(ctx->d_cyl);
     if (ctx->waves.ptr) (void)hipFree(ctx->waves.ptr);
     if (ctx->jobs.ptr) (void)hipFree(ctx->jobs.ptr);
@@ -1291,6 +1402,7 @@ int tdse_sh_add(tdse_ctx* ctx, const tdse_sh_desc* desc, const double* tables, c
     S.out_nl = onl;
     S.fa = dfa;
     S.adi = H.adi ? 1 : 0;
+    S.vel = H.vel ? 1 : 0;
     HIP_TRY(ctx, hipMemcpyAsync(ctx->d_sh + s, &S, sizeof(ShSim), hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // host buffers may be released after return
     H.live = true;

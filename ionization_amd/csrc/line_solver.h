@@ -39,18 +39,22 @@ __device__ __forceinline__ double2 wmul(double2 w, double2 v) {
 // The reduced system  a_k Y_{k-1} + Y_k + c_k Y_{k+1} = d_k,  k < P  (one equation
 // per thread, unit diagonal, a_0 = c_{P-1} = 0): returns Y_k and Y_{k-1}.
 //
-// Cyclic reduction with compacted threads down to what one wave holds, parallel
-// cyclic reduction there, and the back substitution. At stride s the surviving
-// equations kk = 2 s (t + 1) - 1 are updated by threads t = 0, 1, ... (so whole waves
-// drop out as the system shrinks), eliminating kk - s and kk + s. Once the survivors
-// of the block's lines fit 64 lanes, the first wave finishes them without barriers:
-// log2 levels in which every lane updates its own equation, where cyclic reduction
-// would take as many levels up and again down at the same issue cost (a wave's
-// instruction costs the same with one lane active), each behind a block barrier. The
-// eliminated equations s (2 t + 1) - 1 then follow from their solved neighbours.
-// Against cyclic reduction throughout, us per step: one 8192-point line (P = 512) 12.2 ->
-// 10.5, 250 x 100 SH (P = 64) 17.2 -> 16.1, 250 x 100 cylinder 20.2 -> 18.4; R-phase of
-// the 256-simulation scan 0.98 -> 0.92 ms (serial).
+// Cyclic reduction with compacted threads down to what one wave holds. At stride s the
+// surviving equations kk = 2 s (t + 1) - 1 are updated by threads t = 0, 1, ... (so
+// whole waves drop out as the system shrinks), eliminating kk - s and kk + s. Once
+// the survivors of the block's lines fit 64 lanes, the first wave finishes them without
+// block barriers; the eliminated equations s (2 t + 1) - 1 then follow from their solved
+// neighbours. The wave's own part takes one of two forms:
+//  * pcr: parallel cyclic reduction, log2 levels in which every lane updates its own
+//    equation, where cyclic reduction takes as many levels up and again down at the same
+//    issue cost (a wave's instruction costs the same with one lane active);
+//  * otherwise cyclic reduction, the same products as the block-wide levels form. The
+//    velocity gauge and the l-sweep of ADI add and subtract rows of very different size,
+//    so their smallest rows carry the rounding of their largest: there the bits of a solve
+//    show in stored values (the norm in the largest l) that a change in rounding would move.
+// Against cyclic reduction behind block barriers throughout, us per step: one 8192-point
+// line (P = 512) 12.2 -> 10.5, 250 x 100 SH (P = 64) 17.2 -> 16.1, 250 x 100 cylinder
+// 20.2 -> 18.4 (pcr); R-phase of the 256-simulation scan 0.98 -> 0.92 ms (serial).
 //
 // LANES > 1: LANES independent lines share the block, thread k LANES + ln on equation
 // k of line ln, which sits at LDS index k * LANES + ln (each array of 3 holds P * LANES
@@ -62,7 +66,7 @@ constexpr int kRedScratch = 3 * TDSE_WAVE;
 template <int LANES = 1>
 __device__ __forceinline__ void reduced_cr(double2 A, double2 C, double2 D, const int k, const int P,
                                            double2* __restrict__ lds, double2& Yk, double2& Ykm1,
-                                           const int ln = 0) {
+                                           const int ln = 0, const bool pcr = true) {
     double2* pa = lds + ln;
     double2* pc = lds + P * LANES + ln;
     double2* pd = lds + 2 * P * LANES + ln;
@@ -114,13 +118,18 @@ __device__ __forceinline__ void reduced_cr(double2 A, double2 C, double2 D, cons
             c0 = pc[e];
             d0 = pd[e];
         }
-        for (int q = 1; q < left; q <<= 1) {
+        // one wave: its LDS operations complete in order, only the compiler has to keep it
+        auto ordered = []() {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        auto publish = [&]() {
             w[0] = a0;
             w[TDSE_WAVE] = c0;
             w[2 * TDSE_WAVE] = d0;
-            // one wave: its LDS operations complete in order, only the compiler has to keep it
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+        };
+        // this equation without the ones q before and after it
+        auto update = [&](int q) {
             double2 am = zero, cm = zero, dm = zero, apl = zero, cpl = zero, dpl = zero;
             if (k >= q) {
                 am = w[-q * LANES];
@@ -134,6 +143,32 @@ __device__ __forceinline__ void reduced_cr(double2 A, double2 C, double2 D, cons
             }
             __builtin_amdgcn_wave_barrier();
             eliminate(a0, c0, d0, am, cm, dm, apl, cpl, dpl);
+        };
+        if (pcr) {
+            for (int q = 1; q < left; q <<= 1) {
+                publish();
+                ordered();
+                update(q);
+            }
+        } else {
+            publish();
+            int q = 1;
+            for (; q < left; q <<= 1) {
+                ordered();
+                if (on && ((k + 1) & (2 * q - 1)) == 0) {
+                    update(q);
+                    publish();
+                }
+            }
+            for (q >>= 1; q >= 1; q >>= 1) {
+                ordered();
+                if (on && ((k + 1) & (2 * q - 1)) == q) {
+                    const double2 ym = (k >= q) ? w[2 * TDSE_WAVE - q * LANES] : zero;
+                    const double2 yp = (k + q < left) ? w[2 * TDSE_WAVE + q * LANES] : zero;
+                    d0 = csub(csub(d0, cmul(a0, ym)), cmul(c0, yp));
+                    w[2 * TDSE_WAVE] = d0;
+                }
+            }
         }
         if (on) pd[e] = d0;  // no neighbours left: its d is its solution
     }
@@ -285,7 +320,7 @@ __device__ __forceinline__ void cn_partition(double2 (&x)[M], const int k, const
 // EXPLICIT: the right-hand side is the explicit half (1 - i H~) x, formed
 // row by row in pass 1 from x and the chunk neighbours xl = x_{km-1},
 // xr = x_{km+m} (chunk_neighbours); otherwise it is x itself.
-// LANES / ln: several interleaved lines per block, as for reduced_cr.
+// LANES / ln: several interleaved lines per block, as for reduced_cr; pcr: its form.
 //
 // Ratio: when given (not NoRatio), pass 2 takes the sub-diagonal pivot factor
 // rsub_i = i hm_i / den_i from the stored super-diagonal one, g_i = i hp_i / den_i,
@@ -312,7 +347,7 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
                                                    Coef2 coef2, double2* __restrict__ lds,
                                                    const double2 xl = make_double2(0.0, 0.0),
                                                    const double2 xr = make_double2(0.0, 0.0), const int ln = 0,
-                                                   Ratio ratio = Ratio{}, const int ib = -1) {
+                                                   Ratio ratio = Ratio{}, const int ib = -1, const bool pcr = true) {
     double2* __restrict__ alds = lds + (3 * P + k) * LANES + kRedScratch + ln;  // alpha_i at alds[i P LANES]
     double2 ga[M - 1], de[M - 1];
     double2 al = cmk(0.0, 0.0), pi = cmk(1.0, 0.0), sa = cmk(0.0, 0.0), sd = cmk(0.0, 0.0);
@@ -420,7 +455,7 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
         D = cmul(D, ib);
     }
     double2 Lk, Yk;
-    reduced_cr<LANES>(A, C, D, k, P, lds, Yk, Lk, ln);
+    reduced_cr<LANES>(A, C, D, k, P, lds, Yk, Lk, ln, pcr);
     if constexpr (ALPHA_LDS) {
         // passes 2 and 3 in one: z_i = delta_i - alpha_i L_k - gamma_i z_{i+1}
         double2 z = Yk;

@@ -52,6 +52,7 @@ struct ShSim {
     int active;
     int phase;             // 0: g is mid-step (after the R-phase); 1: g is the reference g after `step` steps
     int norm_by_l;         // 1: also reduce the norm of every l at data times
+    int vel;               // 1: velocity gauge (its line solves keep cyclic reduction, reduced_cr)
     int adi;               // 1: AlternatingDirectionImplicit (fs is then zero: the L-phase only masks and observes)
     const double* fa;      // ADI: [N] field times tau ratio per step, E(t_{n+1} + dt/2) tau_n / tau0
     int flags;             // health flags (norm_health), device-updated at data times
@@ -442,12 +443,13 @@ template <int M, int FORM, class Coef, class Coef2, class Ratio = NoRatio, int L
 __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restrict__ gl, const int k, const int P,
                                                Coef coef, Coef2 coef2, double2* __restrict__ lds,
                                                Ratio ratio = Ratio{}, const int ib = -1, const int ln = 0,
-                                               const int stride = -1, const bool store = true) {
+                                               const int stride = -1, const bool store = true,
+                                               const bool pcr = true) {
     const size_t st = stride < 0 ? (size_t)P : (size_t)stride;
     if constexpr (FORM == CN_EXPLICIT) {
         double2 xl, xr;
         chunk_neighbours<M, LANES>(x, k, P, lds, xl, xr, false, ln);
-        cn_implicit_lowreg<M, Coef, Coef2, true, LANES, Ratio>(x, k, P, coef, coef2, lds, xl, xr, ln, ratio, ib);
+        cn_implicit_lowreg<M, Coef, Coef2, true, LANES, Ratio>(x, k, P, coef, coef2, lds, xl, xr, ln, ratio, ib, pcr);
         if (store) {
 #pragma unroll
             for (int i = 0; i < M; ++i) st2s(gl, (size_t)i * st, x[i]);
@@ -459,7 +461,7 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
             for (int i = 0; i < M; ++i) keep[(i * P + k) * LANES + ln] = x[i];
         }
         cn_implicit_lowreg<M, Coef, Coef2, false, LANES, Ratio>(x, k, P, coef, coef2, lds, cmk(0.0, 0.0),
-                                                                cmk(0.0, 0.0), ln, ratio, ib);
+                                                                cmk(0.0, 0.0), ln, ratio, ib, pcr);
         if (!store) return;
 #pragma unroll
         for (int i = 0; i < M; ++i) {
@@ -485,22 +487,9 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 //    double2 of LDS; each thread reads back only what it wrote) or re-read
 //    from memory at the end (CN_CAYLEY_MEM).
 
-template <int M, int MAXT, int WPE, int FORM>
-__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
-k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, ShObs obs) {
-    extern __shared__ double2 lds[];  // 3 * P + kRedScratch, then M * P for CN_CAYLEY_LDS
-    if ((int)blockIdx.x < obs.blocks) {
-        sh_observe_block(obs);
-        return;
-    }
-    // consecutive l-lines of a simulation (which share its coefficient rows) on one XCD
-    const int line = xcd_remap(blockIdx.x - obs.blocks, gridDim.x - obs.blocks);
-    if (line >= n_lines) return;
-    const int2 lt = lines[line];
-    ShSim& S = sims[lt.x];
-    const int n = S.rstep;
-    if (!S.active || n >= S.N) return;  // uniform across the block
-    const int l = lt.y;
+// lds: 3 * P + kRedScratch double2, then M * P for CN_CAYLEY_LDS. n: the step under way.
+template <int M, int FORM>
+__device__ __forceinline__ void sh_rphase_line(const ShSim& S, const int n, const int l, double2* __restrict__ lds) {
     const int P = S.P, npad = S.npad;
     const int k = threadIdx.x;
     const double sn = ld1(S.ts, n);
@@ -555,7 +544,25 @@ k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_line
         hm = sn * carry2;
         carry2 = tv.y;
     };
-    cn_line_finish<M, FORM>(x, gl, k, P, coef, coef2, lds, NoRatio{}, -1, 0, -1, !pad);
+    cn_line_finish<M, FORM>(x, gl, k, P, coef, coef2, lds, NoRatio{}, -1, 0, -1, !pad, !S.vel);
+}
+
+template <int M, int MAXT, int WPE, int FORM>
+__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
+k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, ShObs obs) {
+    extern __shared__ double2 lds[];
+    if ((int)blockIdx.x < obs.blocks) {
+        sh_observe_block(obs);
+        return;
+    }
+    // consecutive l-lines of a simulation (which share its coefficient rows) on one XCD
+    const int line = xcd_remap(blockIdx.x - obs.blocks, gridDim.x - obs.blocks);
+    if (line >= n_lines) return;
+    const int2 lt = lines[line];
+    const ShSim& S = sims[lt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;  // uniform across the block
+    sh_rphase_line<M, FORM>(S, n, lt.y, lds);
 }
 
 // ------------------------------------------------------------------ velocity gauge: h2
@@ -646,19 +653,11 @@ __device__ __forceinline__ void sh_vel_rpairs(double2 (&s)[M / SPLIT], double2 (
 // l-pairs) before the solve and (odd, even) after it. SPLIT threads per chunk
 // (SPLIT P per workgroup), each with M / SPLIT rows: fewer registers, more waves.
 template <int M, bool REV, int SPLIT>
-__global__ void __launch_bounds__(512) k_sh_vphase(ShSim* __restrict__ sims, const int2* __restrict__ pairs,
-                                                   int n_pairs, const double* __restrict__ cl) {
+__device__ __forceinline__ void sh_vphase_pair(const ShSim& S, const int n, const int l, const double* __restrict__ cl,
+                                               double2 (*ex)[512]) {
     constexpr int MH = M / SPLIT;
-    __shared__ double2 ex[4][512];
-    const int pair = xcd_remap(blockIdx.x, gridDim.x);
-    if (pair >= n_pairs) return;
-    const int2 pt = pairs[pair];
-    ShSim& S = sims[pt.x];
-    const int n = S.rstep;
-    if (!S.active || n >= S.N) return;  // uniform across the block
     const double fn = ld1(S.fs, n);
     if (fn == 0.0) return;  // every angle is zero: the factor is the identity
-    const int l = pt.y;
     const int P = S.P, npad = S.npad;
     const int c = threadIdx.x;
     const double f = fn * ld1(cl, l);
@@ -691,6 +690,19 @@ __global__ void __launch_bounds__(512) k_sh_vphase(ShSim* __restrict__ sims, con
         st2s(g0, q, cmk((s[i].x + d[i].x) * kRsqrt2, (s[i].y + d[i].y) * kRsqrt2));
         st2s(g1, q, cmk((s[i].x - d[i].x) * kRsqrt2, (s[i].y - d[i].y) * kRsqrt2));
     }
+}
+
+template <int M, bool REV, int SPLIT>
+__global__ void __launch_bounds__(512) k_sh_vphase(ShSim* __restrict__ sims, const int2* __restrict__ pairs,
+                                                   int n_pairs, const double* __restrict__ cl) {
+    __shared__ double2 ex[4][512];
+    const int pair = xcd_remap(blockIdx.x, gridDim.x);
+    if (pair >= n_pairs) return;
+    const int2 pt = pairs[pair];
+    const ShSim& S = sims[pt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;  // uniform across the block
+    sh_vphase_pair<M, REV, SPLIT>(S, n, pt.y, cl, ex);
 }
 
 // Velocity gauge: the R-phase of one odd l-pair (l, l + 1) together with the
@@ -780,20 +792,14 @@ __device__ __forceinline__ void sh_vpair_factors(double2 (&x)[M], const int k, c
     hadamard();
 }
 
-template <int M, int MAXT, int WPE>
-__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
-k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs,
-                  const double* __restrict__ cl) {
-    extern __shared__ double2 lds[];  // (3 + M - 2) * P * 2 + kRedScratch: the solver's rows and alpha_i of both lines, interleaved
-    const int job = xcd_remap(blockIdx.x, gridDim.x);
-    if (job >= n_pairs) return;
-    const int2 pt = pairs[job];
-    ShSim& S = sims[pt.x];
-    const int n = S.rstep;
-    if (!S.active || n >= S.N) return;  // uniform across the block
+// lds: (3 + M - 2) * P * 2 + kRedScratch double2: the solver's rows and alpha_i of both lines, interleaved.
+// l0: the pair's first row; 2 P threads.
+template <int M>
+__device__ __forceinline__ void sh_vpair_lines(const ShSim& S, const int n, const int l0, const double* __restrict__ cl,
+                                               double2* __restrict__ lds) {
     const int P = S.P, npad = S.npad;
     const int ln = threadIdx.x & 1, k = threadIdx.x >> 1;
-    const int l = pt.y + ln;
+    const int l = l0 + ln;
     const double sn = ld1(S.ts, n);
     const double ll1 = (double)l * (double)(l + 1);
     double2* __restrict__ gl = sh_state(S, n + 1) + (size_t)l * npad + k;
@@ -802,7 +808,7 @@ k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int 
     const int nr = S.n;
     const double a_left = (k > 0) ? ld1(S.tab, SH_AN * npad + (M - 1) * P + k - 1) : 0.0;
     const double fh = ld1(S.fs, n);
-    const double fp = fh * ld1(cl, pt.y);  // the pair's angle factor (row l's combination +theta, row l + 1's -theta)
+    const double fp = fh * ld1(cl, l0);  // the pair's angle factor (row l's combination +theta, row l + 1's -theta)
     const double* __restrict__ av = S.tab + (size_t)SH_AV * npad;
 
     const bool pad = k * M >= nr;  // all rows padding: zeros, neither read nor written (as in the R-phase)
@@ -844,11 +850,26 @@ k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int 
     };
     double2 xl, xr;
     chunk_neighbours<M, 2>(x, k, P, lds, xl, xr, true, ln);
-    cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, 2, NoRatio, true>(x, k, P, coef, coef2, lds, xl, xr, ln);
+    cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, 2, NoRatio, true>(x, k, P, coef, coef2, lds, xl, xr, ln,
+                                                                                     NoRatio{}, -1, false);
     if (fh != 0.0) sh_vpair_factors<M>(x, k, P, ln, lds, av, fp, true);
     if (pad) return;
 #pragma unroll
     for (int i = 0; i < M; ++i) st2s(gl, (size_t)i * P, x[i]);
+}
+
+template <int M, int MAXT, int WPE>
+__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
+k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs,
+                  const double* __restrict__ cl) {
+    extern __shared__ double2 lds[];
+    const int job = xcd_remap(blockIdx.x, gridDim.x);
+    if (job >= n_pairs) return;
+    const int2 pt = pairs[job];
+    const ShSim& S = sims[pt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;  // uniform across the block
+    sh_vpair_lines<M>(S, n, pt.y, cl, lds);
 }
 
 // ------------------------------------------------------------------ AlternatingDirectionImplicit
@@ -872,23 +893,11 @@ k_sh_rphase_vpair(ShSim* __restrict__ sims, const int2* __restrict__ pairs, int 
 // and the explicit half of step n + 1, written to the state buffer of step n + 2; the
 // next replay skips its L-phase and explicit sweep for the simulation (S.ahead). The
 // products are the ones those two sweeps would form.
-template <int M, int MAXT, int WPE, bool EXPL>
-__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
-k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const int* __restrict__ ctl,
-           ShObs obs) {
-    extern __shared__ double2 lds[];  // 3 * P + kRedScratch
-    if ((int)blockIdx.x < obs.blocks) {
-        sh_observe_block(obs);
-        return;
-    }
-    const int line = xcd_remap(blockIdx.x - obs.blocks, gridDim.x - obs.blocks);
-    if (line >= n_lines) return;
-    const int2 lt = lines[line];
-    ShSim& S = sims[lt.x];
-    const int n = S.rstep;
-    if (!S.active || n >= S.N) return;  // uniform across the block
-    if (EXPL && S.ahead) return;         // applied by the previous replay's implicit sweep
-    const int l = lt.y;
+// lds: 3 * P + kRedScratch double2.
+template <int M, bool EXPL>
+__device__ __forceinline__ void sh_adi_r_line(const ShSim& S, const int n, const int l, const int* __restrict__ ctl,
+                                              double2* __restrict__ lds) {
+    if (EXPL && S.ahead) return;  // applied by the previous replay's implicit sweep
     const int P = S.P, npad = S.npad;
     const int k = threadIdx.x;
     const double sn = ld1(S.ts, n);
@@ -902,13 +911,9 @@ k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines
 
     const bool pad = k * M >= nr;  // all rows padding: zeros, neither read nor written (as in the R-phase)
     double2 x[M];
-    if (pad) {
+    // row by row: with one branch around all the loads the m = 16 instance spills 28 VGPRs at 2 waves per SIMD
 #pragma unroll
-        for (int i = 0; i < M; ++i) x[i] = cmk(0.0, 0.0);
-    } else {
-#pragma unroll
-        for (int i = 0; i < M; ++i) x[i] = ld2s(gl, (size_t)i * P);
-    }
+    for (int i = 0; i < M; ++i) x[i] = pad ? cmk(0.0, 0.0) : ld2s(gl, (size_t)i * P);
     // s (T_j + l(l+1) U_j [+ corr0]): the diagonal of s H in tau0 units (thread kk, grid step rd, factor cc)
     auto diag = [&](int i, double T, double s, int kk, double rd, double cc) {
         const int j = kk * M + i;
@@ -960,7 +965,8 @@ k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines
             hm = sn * carry2;
             carry2 = tv.y;
         };
-        cn_implicit_lowreg<M, decltype(coef), decltype(coef2), false, 1>(x, k, P, coef, coef2, lds);
+        cn_implicit_lowreg<M, decltype(coef), decltype(coef2), false, 1>(x, k, P, coef, coef2, lds, cmk(0.0, 0.0),
+                                                                         cmk(0.0, 0.0), 0, NoRatio{}, -1, false);
         if (sh_adi_ahead(S, n, *ctl)) {  // uniform across the block
             const double* mk = S.tab + (size_t)SH_MASK * npad + k;
             asm volatile("" : "+v"(mk));  // loaded after the solve, not hoisted into it
@@ -977,6 +983,24 @@ k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines
     if (pad) return;
 #pragma unroll
     for (int i = 0; i < M; ++i) st2s(gl, (size_t)i * P, x[i]);
+}
+
+template <int M, int MAXT, int WPE, bool EXPL>
+__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
+k_sh_adi_r(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const int* __restrict__ ctl,
+           ShObs obs) {
+    extern __shared__ double2 lds[];
+    if ((int)blockIdx.x < obs.blocks) {
+        sh_observe_block(obs);
+        return;
+    }
+    const int line = xcd_remap(blockIdx.x - obs.blocks, gridDim.x - obs.blocks);
+    if (line >= n_lines) return;
+    const int2 lt = lines[line];
+    const ShSim& S = sims[lt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;  // uniform across the block
+    sh_adi_r_line<M, EXPL>(S, n, lt.y, ctl, lds);
 }
 
 // The l-direction factor (1 - i A)(1 + i A)^-1 at every position: A real
@@ -1041,23 +1065,18 @@ __global__ void __launch_bounds__(256) k_sh_adi_l(ShSim* __restrict__ sims, cons
 // 128 B runs of each row). The explicit right-hand side (1 - i A) x is formed
 // in the solver's first pass, so every element is read and written once.
 constexpr int kAdiLanes = 8, kAdiChunks = 32;
+// Rows per thread of the partition l-solve (even, at least 2); above 16 the Thomas form runs.
+__host__ __device__ constexpr int sh_adi_lp_rows(int L) { return 2 * ((L + 2 * kAdiChunks - 1) / (2 * kAdiChunks)); }
 
+// lds: 3 * kAdiChunks * kAdiLanes + kRedScratch double2.
 template <int M>
-__global__ void __launch_bounds__(kAdiLanes * kAdiChunks) k_sh_adi_lp(ShSim* __restrict__ sims,
-                                                                      const int2* __restrict__ groups, int n_groups,
-                                                                      const double* __restrict__ cl) {
-    extern __shared__ double2 lds[];  // 3 * kAdiChunks * kAdiLanes + kRedScratch
+__device__ __forceinline__ void sh_adi_lp_group(const ShSim& S, const int n, const int group,
+                                                const double* __restrict__ cl, double2* __restrict__ lds) {
     constexpr int LANES = kAdiLanes;
-    const int job = xcd_remap(blockIdx.x, gridDim.x);
-    if (job >= n_groups) return;
-    const int2 gt = groups[job];
-    ShSim& S = sims[gt.x];
-    const int n = S.rstep;
-    if (!S.active || n >= S.N) return;  // uniform across the block
     const int t = threadIdx.x;
     const int ln = t % LANES, c = t / LANES;
     const int L = S.L, npad = S.npad;
-    const int p = gt.y * LANES + ln;
+    const int p = group * LANES + ln;
     const double f = ld1(S.fa, n) * ld1(S.tab, SH_RQ * npad + p);  // zero at padding positions
     double2* __restrict__ g = sh_state(S, n + 1) + p;
     double2 x[M];
@@ -1081,10 +1100,128 @@ __global__ void __launch_bounds__(kAdiLanes * kAdiChunks) k_sh_adi_lp(ShSim* __r
     double2 xl, xr;
     chunk_neighbours<M, LANES>(x, c, kAdiChunks, lds, xl, xr, false, ln);
     cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, LANES>(x, c, kAdiChunks, coef, coef2, lds, xl, xr,
-                                                                        ln);
+                                                                        ln, NoRatio{}, -1, false);
 #pragma unroll
     for (int i = 0; i < M; ++i) {
         const int l = c * M + i;
         if (l < L) st2s(g, (size_t)l * npad, x[i]);
     }
+}
+
+template <int M>
+__global__ void __launch_bounds__(kAdiLanes * kAdiChunks) k_sh_adi_lp(ShSim* __restrict__ sims,
+                                                                      const int2* __restrict__ groups, int n_groups,
+                                                                      const double* __restrict__ cl) {
+    extern __shared__ double2 lds[];
+    const int job = xcd_remap(blockIdx.x, gridDim.x);
+    if (job >= n_groups) return;
+    const int2 gt = groups[job];
+    const ShSim& S = sims[gt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;  // uniform across the block
+    sh_adi_lp_group<M>(S, n, gt.y, cl, lds);
+}
+
+// ------------------------------------------------------------------ all layouts in one launch
+//
+// A batch of a few small or middling meshes has several layouts (rows and threads per line), and a launch
+// for each, forked over streams and joined again, costs more than their work: 12 velocity-gauge simulations of
+// 4.7 M points took 277 us per step, the 256 of the scan at its rate would take 148. These kernels take
+// lines of every layout (P <= kAnyP) in one launch: the workgroup has the threads of the longest line in the
+// batch, whole waves past a line's threads leave before any barrier (s_barrier waits for the surviving waves
+// only), and the rows per thread are chosen by a branch. They hold the registers of the deepest
+// tile, 2 waves per SIMD, which is why a large batch keeps a launch for each layout (any_layouts, engine.hip).
+// Each line's arithmetic is the layout launch's own. us per step: those 12 velocity-gauge simulations 277 -> 194,
+// 12 ADI ones of 4.2 M points 140 -> 106, three small velocity-gauge meshes 47 -> 31, 32 length-gauge ones of
+// 15 M points 240 -> 228.
+constexpr int kAnyP = 256;
+constexpr int kAnyPair = 1 << 16;  // solve entry (slot, l | kAnyPair): the velocity odd l-pair (l, l + 1)
+
+template <class F>
+__device__ __forceinline__ void sh_by_rows(const int m, F&& f) {
+    switch (m) {
+        case 2: f(std::integral_constant<int, 2>{}); break;
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 6: f(std::integral_constant<int, 6>{}); break;
+        case 8: f(std::integral_constant<int, 8>{}); break;
+        case 10: f(std::integral_constant<int, 10>{}); break;
+        case 12: f(std::integral_constant<int, 12>{}); break;
+        case 14: f(std::integral_constant<int, 14>{}); break;
+        default: f(std::integral_constant<int, 16>{}); break;
+    }
+}
+
+// The Crank-Nicolson solves of a split-operator step: single lines and, with PAIRS, velocity-gauge odd l-pairs.
+template <bool PAIRS>
+__global__ void __launch_bounds__(PAIRS ? 2 * kAnyP : kAnyP)
+k_sh_solve_any(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const double* __restrict__ cl,
+               ShObs obs) {
+    extern __shared__ double2 lds[];
+    if ((int)blockIdx.x < obs.blocks) {
+        sh_observe_block(obs);
+        return;
+    }
+    const int line = blockIdx.x - obs.blocks;
+    if (line >= n_lines) return;
+    const int2 lt = lines[line];
+    const ShSim& S = sims[lt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;
+    if (PAIRS && (lt.y & kAnyPair)) {
+        if ((int)threadIdx.x >= 2 * S.P) return;
+        sh_by_rows(S.m, [&](auto m) { sh_vpair_lines<decltype(m)::value>(S, n, lt.y & (kAnyPair - 1), cl, lds); });
+    } else {
+        if ((int)threadIdx.x >= S.P) return;
+        sh_by_rows(S.m, [&](auto m) {
+            constexpr int M = decltype(m)::value;
+            sh_rphase_line<M, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS)>(S, n, lt.y, lds);
+        });
+    }
+}
+
+// Threads per chunk of the h2 kernel where SPLIT P threads stay within a workgroup of 512.
+constexpr int sh_vel_split(int M) { return M == 8 || M == 12 || M == 16 ? 2 : 1; }
+
+template <bool REV>
+__global__ void __launch_bounds__(2 * kAnyP) k_sh_vphase_any(ShSim* __restrict__ sims, const int2* __restrict__ pairs,
+                                                             int n_pairs, const double* __restrict__ cl) {
+    __shared__ double2 ex[4][512];
+    if ((int)blockIdx.x >= n_pairs) return;
+    const int2 pt = pairs[blockIdx.x];
+    const ShSim& S = sims[pt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;
+    sh_by_rows(S.m, [&](auto m) {
+        constexpr int M = decltype(m)::value;
+        if ((int)threadIdx.x < sh_vel_split(M) * S.P) sh_vphase_pair<M, REV, sh_vel_split(M)>(S, n, pt.y, cl, ex);
+    });
+}
+
+template <bool EXPL>
+__global__ void __launch_bounds__(kAnyP) __attribute__((amdgpu_waves_per_eu(2, 8))) k_sh_adi_r_any(ShSim* __restrict__ sims, const int2* __restrict__ lines,
+                                                        int n_lines, const int* __restrict__ ctl, ShObs obs) {
+    extern __shared__ double2 lds[];
+    if ((int)blockIdx.x < obs.blocks) {
+        sh_observe_block(obs);
+        return;
+    }
+    const int line = blockIdx.x - obs.blocks;
+    if (line >= n_lines) return;
+    const int2 lt = lines[line];
+    const ShSim& S = sims[lt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N || (int)threadIdx.x >= S.P) return;
+    sh_by_rows(S.m, [&](auto m) { sh_adi_r_line<decltype(m)::value, EXPL>(S, n, lt.y, ctl, lds); });
+}
+
+__global__ void __launch_bounds__(kAdiLanes * kAdiChunks) __attribute__((amdgpu_waves_per_eu(2, 8))) k_sh_adi_lp_any(ShSim* __restrict__ sims,
+                                                                          const int2* __restrict__ groups,
+                                                                          int n_groups, const double* __restrict__ cl) {
+    extern __shared__ double2 lds[];
+    if ((int)blockIdx.x >= n_groups) return;
+    const int2 gt = groups[blockIdx.x];
+    const ShSim& S = sims[gt.x];
+    const int n = S.rstep;
+    if (!S.active || n >= S.N) return;
+    sh_by_rows(sh_adi_lp_rows(S.L), [&](auto m) { sh_adi_lp_group<decltype(m)::value>(S, n, gt.y, cl, lds); });
 }
