@@ -251,6 +251,16 @@ int tdse_sim_state(tdse_ctx *ctx, int32_t kind, int32_t slot, int32_t *step, int
 int tdse_download(tdse_ctx *ctx, int32_t kind, int32_t slot, double *g, double *norms, double *lnorms, double *ips);
 
 /*
+ * The wavefunction in the reference's own order, reordered on the device: SH
+ * l_bound * r_points, Line z_points, Cyl z_points * rho_points complex doubles.
+ * tdse_download_g copies it to the host; tdse_upload_g is tdse_upload_state for
+ * that order (padding positions keep their zeros). Replaces reading and
+ * assigning sim.mesh.g (sims.py:255-346).
+ */
+int tdse_download_g(tdse_ctx *ctx, int32_t kind, int32_t slot, double *g);
+int tdse_upload_g(tdse_ctx *ctx, int32_t kind, int32_t slot, const double *g, int32_t step);
+
+/*
  * Make the device copy of an SH simulation's wavefunction equal to the
  * reference g after its current step count (the step pipeline otherwise keeps
  * the last half of step n-1 fused with the first half of step n). Needed

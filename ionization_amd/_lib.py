@@ -131,6 +131,8 @@ SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32] + [c_double_p] * 4,
     ),
+    "tdse_download_g": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, c_double_p]),
+    "tdse_upload_g": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, c_double_p, ctypes.c_int32]),
     "tdse_download_norm_by_l": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, c_double_p]),
     "tdse_upload_state": (
         ctypes.c_int,

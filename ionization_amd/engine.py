@@ -734,13 +734,17 @@ class DeviceContext:
         """(g (z_points, rho_points), norms, inner products) of a cylindrical simulation."""
         c = self._cyl[slot]
         _, _, nd = self.state(KIND_CYL, slot)
-        g = np.empty((c.nrpad, c.npz), dtype=np.complex128) if with_g else None
         norms = np.empty(nd)
         ips = np.empty((nd, max(1, len(c.basis))), dtype=np.complex128)
-        self._check(self._lib.tdse_download(self._ctx, KIND_CYL, slot, _lib.dptr(g), _lib.dptr(norms), None,
-                                            _lib.dptr(ips)))
-        gn = from_cyl_positions(g, c.z_points, c.rho_points, c.Pz, c.Mz) if with_g else None
-        return gn, norms, ips[:, : len(c.basis)]
+        self._check(self._lib.tdse_download(self._ctx, KIND_CYL, slot, None, _lib.dptr(norms), None, _lib.dptr(ips)))
+        g = self._download_g(KIND_CYL, slot, (c.z_points, c.rho_points)) if with_g else None
+        return g, norms, ips[:, : len(c.basis)]
+
+    def _download_g(self, kind: int, slot: int, shape) -> np.ndarray:
+        """g in natural order: reordered on the device, so the host copies it once."""
+        g = np.empty(shape, dtype=np.complex128)
+        self._check(self._lib.tdse_download_g(self._ctx, kind, slot, _lib.dptr(g)))
+        return g
 
     def run(self, n_steps: int, use_graph: bool = True) -> float:
         """Advance every simulation by n_steps steps; returns the device time in ms."""
@@ -769,13 +773,12 @@ class DeviceContext:
     def download_sh(self, slot: int, with_g: bool = True) -> ShResult:
         c = self._sh[slot]
         _, _, nd = self.state(KIND_SH, slot)
-        g = np.empty((c.l_bound, c.npad), dtype=np.complex128) if with_g else None
         norms = np.empty(nd)
         lnorms = np.empty(nd)
         ips = np.empty((nd, max(1, len(c.basis_l))), dtype=np.complex128)
-        self._check(self._lib.tdse_download(self._ctx, KIND_SH, slot, _lib.dptr(g), _lib.dptr(norms),
-                                            _lib.dptr(lnorms), _lib.dptr(ips)))
-        gn = from_positions(g, c.r_points, c.P, c.m) if with_g else None
+        self._check(self._lib.tdse_download(self._ctx, KIND_SH, slot, None, _lib.dptr(norms), _lib.dptr(lnorms),
+                                            _lib.dptr(ips)))
+        gn = self._download_g(KIND_SH, slot, (c.l_bound, c.r_points)) if with_g else None
         nbl = None
         if c.norm_by_l:
             nbl = np.empty((nd, c.l_bound))
@@ -785,21 +788,20 @@ class DeviceContext:
     def download_line(self, slot: int):
         c = self._line[slot]
         _, _, nd = self.state(KIND_LINE, slot)
-        g = np.empty(c.npad, dtype=np.complex128)
         norms = np.empty(nd)
         ips = np.empty((nd, max(1, len(c.basis))), dtype=np.complex128)
-        self._check(self._lib.tdse_download(self._ctx, KIND_LINE, slot, _lib.dptr(g), _lib.dptr(norms), None,
-                                            _lib.dptr(ips)))
-        return from_positions(g, c.z_points, c.P, c.m), norms, ips[:, : len(c.basis)]
+        self._check(self._lib.tdse_download(self._ctx, KIND_LINE, slot, None, _lib.dptr(norms), None, _lib.dptr(ips)))
+        return self._download_g(KIND_LINE, slot, (c.z_points,)), norms, ips[:, : len(c.basis)]
 
     def upload_state(self, kind: int, slot: int, g_natural: np.ndarray, step: int):
         if kind == KIND_CYL:
             c = self._cyl[slot]
-            gp = np.ascontiguousarray(to_cyl_positions(np.asarray(g_natural, np.complex128), c.Pz, c.Mz, c.nrpad))
+            shape = (c.z_points, c.rho_points)
         else:
             c = self._sh[slot] if kind == KIND_SH else self._line[slot]
-            gp = np.ascontiguousarray(to_positions(np.asarray(g_natural, np.complex128), c.P, c.m))
-        self._check(self._lib.tdse_upload_state(self._ctx, kind, slot, _lib.dptr(gp), int(step)))
+            shape = (c.l_bound, c.r_points) if kind == KIND_SH else (c.z_points,)
+        g = np.ascontiguousarray(g_natural, dtype=np.complex128).reshape(shape)
+        self._check(self._lib.tdse_upload_g(self._ctx, kind, slot, _lib.dptr(g), int(step)))
 
     def materialize(self, kind: int, slot: int):
         """Make the device g equal to the reference g after the current step count."""
