@@ -113,13 +113,8 @@ __device__ __forceinline__ void sh_count_step(ShSim& S, int ctl) {
 // (mesh_operators.py:1201-1250, 1252-1408), diagonal cos a, super-diagonal
 // sin a, sub-diagonal -sin a:
 //     y0 = cos a x0 + sin a x1,    y1 = -sin a x0 + cos a x1.
-// When every lane's angle is small (a weak field: most steps away from a
-// pulse's peak) the whole wave takes the reduction-free series.
-template <bool VEL = false>
-__device__ __forceinline__ void sh_rotate(double a, double2& x0, double2& x1) {
-    double s, c;
-    if (__all(fabs(a) <= kSmallAngle)) tdse_sincos_small(a, &s, &c);
-    else tdse_sincos(a, &s, &c);
+template <bool VEL>
+__device__ __forceinline__ void sh_turn(double s, double c, double2& x0, double2& x1) {
     if constexpr (VEL) {
         const double2 y0 = cmk(fma(c, x0.x, s * x1.x), fma(c, x0.y, s * x1.y));
         const double2 y1 = cmk(fma(c, x1.x, -s * x0.x), fma(c, x1.y, -s * x0.y));
@@ -131,6 +126,62 @@ __device__ __forceinline__ void sh_rotate(double a, double2& x0, double2& x1) {
         x0 = y0;
         x1 = y1;
     }
+}
+
+// When every lane's angle is small (a weak field: most steps away from a
+// pulse's peak) the whole wave takes the reduction-free series.
+template <bool VEL>
+__device__ __forceinline__ void sh_rotate(double a, double2& x0, double2& x1) {
+    double s, c;
+    if (__all(fabs(a) <= kSmallAngle)) tdse_sincos_small(a, &s, &c);
+    else tdse_sincos(a, &s, &c);
+    sh_turn<VEL>(s, c, x0, x1);
+}
+
+// The angles of one half step at a lane's radial position: theta times the coupling of the pair.
+//
+// Length gauge: the coupling c_l = (l + 1) / sqrt((2 l + 1)(2 l + 3)) lies just above 1/2 (0.577 at
+// l = 0, 1/2 + 1/(16 (l + 1)^2) far out), so the sine and cosine of theta / 2 are taken once per wave and
+// each pair adds delta = theta (c_l - 1/2) to that angle by its addition theorem. Where |delta| <= 1/256 the
+// series of delta end at delta^5 and delta^4 (the first omitted terms are below 6e-18): 11 operations and no
+// branch on the lanes' angles against 14 (|a| <= 1/8) or 45 and two tests for a sine and cosine of its own.
+// From l + 1 >= sqrt(256 |theta| / 12) on that holds (c_l - 1/2 <= 1 / (12 (l + 1)^2)): sh_short_rows.
+template <bool VEL>
+struct ShAngle {
+    double theta, half, s0, c0;
+    __device__ __forceinline__ explicit ShAngle(double th) : theta(th), half(0.5 * th), s0(0.0), c0(1.0) {
+        if constexpr (!VEL) {
+            if (__all(fabs(half) <= kSmallAngle)) tdse_sincos_small(half, &s0, &c0);
+            else tdse_sincos(half, &s0, &c0);
+        }
+    }
+    // the sum of two angles
+    __device__ __forceinline__ ShAngle(const ShAngle& a, const ShAngle& b)
+        : theta(a.theta + b.theta), half(0.5 * theta), s0(fma(a.s0, b.c0, a.c0 * b.s0)),
+          c0(fma(a.c0, b.c0, -(a.s0 * b.s0))) {}
+    // c: the pair's coupling, uniform (0 where there is no such pair: the identity); is_short: its row is past
+    // sh_short_rows and the pair exists
+    __device__ __forceinline__ void rotate(double c, bool is_short, double2& x0, double2& x1) const {
+        if (!VEL && is_short) {
+            const double d = fma(theta, c, -half);
+            const double d2 = d * d;
+            const double sd = fma(fma(d2, 0.008333333333333333, -0.16666666666666666) * d2, d, d);
+            const double cd = fma(fma(d2, 0.041666666666666664, -0.5), d2, 1.0);
+            sh_turn<VEL>(fma(s0, cd, c0 * sd), fma(c0, cd, -(s0 * sd)), x0, x1);
+        } else {
+            sh_rotate<VEL>(theta * c, x0, x1);
+        }
+    }
+};
+
+// First row l whose pairs may take the short form in every lane of the wave.
+template <bool VEL>
+__device__ __forceinline__ int sh_short_rows(const ShAngle<VEL>& a, const ShAngle<VEL>& b, const ShAngle<VEL>& c) {
+    if constexpr (VEL) return 0;
+    const double most = fmax(fabs(a.theta), fmax(fabs(b.theta), fabs(c.theta)));
+    // rounded up generously; a huge or non-finite angle never takes the short form
+    int rows = most <= 1e6 ? (int)(sqrtf((float)most * (256.0f / 12.0f)) + 1.01f) : (1 << 28);
+    return wave_max(rows);
 }
 
 // ------------------------------------------------------------------ L-phase
@@ -162,6 +213,14 @@ struct ShWave {
     int sim, p0, lo, hi;
 };
 
+// What bounds it: HBM in large batches (256 simulations: 0.73 ms for 3.56 GB algorithmic, 3.8 GB real = 5.2 TB/s against
+// 6.1 for a copy), its own instructions and the chain table entry -> simulation -> rows in small ones. The row
+// control is scalar, loads take any row (clamped) instead of testing each lane, the ring's slots keep
+// their registers and most rotations take the short sines (ShAngle): about 110 vector instructions per two rows
+// instead of 330. us per step: 250 x 100 16.1 -> 14.5, 200 x 1000 with data every step 24.4 -> 22.2; 256-simulation
+// L-phase 0.748 -> 0.730 ms, with data every step the whole step 1.739 -> 1.687. 4 waves per SIMD (128 VGPRs,
+// 4 spilled): 0.761.
+//
 // BY_L: the instance that can also reduce the norm in every l (launched only
 // while some simulation asks for it: the reductions cost registers).
 // VEL: velocity-gauge simulations. Their h1 coupling has the same pairs and
@@ -174,8 +233,9 @@ template <bool BY_L, bool VEL>
 __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, const ShWave* __restrict__ waves,
                                                    int n_waves, const double* __restrict__ cl, int end_only,
                                                    ShSim* counters) {
-    constexpr int PF = 4;  // prefetch depth in iterations (2 rows each)
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / TDSE_WAVE;
+    constexpr int PF = 4;  // prefetch depth in iterations (2 rows each), and the unrolling of the row loop
+    // the wave's own index, its table entry and all row arithmetic are scalar
+    const int wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / TDSE_WAVE);
     const int lane = threadIdx.x % TDSE_WAVE;
     if (wave >= n_waves) return;
     const ShWave wt = waves[wave];
@@ -199,7 +259,7 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
     const int lo = wt.lo, hi = wt.hi;
     // read once: inside the row loop the snapshot stores could otherwise make the compiler
     // reload these fields every iteration
-    const int LB = S.LB;
+    const int LB = S.LB, n_part = S.n_part;
     double2* __restrict__ const snap = S.snap;
     double* __restrict__ const part_l = S.part_l;
     double* __restrict__ const part = S.part;
@@ -210,23 +270,21 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
     const int q = __builtin_amdgcn_readfirstlane((j & 1) & (L & 1));
     const double rq = ld1(S.tab, SH_RQ * npad + p);
     const double mk = ld1(S.tab, SH_MASK * npad + p);
-    const double f_end = do_end ? ld1(S.fs, n - 1) * rq : 0.0;
-    const double f_start = do_start ? ld1(S.fs, n) * rq : 0.0;
-    const double f_sum = f_end + f_start;
-    const double2* __restrict__ gin = sh_state(S, n) + p;
-    double2* __restrict__ g = sh_state(S, n + 1) + p;
-    // Output row r depends on input rows up to r + 3, so rows from hi + 3 on
-    // (which the prefetch ring would otherwise read up to 2 PF rows ahead) are
-    // not loaded: the next segment's wave reads them.
-    const int l_stop = min(L, hi + 3);
-    auto load_row = [gin, live, l_stop, npad](int l) -> double2 {
-        double2 v = make_double2(0.0, 0.0);
-        if (live && l >= 0 && l < l_stop) v = ld2(gin, (size_t)l * npad);
-        return v;
-    };
-    // coupling of the pair starting at virtual row v (0 when the pair does not exist:
-    // a rotation by 0 is exactly the identity)
-    auto load_c = [cl, q, L](int v) -> double {
+    const ShAngle<VEL> a_end(do_end ? ld1(S.fs, n - 1) * rq : 0.0);
+    const ShAngle<VEL> a_start(do_start ? ld1(S.fs, n) * rq : 0.0);
+    const ShAngle<VEL> a_sum(a_end, a_start);
+    // rows from which every lane of the wave may take the short form of the sines
+    const int l_short = sh_short_rows<VEL>(a_end, a_start, a_sum);
+    auto is_short = [=](int l) { return l >= l_short && l + 1 < L; };
+    const double2* __restrict__ const gin = sh_state(S, n);
+    double2* __restrict__ const gout = sh_state(S, n + 1);
+    // Output row r depends on input rows up to r + 3, so rows from hi + 3 on (which the prefetch ring would
+    // otherwise read up to 2 PF rows ahead) are not read: the next segment's wave reads them. Rows outside
+    // the range stand in for rows nothing depends on (a pair that reaches over the end of l has no coupling).
+    const int l_last = min(L, hi + 3) - 1;
+    auto load_row = [=](int l) -> double2 { return ld2(gin + (size_t)min(max(l, 0), l_last) * npad, (unsigned)p); };
+    // coupling of the pair starting at virtual row v; 0 when the pair does not exist
+    auto load_c = [=](int v) -> double {
         const int l = v - q;
         return (l >= 0 && l + 1 < L) ? ld1(cl, l) : 0.0;
     };
@@ -238,43 +296,33 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
     const int wpl = npad / TDSE_WAVE, wcol = wt.p0 / TDSE_WAVE;
     const double2 zero = make_double2(0.0, 0.0);
     double2 carry_u = zero, carry_s1 = zero, carry_s3 = zero;
+    // couplings of the pairs at virtual rows v0 - 3, v0 - 2, v0 - 1, and of the next iteration's two new ones
     double c_m3 = load_c(2 * it0 - 3), c_m2 = load_c(2 * it0 - 2), c_m1 = load_c(2 * it0 - 1);
+    double c_p0 = load_c(2 * it0), c_p1 = load_c(2 * it0 + 1);
     double acc_norm = 0.0, acc_lnorm = 0.0;
     double2 ring0[PF], ring1[PF];
-    double ringc0[PF], ringc1[PF];
 #pragma unroll
     for (int d = 0; d < PF; ++d) {
         ring0[d] = load_row(2 * (it0 + d) - q);
         ring1[d] = load_row(2 * (it0 + d) + 1 - q);
-        ringc0[d] = load_c(2 * (it0 + d));
-        ringc1[d] = load_c(2 * (it0 + d) + 1);
     }
 
-    for (int it = it0; it <= it_end; ++it) {
+    auto iterate = [&](const int it, double2& slot0, double2& slot1) {
         const int v0 = 2 * it;
-        const double2 u0 = ring0[0], u1 = ring1[0];
-        const double c0 = ringc0[0], c1 = ringc1[0];
-#pragma unroll
-        for (int d = 0; d + 1 < PF; ++d) {
-            ring0[d] = ring0[d + 1];
-            ring1[d] = ring1[d + 1];
-            ringc0[d] = ringc0[d + 1];
-            ringc1[d] = ringc1[d + 1];
-        }
-        ring0[PF - 1] = load_row(v0 + 2 * PF - q);
-        ring1[PF - 1] = load_row(v0 + 2 * PF + 1 - q);
-        ringc0[PF - 1] = load_c(v0 + 2 * PF);
-        ringc1[PF - 1] = load_c(v0 + 2 * PF + 1);
+        const double2 u0 = slot0, u1 = slot1;
+        slot0 = load_row(v0 + 2 * PF - q);
+        slot1 = load_row(v0 + 2 * PF + 1 - q);
+        const double c_n0 = load_c(v0 + 2), c_n1 = load_c(v0 + 3);
+        const int le = v0 - 2 - q;
 
         // stage 1: O_end on (v0-1, v0)
         double2 s1m = carry_u, s10 = u0;
-        if (do_end) sh_rotate<VEL>(f_end * c_m1, s1m, s10);
+        if (do_end) a_end.rotate(c_m1, is_short(le + 1), s1m, s10);
         // stage 2: E_end on (v0-2, v0-1), mask; stage 3: E_start on the same pair
         double2 s2a = carry_s1, s2b = s1m;
-        const int le = v0 - 2 - q;
         if (both && !observe) {
             // E_end and E_start as one rotation (the mask, a function of r only, commutes with both)
-            sh_rotate<VEL>(f_sum * c_m2, s2a, s2b);
+            a_sum.rotate(c_m2, is_short(le), s2a, s2b);
             s2a = cscale(mk, s2a);
             s2b = cscale(mk, s2b);
         } else {
@@ -286,15 +334,15 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
             double2 oa = s2a, ob = s2b;  // the observed rows: g after step n
             if (both) {
                 if (by_l || per_row) {
-                    sh_rotate<VEL>(f_end * c_m2, oa, ob);
+                    a_end.rotate(c_m2, is_short(le), oa, ob);
                     oa = cscale(mk, oa);
                     ob = cscale(mk, ob);
                 }
-                sh_rotate<VEL>(f_sum * c_m2, s2a, s2b);
+                a_sum.rotate(c_m2, is_short(le), s2a, s2b);
                 s2a = cscale(mk, s2a);
                 s2b = cscale(mk, s2b);
             } else if (do_end) {
-                sh_rotate<VEL>(f_end * c_m2, s2a, s2b);
+                a_end.rotate(c_m2, is_short(le), s2a, s2b);
                 s2a = cscale(mk, s2a);
                 s2b = cscale(mk, s2b);
                 oa = s2a;
@@ -307,10 +355,10 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
                     if (!per_row) {
                         acc_norm += cabs2(s2a) + cabs2(s2b);
                     } else {
-                        // rows -1 and L are zero
-                        acc_norm += cabs2(oa) + cabs2(ob);
-                        if (le == L - 1) acc_lnorm = cabs2(oa);
-                        if (le + 1 == L - 1) acc_lnorm = cabs2(ob);
+                        const double na = le >= 0 ? cabs2(oa) : 0.0, nb = le + 1 < L ? cabs2(ob) : 0.0;
+                        acc_norm += na + nb;
+                        if (le == L - 1) acc_lnorm = na;
+                        if (le + 1 == L - 1) acc_lnorm = nb;
                         if (le >= 0 && le < LB) st2(snap, (size_t)le * npad + p, oa);
                         if (le + 1 < LB) st2(snap, (size_t)(le + 1) * npad + p, ob);
                     }
@@ -323,7 +371,7 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
                 }
                 if (last) {
                     const double sum = wave_sum_last(acc_lnorm);
-                    if (lane == TDSE_WAVE - 1) part[S.n_part + wcol] = sum;
+                    if (lane == TDSE_WAVE - 1) part[n_part + wcol] = sum;
                 }
             }
             if (by_l) {
@@ -333,22 +381,31 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
                     if (le + 1 >= lo && le + 1 < hi) part_l[(size_t)(le + 1) * wpl + wcol] = rb;
                 }
             }
-            if (!both && do_start) sh_rotate<VEL>(f_start * c_m2, s2a, s2b);
+            if (!both && do_start) a_start.rotate(c_m2, is_short(le), s2a, s2b);
         }
         // stage 4: O_start on (v0-3, v0-2)
         double2 o_a = carry_s3, o_b = s2a;
-        if (do_start) sh_rotate<VEL>(f_start * c_m3, o_a, o_b);
-        const int lo_row = v0 - 3 - q;
+        if (do_start) a_start.rotate(c_m3, is_short(le - 1), o_a, o_b);
+        const int lo_row = le - 1;
         if (live) {
-            if (lo_row >= lo && lo_row < hi) st2s(g, (size_t)lo_row * npad, o_a);
-            if (lo_row + 1 >= lo && lo_row + 1 < hi) st2s(g, (size_t)(lo_row + 1) * npad, o_b);
+            if (lo_row >= lo && lo_row < hi) st2s(gout + (size_t)lo_row * npad, (unsigned)p, o_a);
+            if (lo_row + 1 >= lo && lo_row + 1 < hi) st2s(gout + (size_t)(lo_row + 1) * npad, (unsigned)p, o_b);
         }
         carry_u = u1;
         carry_s1 = s10;
         carry_s3 = s2b;
         c_m3 = c_m1;
-        c_m2 = c0;
-        c_m1 = c1;
+        c_m2 = c_p0;
+        c_m1 = c_p1;
+        c_p0 = c_n0;
+        c_p1 = c_n1;
+    };
+    // unrolled over the prefetch ring, whose slots so keep their registers: shifting it by an iteration was 48 register
+    // moves of about 200 instructions (unrolled by 1, 2 and 4: 1.587, 1.559 and 1.543 ms per step of the scan)
+    for (int it = it0; it <= it_end; it += PF) {
+#pragma unroll
+        for (int d = 0; d < PF; ++d)
+            if (it + d <= it_end) iterate(it + d, ring0[d], ring1[d]);
     }
     if (begins) counters[wt.sim].rstep = n;
 }
