@@ -35,8 +35,9 @@
 struct CylSim {
     double2* g;             // [nrpad][npz]
     const double* zt;       // [npz] z of every position (0 for padding)
-    const double* rt;       // [nrpad] rho of every rho index (0 for padding)
-    const double* roff;     // [nrpad] rho off-diagonal between j and j + 1: rp c(j + 1); 0 past the line
+    const double* rtab;     // [2][nrpad] of row j = c Mr + i at i Cr + c: the off-diagonal rp c(j + 1) of rho between j and
+                            // j + 1 (row nr - 1: that of row nr - 2; 0 past the line) and its ratio to the one before
+                            // it, off_{j-1} / off_j (0 at j = 0 and past the line)
     const double* fs;       // [N] E(t_{n+1})
     const double* ts;       // [N] tau_n = (t_{n+1} - t_n) / (2 hbar)
     double* part;           // [n_groups][1 + 2 n_basis] observation partials of the rho-sweep blocks
@@ -78,20 +79,12 @@ __device__ __forceinline__ double cyl_half_potential(const CylSim& S, double z, 
     return 0.5 * (S.kc * cyl_rsqrt(z * z + rho * rho)) + 0.5 * (-z * S.q * E);
 }
 
-// Off-diagonal of H_rho between rho indices j and j + 1: rp c(j + 1),
-// c(m) = m / sqrt(m^2 - 1/4) (mesh_operators.py:582-592); 0 past the line.
 // Device order of a cylindrical g (and of its basis states): rho rows in pairs
 // (2 q, 2 q + 1) interleaved position by position, element (r, p) at
 // ((r / 2) npz + p) 2 + r % 2 (nrpad is even). The z-sweep's threads then read
 // whole lines in pairs and the rho-sweep's four positions whole 128 B lines.
 __device__ __forceinline__ size_t cyl_at(int r, int p, int npz) {
     return ((size_t)(r >> 1) * npz + p) * 2 + (r & 1);
-}
-
-__device__ __forceinline__ double cyl_rho_off(const CylSim& S, int j) {
-    if (j < 0 || j + 1 >= S.nr) return 0.0;
-    const double m = (double)(j + 1);
-    return (m * cyl_rsqrt(m * m - 0.25)) * S.rp;
 }
 
 // RadialCosineMask.__call__ (potentials/masks.py:76-89) at r.
@@ -226,21 +219,19 @@ k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, 
         const double z = fma((double)j, dz, z0);
         h = live ? fma(tau, cyl_half_potential(S, z, rho, E), tdiag) : 0.0;
         hm = (live && j >= 1) ? tzp : 0.0;
-        hp = (j + 1 < nz) ? tzp : 0.0;
+        hp = live ? tzp : 0.0;  // row nz - 1 too: its neighbour is a zero padding row
     };
     auto coef2 = [&](int i, double& hm, double& h) {
         double hp;
         coef(i, hm, h, hp);
     };
-    // equal off-diagonals inside the line: hm / hp = 1 from row 1 to nz - 2, so
-    // pass 2 reuses the stored pivots; row nz - 1 (hp = 0) is rebuilt
+    // equal off-diagonals: hm / hp = 1 from row 1 to nz - 1, pass 2 reuses the stored pivots
     auto ratio = [&](int i) {
         const int j = k * M + i;
-        return (j >= 1 && j + 1 < nz) ? 1.0 : 0.0;
+        return (j >= 1 && j < nz) ? 1.0 : 0.0;
     };
-    const int ib = ((nz - 1) / M == k) ? (nz - 1) % M : -1;
     cn_line_finish<M, FORM, decltype(coef), decltype(coef2), decltype(ratio), 2>(x, gl, k, P, coef, coef2, lds, ratio,
-                                                                               ib, ln, 2 * P);
+                                                                               ln, 2 * P);
 }
 
 // ---------------------------------------------------------------- rho-sweep
@@ -248,14 +239,28 @@ k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, 
 // One workgroup of LANES * Cr threads per (simulation, group of LANES
 // consecutive positions): thread t works on line ln = t % LANES (position
 // p = LANES * group + ln) and chunk c = t / LANES (rho rows c Mr .. c Mr + Mr - 1).
-// H_rho: diagonal -2 rp + V/2 - z q E / 2, off-diagonals rp c(j + 1)
+// H_rho: diagonal -2 rp + V/2 - z q E / 2, off-diagonals rp c(j + 1), c(m) = m / sqrt(m^2 - 1/4)
 // (mesh_operators.py:578-600).
+//
+// What bounds it: FP64 issue at 4 waves per SIMD (128 VGPRs). The couplings and their ratios come from the
+// simulation's table, staged in LDS once per workgroup: formed from m each time, they were a reciprocal square root
+// three times per row and a reciprocal, and kept registers busy over the solve. With half the potential in LDS
+// too, the explicit half gained nothing (139.6 us against 140.1 per step of four 2000 x 1000 simulations), so it is
+// formed again. A wave whose points all lie inside the mask's ramp skips it. Padding rows hold zeros, so nothing
+// selects on them. Per step, before and after: one 250 x 100 simulation 18.4 -> 16.3 us, four of 2000 x 1000
+// 151 -> 140, 32 of them 1070 -> 972.
 //
 // MAIN (every step n < N):  implicit half of step n, mask, observables of the
 //     exact g after n + 1 steps at data times, explicit half of step n + 1
 //     unless n + 1 == N or the simulation holds exact states.
 // PRE (phase 1 only): observables of g at step 0, explicit half of step n.
 enum { CYL_PRE = 0, CYL_MAIN = 1 };
+
+// LDS of the rho-sweep: the solver's rows, the couplings and their ratios, reduction scratch.
+constexpr size_t cyl_rho_lds_bytes(int M, int LANES, int P) {
+    return ((size_t)3 * P * LANES + kRedScratch) * sizeof(double2) +
+           ((size_t)2 * M * P + 16) * sizeof(double);
+}
 
 template <int LANES>
 __device__ __forceinline__ double cyl_block_sum(double v, double* red, int t, int nthreads) {
@@ -272,7 +277,7 @@ __device__ __forceinline__ double cyl_block_sum(double v, double* red, int t, in
 template <int M, int LANES, int MODE, int MAXT, int WPE>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_cyl_rho(CylSim* __restrict__ sims, const int2* __restrict__ groups,
                                                   int n_groups, CylJobs jobs) {
-    extern __shared__ double2 lds[];  // 3 * Cr * LANES + kRedScratch double2, then 16 doubles for reductions
+    extern __shared__ double2 lds[];  // cyl_rho_lds_bytes(M, LANES, Cr)
     if ((int)blockIdx.x < jobs.blocks) {
         if (MODE == CYL_MAIN) cyl_job_block<true>(jobs);
         return;
@@ -287,93 +292,55 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
     const int ln = t % LANES, c = t / LANES;
     const int P = S.Cr, nr = S.nr, npz = S.npz;
     const int p = gt.y * LANES + ln;
-    const int jz = (p % S.Pz) * S.Mz + p / S.Pz;
-    const bool line_live = jz < S.nz;
-    const double z = ld1(S.zt, p);
+    double z = ld1(S.zt, p);
     // rows c M .. c M + M - 1 (M even): row c M + i at gl[cyl_at(i, 0, npz)]; with the two
     // rows of a pair adjacent, LANES = 4 neighbouring positions read whole 128 B lines
     double2* __restrict__ gl = S.g + cyl_at(c * M, p, npz);
-    double* red = reinterpret_cast<double*>(lds + 3 * P * LANES + kRedScratch);
+    double* const off = reinterpret_cast<double*>(lds + 3 * P * LANES + kRedScratch);  // [M][P], then the ratios
+    double* const rat = off + M * P;
+    double* const red = rat + M * P;
 
     double2 x[M];
 #pragma unroll
     for (int i = 0; i < M; ++i) x[i] = ld2(gl, cyl_at(i, 0, npz));
+    for (int i = t; i < 2 * M * P; i += P * LANES) off[i] = ld1(S.rtab, i);
+    __syncthreads();
 
-    // rho-direction coefficients of row i (rho index j = c M + i) for (tau, E),
-    // from the grid: rho_j recomputed, the sub-diagonal carried from the
-    // previous row (callers visit rows in order, starting from `carry` =
-    // cyl_rho_off(j0 - 1)).
-    const double a_left = line_live ? cyl_rho_off(S, c * M - 1) : 0.0;
-    // With few rows per thread, half the Coulomb potential (0.5 k Q q / r) and r
-    // (for the mask) are computed once per row, from one refined reciprocal
-    // square root, and kept; with more rows they are recomputed where needed.
-    constexpr bool KEEP = M <= 4;
-    double vhalf[KEEP ? M : 1], rad[KEEP ? M : 1];
-    auto rho_of = [&](int i) { return fma((double)(c * M + i), S.drho, S.rho0); };
-    if constexpr (KEEP) {
-#pragma unroll
-        for (int i = 0; i < M; ++i) {
-            const int j = c * M + i;
-            const double rho = rho_of(i);
-            const double r2 = z * z + rho * rho;
-            const double ri = cyl_rsqrt(r2);
-            vhalf[i] = (line_live && j < nr) ? 0.5 * (S.kc * ri) : 0.0;
-            rad[i] = r2 * ri;
-        }
-    }
-    auto half_v = [&](int i) {
-        if constexpr (KEEP) return vhalf[i < M ? i : 0];
-        const double rho = rho_of(i);
-        return 0.5 * (S.kc * cyl_rsqrt(z * z + rho * rho));
+    const double hk = 0.5 * S.kc, drho = S.drho, rp = S.rp;
+    double rho_c = fma((double)(c * M), drho, S.rho0);  // of row c M
+    auto radius2 = [&](int i) {
+        const double rho = fma((double)i, drho, rho_c);
+        return fma(rho, rho, z * z);
     };
-    auto radius = [&](int i) {
-        if constexpr (KEEP) return rad[i < M ? i : 0];
-        const double rho = rho_of(i);
-        return sqrt(z * z + rho * rho);
-    };
-    auto rho_coef = [&](double& carry, double tau, double E, int i, double& hm, double& h, double& hp) {
-        const int j = c * M + i;
-        const bool live = line_live && j < nr;
-        const double off = live ? cyl_rho_off(S, j) : 0.0;
-        h = live ? fma(tau, half_v(i) + 0.5 * (-z * S.q * E), tau * (S.rp * -2.0)) : 0.0;
-        hm = (live && j >= 1) ? tau * carry : 0.0;
-        hp = tau * off;
-        carry = off;
-    };
+    const double left = c > 0 ? off[(M - 1) * P + c - 1] : 0.0;  // off_{c M - 1}
 
     if constexpr (MODE == CYL_MAIN) {
-        const double tau = ld1(S.ts, n), E = ld1(S.fs, n);
-        double carry1 = a_left, carry3 = a_left;
-        auto coef = [&](int i, double& hm, double& h, double& hp) { rho_coef(carry1, tau, E, i, hm, h, hp); };
-        // row i's coefficients on their own (the one row whose pass-2 pivot is rebuilt)
-        auto coef2 = [&](int i, double& hm, double& h) {
-            double hp, left = cyl_rho_off(S, c * M + i - 1);
-            rho_coef(left, tau, E, i, hm, h, hp);
+        const double tau = ld1(S.ts, n), w = 0.5 * (-z * S.q * ld1(S.fs, n)), kin = tau * (rp * -2.0);
+        double carry = left;
+        auto coef = [&](int i, double& hm, double& h, double& hp) {
+            const double v = fma(hk, cyl_rsqrt(radius2(i)), w);
+            const double o = off[i * P + c];
+            h = fma(tau, v, kin);
+            hm = (c * M + i == nr) ? 0.0 : tau * carry;  // row nr - 1 couples to the first padding row, not it back
+            hp = tau * o;
+            carry = o;
         };
-        // pass-2 pivot ratios hm / hp = c(j) / c(j + 1) (tau cancels), rows in order
-        auto ratio = [&](int i) {
-            const int j = c * M + i;
-            const bool live = line_live && j < nr;
-            const double off = live ? cyl_rho_off(S, j) : 0.0;
-            const double q = (live && j >= 1 && off != 0.0) ? carry3 * tdse_rcp(off) : 0.0;
-            carry3 = off;
-            return q;
-        };
-        const int ib = (line_live && (nr - 1) / M == c) ? (nr - 1) % M : -1;
+        auto coef2 = [](int, double&, double&) {};
+        auto ratio = [&](int i) { return rat[i * P + c]; };
         cn_implicit_lowreg<M, decltype(coef), decltype(coef2), false, LANES, decltype(ratio)>(
-            x, c, P, coef, coef2, lds, cmk(0.0, 0.0), cmk(0.0, 0.0), ln, ratio, ib);
+            x, c, P, coef, coef2, lds, cmk(0.0, 0.0), cmk(0.0, 0.0), ln, ratio);
+        asm volatile("" : "+v"(rho_c), "+v"(z));  // the squared radii are formed again, not kept over the solve
         if (S.has_mask) {
-            // inside the inner radius (most points) the mask is 1: decided on r^2, without the root
-            const double in2 = S.m_inner * S.m_inner;
+            // rows lie at growing radius: inside the inner radius (most points) the mask is 1, from the outer on 0
+            const double in2 = S.m_inner * S.m_inner, out2 = S.m_outer * S.m_outer;
+            if (!__all(radius2(M - 1) < in2)) {
 #pragma unroll
-            for (int i = 0; i < M; ++i) {
-                const int j = c * M + i;
-                double mk = 0.0;
-                if (line_live && j < nr) {
-                    const double rho = rho_of(i);
-                    mk = (!KEEP && z * z + rho * rho < in2) ? 1.0 : cyl_mask_r(S, radius(i));
+                for (int i = 0; i < M; ++i) {
+                    const double r2 = radius2(i);
+                    double mk = r2 < in2 ? 1.0 : 0.0;
+                    if (r2 >= in2 && r2 < out2) mk = cyl_mask_r(S, sqrt(r2));
+                    x[i] = cscale(mk, x[i]);
                 }
-                x[i] = cscale(mk, x[i]);
             }
         }
     }
@@ -412,15 +379,19 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
     const int ne = (MODE == CYL_MAIN) ? n + 1 : n;
     const bool expl = (MODE == CYL_PRE) || (ne < S.N && !S.hold);
     if (expl) {
-        const double tau = ld1(S.ts, ne), E = ld1(S.fs, ne);
+        const double tau = ld1(S.ts, ne), w = 0.5 * (-z * S.q * ld1(S.fs, ne)), kin = tau * (rp * -2.0);
         double2 xl, xr;
         chunk_neighbours<M, LANES>(x, c, P, lds, xl, xr, true, ln);
         double2 prev = xl;
-        double carry3 = a_left;
+        int c1 = c;
+        asm volatile("" : "+v"(c1));  // the table is read again, its rows are not kept over the solve
+        double carry = c1 > 0 ? off[(M - 1) * P + c1 - 1] : 0.0;
 #pragma unroll
         for (int i = 0; i < M; ++i) {
-            double hm, h, hp;
-            rho_coef(carry3, tau, E, i, hm, h, hp);
+            const double v = fma(hk, cyl_rsqrt(radius2(i)), w);
+            const double o = off[i * P + c1];
+            const double h = fma(tau, v, kin), hm = (c1 * M + i == nr) ? 0.0 : tau * carry, hp = tau * o;
+            carry = o;
             const double2 xp = (i + 1 < M) ? x[i + 1 < M ? i + 1 : i] : xr;
             const double2 hx = cmk(fma(hm, prev.x, fma(h, x[i].x, hp * xp.x)), fma(hm, prev.y, fma(h, x[i].y, hp * xp.y)));
             prev = x[i];

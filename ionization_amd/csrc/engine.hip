@@ -786,7 +786,7 @@ void dispatch_cyl_z(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
 template <int M, int LANES, int MAXT, int WPE>
 void launch_cyl_rho(tdse_ctx* ctx, const Bucket& b, hipStream_t st, int mode, bool ride) {
     const CylJobs jobs = cyl_jobs_of(ctx, ctx->cyl_count_jobs, b.Cr * LANES, ride);
-    const size_t lds = (3 * (size_t)b.Cr * LANES + kRedScratch) * sizeof(double2) + 16 * sizeof(double);
+    const size_t lds = cyl_rho_lds_bytes(M, LANES, b.Cr);
     const dim3 grid((unsigned)(b.rlines.count + jobs.blocks)), block((unsigned)(b.Cr * LANES));
     if (mode == CYL_PRE)
         hipLaunchKernelGGL((k_cyl_rho<M, LANES, CYL_PRE, MAXT, WPE>), grid, block, lds, st, ctx->d_cyl,
@@ -1650,12 +1650,20 @@ int tdse_cyl_add(tdse_ctx* ctx, const tdse_cyl_desc* desc, const double* zt, con
     H.n_data = n_data_points(S.N, S.store_every);
     const size_t pts = (size_t)S.nrpad * S.npz;
     double2 *g, *oip, *bas = nullptr;
-    double *dzt, *drt, *droff, *dfs, *dts, *part, *on;
+    double *dzt, *drtab, *dfs, *dts, *part, *on;
+    std::vector<double> rtab(2 * (size_t)S.nrpad, 0.0);  // couplings, then ratios, in the rho-sweep's order
+    double before = 0.0;  // the kernels use the uniform grid and rp of the descriptor, not rt and roff
+    for (int j = 0; j < S.nr; ++j) {
+        const double m = std::min(j + 1, S.nr - 1), o = (m * (1.0 / std::sqrt(m * m - 0.25))) * S.rp;
+        const size_t at = (size_t)(j % Mr) * Cr + j / Mr;
+        rtab[at] = o;
+        rtab[S.nrpad + at] = o != 0.0 ? before / o : 0.0;
+        before = o;
+    }
     int rc = 0;
     if ((rc = copy_to_device(ctx, H.blocks, reinterpret_cast<const double2*>(g0), pts, &g)) ||
         (rc = copy_to_device(ctx, H.blocks, zt, (size_t)S.npz, &dzt)) ||
-        (rc = copy_to_device(ctx, H.blocks, rt, (size_t)S.nrpad, &drt)) ||
-        (rc = copy_to_device(ctx, H.blocks, roff, (size_t)S.nrpad, &droff)) ||
+        (rc = copy_to_device(ctx, H.blocks, rtab.data(), rtab.size(), &drtab)) ||
         (rc = copy_to_device(ctx, H.blocks, fs, (size_t)S.N, &dfs)) ||
         (rc = copy_to_device(ctx, H.blocks, ts, (size_t)S.N, &dts)) ||
         (rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)S.n_groups * (1 + 2 * S.n_basis), &part)) ||
@@ -1669,8 +1677,7 @@ int tdse_cyl_add(tdse_ctx* ctx, const tdse_cyl_desc* desc, const double* zt, con
     }
     S.g = g;
     S.zt = dzt;
-    S.rt = drt;
-    S.roff = droff;
+    S.rtab = drtab;
     S.fs = dfs;
     S.ts = dts;
     S.part = part;

@@ -229,7 +229,7 @@ __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double
                 const double zq = (j < nz) ? fma((double)j, dzq, zq0) : 0.0;
                 h = sw * fma(f, zq, ld1(H1, i * P));
                 hm = (j >= 1 && j < nz) ? so : 0.0;
-                hp = (j + 1 < nz) ? so : 0.0;
+                hp = (j < nz) ? so : 0.0;  // row nz - 1 too: its neighbour is a zero padding row
             };
             auto coef2 = [&](int i, double& hm, double& h) {
                 const double* H2 = H;
@@ -239,15 +239,13 @@ __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double
                 h = sw * fma(f, zq, ld1(H2, i * P));
                 hm = (j >= 1 && j < nz) ? so : 0.0;
             };
-            // equal off-diagonals inside the line: pass 2 reuses the stored pivots
-            // (hm / hp = 1 from row 1 to nz - 2); row nz - 1 (hp = 0) is rebuilt
+            // equal off-diagonals: pass 2 reuses the stored pivots (hm / hp = 1 from row 1 to nz - 1)
             auto ratio = [&](int i) {
                 const int j = k * M + i;
-                return (j >= 1 && j + 1 < nz) ? 1.0 : 0.0;
+                return (j >= 1 && j < nz) ? 1.0 : 0.0;
             };
-            const int ib = ((nz - 1) / M == k) ? (nz - 1) % M : -1;
             cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, 1, decltype(ratio), line_alpha_lds(M)>(
-                x, k, P, coef, coef2, lds, xl, xr, 0, ratio, ib);
+                x, k, P, coef, coef2, lds, xl, xr, 0, ratio);
             if constexpr (METHOD == LINE_SIO_LEN) line_phase<M>(x, k, sw * fs, S.zq0, S.dzq);
             if constexpr (METHOD == LINE_SIO_VEL) line_vel_pairs<M>(x, k, P, lds, sw * fs * S.vq, nz, true);
         } else {

@@ -315,7 +315,7 @@ __device__ __forceinline__ void cn_partition(double2 (&x)[M], const int k, const
 //          pivots recomputed from the stored gamma, delta_i <- delta_i - mu_i;
 //  pass 3 (backward): z_{m-1} = Y_k, z_i = delta_i - gamma_i z_{i+1}.
 // coef(i, hm, h, hp) as for cn_partition; sub = i hm, diag = 1 + i h, sup = i hp.
-// coef2 is called in pass 2 and must re-read the coefficients (not reuse
+// coef2 is called in pass 2 (without Ratio) and must re-read the coefficients (not reuse
 // pass-1 values held in registers across the reduced solve).
 // EXPLICIT: the right-hand side is the explicit half (1 - i H~) x, formed
 // row by row in pass 1 from x and the chunk neighbours xl = x_{km-1},
@@ -324,9 +324,10 @@ __device__ __forceinline__ void cn_partition(double2 (&x)[M], const int k, const
 //
 // Ratio: when given (not NoRatio), pass 2 takes the sub-diagonal pivot factor
 // rsub_i = i hm_i / den_i from the stored super-diagonal one, g_i = i hp_i / den_i,
-// as rsub_i = g_i (hm_i / hp_i), with ratio(i) = hm_i / hp_i (0 where hm_i = 0):
-// a product instead of rebuilding den_i and its reciprocal. Row ib of the thread
-// (the one row of the line with hp = 0 and hm != 0, or -1) is rebuilt as before.
+// as rsub_i = g_i (hm_i / hp_i), with ratio(i) = hm_i / hp_i: a product instead of
+// rebuilding den_i and its reciprocal. It needs hp_i != 0 wherever hm_i != 0, so the
+// caller couples the line's last row n - 1 to row n as well: row n is padding, x_n = 0 and
+// uncoupled itself (hm_n = 0), so y_n = 0 and the coupling adds nothing.
 //
 // ALPHA_LDS (fewer instructions and registers; used where the two-line kernel
 // would otherwise spill):
@@ -347,7 +348,7 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
                                                    Coef2 coef2, double2* __restrict__ lds,
                                                    const double2 xl = make_double2(0.0, 0.0),
                                                    const double2 xr = make_double2(0.0, 0.0), const int ln = 0,
-                                                   Ratio ratio = Ratio{}, const int ib = -1, const bool pcr = true) {
+                                                   Ratio ratio = Ratio{}, const bool pcr = true) {
     double2* __restrict__ alds = lds + (3 * P + k) * LANES + kRedScratch + ln;  // alpha_i at alds[i P LANES]
     double2 ga[M - 1], de[M - 1];
     double2 al = cmk(0.0, 0.0), pi = cmk(1.0, 0.0), sa = cmk(0.0, 0.0), sd = cmk(0.0, 0.0);
@@ -473,19 +474,15 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
 #pragma unroll
     for (int i = 0; i < M - 1; ++i) {
         double2 rsub;
-        auto direct = [&]() {
+        if constexpr (std::is_same_v<Ratio, NoRatio>) {
             double hm, h;
             coef2(i, hm, h);
             const double2 den = (i == 0) ? cmk(1.0, h) : cmk(fma(hm, ga[i - 1 > 0 ? i - 1 : 0].y, 1.0),
                                                               fma(-hm, ga[i - 1 > 0 ? i - 1 : 0].x, h));
-            return cimul(hm, crecip(den));
-        };
-        if constexpr (std::is_same_v<Ratio, NoRatio>) {
-            rsub = direct();
+            rsub = cimul(hm, crecip(den));
         } else {
             const double q = ratio(i);
             rsub = cmk(ga[i].x * q, ga[i].y * q);
-            if (i == ib) rsub = direct();
         }
         mu = (i == 0) ? cmul(rsub, Lk) : cneg(cmul(rsub, mu));
         de[i] = csub(de[i], mu);

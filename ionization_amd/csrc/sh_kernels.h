@@ -493,20 +493,19 @@ enum { CN_CAYLEY_MEM = 0, CN_CAYLEY_LDS = 1, CN_EXPLICIT = 2 };
 
 // Shared tail of the CN line kernels: x holds the thread's M rows of the line
 // at gl (row i at gl[i * stride]; stride P by default); solves and stores
-// y = (1 + i H~)^-1 (1 - i H~) x. Ratio / ib: optional pass-2 pivot ratios
+// y = (1 + i H~)^-1 (1 - i H~) x. Ratio: optional pass-2 pivot ratios
 // (cn_implicit_lowreg). LANES / ln: LANES lines per workgroup, interleaved in LDS.
 // store = false: the thread solves but writes nothing (rows that are all padding).
 template <int M, int FORM, class Coef, class Coef2, class Ratio = NoRatio, int LANES = 1>
 __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restrict__ gl, const int k, const int P,
                                                Coef coef, Coef2 coef2, double2* __restrict__ lds,
-                                               Ratio ratio = Ratio{}, const int ib = -1, const int ln = 0,
-                                               const int stride = -1, const bool store = true,
+                                               Ratio ratio = Ratio{}, const int ln = 0, const int stride = -1, const bool store = true,
                                                const bool pcr = true) {
     const size_t st = stride < 0 ? (size_t)P : (size_t)stride;
     if constexpr (FORM == CN_EXPLICIT) {
         double2 xl, xr;
         chunk_neighbours<M, LANES>(x, k, P, lds, xl, xr, false, ln);
-        cn_implicit_lowreg<M, Coef, Coef2, true, LANES, Ratio>(x, k, P, coef, coef2, lds, xl, xr, ln, ratio, ib, pcr);
+        cn_implicit_lowreg<M, Coef, Coef2, true, LANES, Ratio>(x, k, P, coef, coef2, lds, xl, xr, ln, ratio, pcr);
         if (store) {
 #pragma unroll
             for (int i = 0; i < M; ++i) st2s(gl, (size_t)i * st, x[i]);
@@ -518,7 +517,7 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
             for (int i = 0; i < M; ++i) keep[(i * P + k) * LANES + ln] = x[i];
         }
         cn_implicit_lowreg<M, Coef, Coef2, false, LANES, Ratio>(x, k, P, coef, coef2, lds, cmk(0.0, 0.0),
-                                                                cmk(0.0, 0.0), ln, ratio, ib, pcr);
+                                                                cmk(0.0, 0.0), ln, ratio, pcr);
         if (!store) return;
 #pragma unroll
         for (int i = 0; i < M; ++i) {
@@ -601,7 +600,7 @@ __device__ __forceinline__ void sh_rphase_line(const ShSim& S, const int n, cons
         hm = sn * carry2;
         carry2 = tv.y;
     };
-    cn_line_finish<M, FORM>(x, gl, k, P, coef, coef2, lds, NoRatio{}, -1, 0, -1, !pad, !S.vel);
+    cn_line_finish<M, FORM>(x, gl, k, P, coef, coef2, lds, NoRatio{}, 0, -1, !pad, !S.vel);
 }
 
 template <int M, int MAXT, int WPE, int FORM>
@@ -908,7 +907,7 @@ __device__ __forceinline__ void sh_vpair_lines(const ShSim& S, const int n, cons
     double2 xl, xr;
     chunk_neighbours<M, 2>(x, k, P, lds, xl, xr, true, ln);
     cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, 2, NoRatio, true>(x, k, P, coef, coef2, lds, xl, xr, ln,
-                                                                                     NoRatio{}, -1, false);
+                                                                                     NoRatio{}, false);
     if (fh != 0.0) sh_vpair_factors<M>(x, k, P, ln, lds, av, fp, true);
     if (pad) return;
 #pragma unroll
@@ -1023,7 +1022,7 @@ __device__ __forceinline__ void sh_adi_r_line(const ShSim& S, const int n, const
             carry2 = tv.y;
         };
         cn_implicit_lowreg<M, decltype(coef), decltype(coef2), false, 1>(x, k, P, coef, coef2, lds, cmk(0.0, 0.0),
-                                                                         cmk(0.0, 0.0), 0, NoRatio{}, -1, false);
+                                                                         cmk(0.0, 0.0), 0, NoRatio{}, false);
         if (sh_adi_ahead(S, n, *ctl)) {  // uniform across the block
             const double* mk = S.tab + (size_t)SH_MASK * npad + k;
             asm volatile("" : "+v"(mk));  // loaded after the solve, not hoisted into it
@@ -1157,7 +1156,7 @@ __device__ __forceinline__ void sh_adi_lp_group(const ShSim& S, const int n, con
     double2 xl, xr;
     chunk_neighbours<M, LANES>(x, c, kAdiChunks, lds, xl, xr, false, ln);
     cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, LANES>(x, c, kAdiChunks, coef, coef2, lds, xl, xr,
-                                                                        ln, NoRatio{}, -1, false);
+                                                                        ln, NoRatio{}, false);
 #pragma unroll
     for (int i = 0; i < M; ++i) {
         const int l = c * M + i;
