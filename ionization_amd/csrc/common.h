@@ -62,6 +62,10 @@ __device__ __forceinline__ double2 cneg(double2 a) { return cmk(-a.x, -a.y); }
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
     return cmk(fma(a.x, b.x, -a.y * b.y), fma(a.x, b.y, a.y * b.x));
 }
+// c + a b in four fused operations (cadd(c, cmul(a, b)) takes six)
+__device__ __forceinline__ double2 cmla(double2 c, double2 a, double2 b) {
+    return cmk(fma(a.x, b.x, fma(-a.y, b.y, c.x)), fma(a.x, b.y, fma(a.y, b.x, c.y)));
+}
 __device__ __forceinline__ double2 cscale(double s, double2 a) { return cmk(s * a.x, s * a.y); }
 // (i * s) * a for real s: i s (x + iy) = -s y + i s x
 __device__ __forceinline__ double2 cimul(double s, double2 a) { return cmk(-s * a.y, s * a.x); }

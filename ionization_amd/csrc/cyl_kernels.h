@@ -35,9 +35,8 @@
 struct CylSim {
     double2* g;             // [nrpad][npz]
     const double* zt;       // [npz] z of every position (0 for padding)
-    const double* rtab;     // [2][nrpad] of row j = c Mr + i at i Cr + c: the off-diagonal rp c(j + 1) of rho between j and
-                            // j + 1 (row nr - 1: that of row nr - 2; 0 past the line) and its ratio to the one before
-                            // it, off_{j-1} / off_j (0 at j = 0 and past the line)
+    const double* roff;     // [nrpad] off-diagonal rp c(j + 1) of rho between j = c Mr + i and j + 1, at i Cr + c; 0 past
+                            // the line
     const double* fs;       // [N] E(t_{n+1})
     const double* ts;       // [N] tau_n = (t_{n+1} - t_n) / (2 hbar)
     double* part;           // [n_groups][1 + 2 n_basis] observation partials of the rho-sweep blocks
@@ -213,25 +212,17 @@ k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, 
 #pragma unroll
     for (int i = 0; i < M; ++i) x[i] = ld2(gl, (size_t)i * P * 2);
     // coefficients from the grid, no table reads
-    auto coef = [&](int i, double& hm, double& h, double& hp) {
+    auto off = [&](int i) { return (k * M + i + 1 < nz) ? tzp : 0.0; };
+    auto coef = [&](int i, double& h, double& o) {
         const int j = k * M + i;
-        const bool live = j < nz;
         const double z = fma((double)j, dz, z0);
-        h = live ? fma(tau, cyl_half_potential(S, z, rho, E), tdiag) : 0.0;
-        hm = (live && j >= 1) ? tzp : 0.0;
-        hp = live ? tzp : 0.0;  // row nz - 1 too: its neighbour is a zero padding row
+        h = j < nz ? fma(tau, cyl_half_potential(S, z, rho, E), tdiag) : 0.0;
+        o = off(i);
     };
-    auto coef2 = [&](int i, double& hm, double& h) {
-        double hp;
-        coef(i, hm, h, hp);
+    auto solve = [&](auto expl, const double2 xl, const double2 xr) {
+        cn_symmetric<M, decltype(expl)::value, 2>(x, k, P, (k > 0 && k * M < nz) ? tzp : 0.0, coef, off, lds, xl, xr, ln);
     };
-    // equal off-diagonals: hm / hp = 1 from row 1 to nz - 1, pass 2 reuses the stored pivots
-    auto ratio = [&](int i) {
-        const int j = k * M + i;
-        return (j >= 1 && j < nz) ? 1.0 : 0.0;
-    };
-    cn_line_finish<M, FORM, decltype(coef), decltype(coef2), decltype(ratio), 2>(x, gl, k, P, coef, coef2, lds, ratio,
-                                                                               ln, 2 * P);
+    cn_line_finish<M, FORM, 2>(x, gl, k, P, lds, solve, ln, 2 * P, true);
 }
 
 // ---------------------------------------------------------------- rho-sweep
@@ -242,13 +233,13 @@ k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, 
 // H_rho: diagonal -2 rp + V/2 - z q E / 2, off-diagonals rp c(j + 1), c(m) = m / sqrt(m^2 - 1/4)
 // (mesh_operators.py:578-600).
 //
-// What bounds it: FP64 issue at 4 waves per SIMD (128 VGPRs). The couplings and their ratios come from the
-// simulation's table, staged in LDS once per workgroup: formed from m each time, they were a reciprocal square root
-// three times per row and a reciprocal, and kept registers busy over the solve. With half the potential in LDS
-// too, the explicit half gained nothing (139.6 us against 140.1 per step of four 2000 x 1000 simulations), so it is
-// formed again. A wave whose points all lie inside the mask's ramp skips it. Padding rows hold zeros, so nothing
-// selects on them. Per step, before and after: one 250 x 100 simulation 18.4 -> 16.3 us, four of 2000 x 1000
-// 151 -> 140, 32 of them 1070 -> 972.
+// What bounds it: FP64 issue at 4 waves per SIMD (128 VGPRs). The couplings come from the simulation's table,
+// staged in LDS once per workgroup: formed from m each time, they were a reciprocal square root three times per row
+// and a reciprocal for their ratio, and kept registers busy over the solve. With half the potential in LDS too, the
+// explicit half gained nothing (139.6 us against 140.1 per step of four 2000 x 1000 simulations), so it is formed
+// again. A wave whose points all lie inside the mask's ramp skips it. Padding rows hold zeros, so nothing selects on
+// them. Per step, before and after (with cn_symmetric): one 250 x 100 simulation 18.4 -> 16.0 us, four of 2000 x 1000
+// 151 -> 133, 32 of them 1070 -> 942.
 //
 // MAIN (every step n < N):  implicit half of step n, mask, observables of the
 //     exact g after n + 1 steps at data times, explicit half of step n + 1
@@ -259,7 +250,7 @@ enum { CYL_PRE = 0, CYL_MAIN = 1 };
 // LDS of the rho-sweep: the solver's rows, the couplings and their ratios, reduction scratch.
 constexpr size_t cyl_rho_lds_bytes(int M, int LANES, int P) {
     return ((size_t)3 * P * LANES + kRedScratch) * sizeof(double2) +
-           ((size_t)2 * M * P + 16) * sizeof(double);
+           ((size_t)M * P + 16) * sizeof(double);
 }
 
 template <int LANES>
@@ -290,20 +281,19 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
     if (MODE == CYL_PRE && S.phase != 1) return;
     const int t = threadIdx.x;
     const int ln = t % LANES, c = t / LANES;
-    const int P = S.Cr, nr = S.nr, npz = S.npz;
+    const int P = S.Cr, npz = S.npz;
     const int p = gt.y * LANES + ln;
     double z = ld1(S.zt, p);
     // rows c M .. c M + M - 1 (M even): row c M + i at gl[cyl_at(i, 0, npz)]; with the two
     // rows of a pair adjacent, LANES = 4 neighbouring positions read whole 128 B lines
     double2* __restrict__ gl = S.g + cyl_at(c * M, p, npz);
-    double* const off = reinterpret_cast<double*>(lds + 3 * P * LANES + kRedScratch);  // [M][P], then the ratios
-    double* const rat = off + M * P;
-    double* const red = rat + M * P;
+    double* const off = reinterpret_cast<double*>(lds + 3 * P * LANES + kRedScratch);  // [M][P]
+    double* const red = off + M * P;
 
     double2 x[M];
 #pragma unroll
     for (int i = 0; i < M; ++i) x[i] = ld2(gl, cyl_at(i, 0, npz));
-    for (int i = t; i < 2 * M * P; i += P * LANES) off[i] = ld1(S.rtab, i);
+    for (int i = t; i < M * P; i += P * LANES) off[i] = ld1(S.roff, i);
     __syncthreads();
 
     const double hk = 0.5 * S.kc, drho = S.drho, rp = S.rp;
@@ -316,20 +306,17 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
 
     if constexpr (MODE == CYL_MAIN) {
         const double tau = ld1(S.ts, n), w = 0.5 * (-z * S.q * ld1(S.fs, n)), kin = tau * (rp * -2.0);
-        double carry = left;
-        auto coef = [&](int i, double& hm, double& h, double& hp) {
-            const double v = fma(hk, cyl_rsqrt(radius2(i)), w);
-            const double o = off[i * P + c];
-            h = fma(tau, v, kin);
-            hm = (c * M + i == nr) ? 0.0 : tau * carry;  // row nr - 1 couples to the first padding row, not it back
-            hp = tau * o;
-            carry = o;
+        auto off_at = [&](int i) {
+            int c2 = c;
+            asm volatile("" : "+v"(c2));  // the table is read again, its rows are not kept over the solve
+            return tau * off[i * P + c2];
         };
-        auto coef2 = [](int, double&, double&) {};
-        auto ratio = [&](int i) { return rat[i * P + c]; };
-        cn_implicit_lowreg<M, decltype(coef), decltype(coef2), false, LANES, decltype(ratio)>(
-            x, c, P, coef, coef2, lds, cmk(0.0, 0.0), cmk(0.0, 0.0), ln, ratio);
-        asm volatile("" : "+v"(rho_c), "+v"(z));  // the squared radii are formed again, not kept over the solve
+        auto coef = [&](int i, double& h, double& o) {
+            h = fma(tau, fma(hk, cyl_rsqrt(radius2(i)), w), kin);
+            o = tau * off[i * P + c];
+        };
+        cn_symmetric<M, false, LANES>(x, c, P, tau * left, coef, off_at, lds, cmk(0.0, 0.0), cmk(0.0, 0.0), ln);
+        asm volatile("" : "+v"(rho_c), "+v"(z), "+v"(gl));  // radii and addresses are formed again, not kept over the solve
         if (S.has_mask) {
             // rows lie at growing radius: inside the inner radius (most points) the mask is 1, from the outer on 0
             const double in2 = S.m_inner * S.m_inner, out2 = S.m_outer * S.m_outer;
@@ -384,13 +371,13 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 
         chunk_neighbours<M, LANES>(x, c, P, lds, xl, xr, true, ln);
         double2 prev = xl;
         int c1 = c;
-        asm volatile("" : "+v"(c1));  // the table is read again, its rows are not kept over the solve
+        asm volatile("" : "+v"(c1));  // as above
         double carry = c1 > 0 ? off[(M - 1) * P + c1 - 1] : 0.0;
 #pragma unroll
         for (int i = 0; i < M; ++i) {
             const double v = fma(hk, cyl_rsqrt(radius2(i)), w);
             const double o = off[i * P + c1];
-            const double h = fma(tau, v, kin), hm = (c1 * M + i == nr) ? 0.0 : tau * carry, hp = tau * o;
+            const double h = fma(tau, v, kin), hm = tau * carry, hp = tau * o;
             carry = o;
             const double2 xp = (i + 1 < M) ? x[i + 1 < M ? i + 1 : i] : xr;
             const double2 hx = cmk(fma(hm, prev.x, fma(h, x[i].x, hp * xp.x)), fma(hm, prev.y, fma(h, x[i].y, hp * xp.y)));

@@ -146,6 +146,7 @@ struct Bucket {
     int M = 0;  // exact rows per chunk-thread
     int P = 0;
     bool imag = false;  // Line: complex time steps (imaginary-time relaxation)
+    bool vel = false;   // SH: velocity gauge
     int method = 0;     // Line: LINE_ADI, LINE_SIO_LEN or LINE_SIO_VEL
     size_t lds = 0;     // Line, M == 0 (any layouts): dynamic LDS of the launch
     int Mr = 0, Cr = 0, lanes = 1;  // cylindrical rho-sweep: rows per thread, chunks, lines per workgroup
@@ -219,10 +220,10 @@ struct tdse_ctx {
     hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
     // every layout in one launch for each sweep (any_layouts): the buckets' lines, longest first
     bool any_sh = false, any_adi = false;
-    DevVec<int2> any_lines, any_pairs, any_adi_lines, any_adi_groups;
-    int any_threads = 0, any_pair_threads = 0, any_adi_threads = 0;
-    size_t any_lds = 0, any_adi_lds = 0;
-    bool any_has_pairs = false;  // some entries of any_lines are velocity odd l-pairs
+    // (any_lines: length gauge; any_vlines: velocity gauge, its odd l-pairs marked kAnyPair; any_pairs: its even ones)
+    DevVec<int2> any_lines, any_vlines, any_pairs, any_adi_lines, any_adi_groups;
+    int any_threads = 0, any_vthreads = 0, any_pair_threads = 0, any_adi_threads = 0;
+    size_t any_lds = 0, any_vlds = 0, any_adi_lds = 0;
     std::vector<Bucket> line_buckets;
     bool dirty = true;
     bool sh_norm_by_l = false;   // some live SH simulation reduces the norm in every l (L-phase instance)
@@ -284,7 +285,7 @@ void drop_graph(tdse_ctx* ctx) {
     ctx->graph_k = nullptr;
 }
 
-size_t line_lds_bytes(int M, int P, bool real_steps);
+size_t line_lds_bytes(int P);
 size_t cn_lds_bytes(int M, int P, int form);
 int cn_form(int M, int P);
 size_t vpair_lds_bytes(int M, int P);
@@ -302,8 +303,9 @@ bool any_layouts(const Layouts& lines, const Layouts& pairs, int64_t limit) {
     int64_t points = 0;
     for (const Layouts* m : {&lines, &pairs})
         for (auto& kv : *m) {
-            if (kv.first.second > kAnyP) return false;
-            points += (int64_t)kv.second.size() * kv.first.first * kv.first.second;
+            const int P = kv.first.second % 4096;
+            if (P > kAnyP) return false;
+            points += (int64_t)kv.second.size() * kv.first.first * P;
         }
     return lines.size() + pairs.size() > 1 && points <= limit;
 }
@@ -311,32 +313,34 @@ bool any_layouts(const Layouts& lines, const Layouts& pairs, int64_t limit) {
 // The single-launch tables of the split-operator and ADI simulations (longest lines first).
 int build_any(tdse_ctx* ctx, const Layouts& lines, const Layouts (&vpairs)[2], const Layouts& fpairs,
               const Layouts& adi, const Layouts& adi_groups) {
-    std::vector<int2> solve, pairs, al, ag;
+    std::vector<int2> solve, vsolve, pairs, al, ag;
     int rc;
     // pairs count half their points (one entry for two rows)
     ctx->any_sh = any_layouts(lines, fpairs, fpairs.empty() ? kAnyPoints : kAnyPointsMore / 2);
     ctx->any_adi = any_layouts(adi, adi_groups, kAnyPointsMore) && ctx->adi_waves.count == 0;
-    ctx->any_threads = ctx->any_pair_threads = ctx->any_adi_threads = 0;
-    ctx->any_lds = ctx->any_adi_lds = 0;
-    ctx->any_has_pairs = false;
+    ctx->any_threads = ctx->any_vthreads = ctx->any_pair_threads = ctx->any_adi_threads = 0;
+    ctx->any_lds = ctx->any_vlds = ctx->any_adi_lds = 0;
     if (ctx->any_sh) {
         for (auto it = fpairs.rbegin(); it != fpairs.rend(); ++it) {
-            const int M = it->first.first, P = it->first.second;
-            for (const int2& e : it->second) solve.push_back(make_int2(e.x, e.y | kAnyPair));
-            ctx->any_has_pairs = true;
-            ctx->any_threads = std::max(ctx->any_threads, 2 * P);
-            ctx->any_lds = std::max(ctx->any_lds, vpair_lds_bytes(M, P));
+            const int M = it->first.first, P = it->first.second % 4096;
+            for (const int2& e : it->second) vsolve.push_back(make_int2(e.x, e.y | kAnyPair));
+            ctx->any_vthreads = std::max(ctx->any_vthreads, 2 * P);
+            ctx->any_vlds = std::max(ctx->any_vlds, vpair_lds_bytes(M, P));
         }
         for (auto it = lines.rbegin(); it != lines.rend(); ++it) {
-            const int M = it->first.first, P = it->first.second;
-            solve.insert(solve.end(), it->second.begin(), it->second.end());
-            ctx->any_threads = std::max(ctx->any_threads, P);
-            ctx->any_lds = std::max(ctx->any_lds, cn_lds_bytes(M, P, cn_form(M, P)));
+            const int M = it->first.first, P = it->first.second % 4096;
+            const bool vel = it->first.second >= 4096;
+            auto& list = vel ? vsolve : solve;
+            list.insert(list.end(), it->second.begin(), it->second.end());
+            int& threads = vel ? ctx->any_vthreads : ctx->any_threads;
+            size_t& lds = vel ? ctx->any_vlds : ctx->any_lds;
+            threads = std::max(threads, P);
+            lds = std::max(lds, cn_lds_bytes(M, P, cn_form(M, P)));
         }
         // up to kAnyP threads the odd l-pairs are solved with the lines: only the even ones are left
         for (auto it = vpairs[0].rbegin(); it != vpairs[0].rend(); ++it) {
             pairs.insert(pairs.end(), it->second.begin(), it->second.end());
-            ctx->any_pair_threads = std::max(ctx->any_pair_threads, sh_vel_split(it->first.first) * it->first.second);
+            ctx->any_pair_threads = std::max(ctx->any_pair_threads, sh_vel_split(it->first.first) * (it->first.second % 4096));
         }
     }
     if (ctx->any_adi) {
@@ -348,7 +352,8 @@ int build_any(tdse_ctx* ctx, const Layouts& lines, const Layouts (&vpairs)[2], c
         for (auto it = adi_groups.rbegin(); it != adi_groups.rend(); ++it)
             ag.insert(ag.end(), it->second.begin(), it->second.end());
     }
-    if ((rc = devvec_upload(ctx, ctx->any_lines, solve)) || (rc = devvec_upload(ctx, ctx->any_pairs, pairs)) ||
+    if ((rc = devvec_upload(ctx, ctx->any_lines, solve)) || (rc = devvec_upload(ctx, ctx->any_vlines, vsolve)) ||
+        (rc = devvec_upload(ctx, ctx->any_pairs, pairs)) ||
         (rc = devvec_upload(ctx, ctx->any_adi_lines, al)) || (rc = devvec_upload(ctx, ctx->any_adi_groups, ag)))
         return rc;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // the host vectors end here
@@ -360,7 +365,7 @@ int rebuild_tables(tdse_ctx* ctx) {
     std::vector<ShWave> waves;
     std::vector<int2> jobs, ajobs;
     ctx->n_len_waves = -1;
-    std::map<std::pair<int, int>, std::vector<int2>> shb, lnb;  // (rows, chunks [+ 4096 if complex steps])
+    std::map<std::pair<int, int>, std::vector<int2>> shb, lnb;  // (rows, chunks [+ 4096 if velocity gauge / complex steps])
     std::map<std::pair<bool, int>, std::vector<int>> lna;       // lines of any layout, (complex steps, method)
     std::map<std::pair<int, int>, std::vector<int2>> vpb[2];    // velocity l-pairs by parity, (rows, chunks)
     std::map<std::pair<int, int>, std::vector<int2>> fpb;       // velocity odd l-pairs solved in one workgroup
@@ -405,7 +410,8 @@ int rebuild_tables(tdse_ctx* ctx) {
             }
             continue;
         }
-        auto& v = shb[{h.dev.m, h.dev.P}];
+        const std::pair<int, int> layout{h.dev.m, h.dev.P + (h.vel ? 4096 : 0)};
+        auto& v = shb[layout];
         // velocity gauge: where two lines fit one workgroup (2 P <= 512) the odd l-pairs are
         // solved together with their h2 factors; the rows outside them stay single lines
         const bool fuse = h.vel && 2 * h.dev.P <= kMaxPairThreads;
@@ -415,8 +421,8 @@ int rebuild_tables(tdse_ctx* ctx) {
         }
         if (h.vel)
             for (int l = 0; l + 1 < h.dev.L; ++l) {
-                if (fuse && (l & 1)) fpb[{h.dev.m, h.dev.P}].push_back(make_int2(s, l));
-                else vpb[l & 1][{h.dev.m, h.dev.P}].push_back(make_int2(s, l));
+                if (fuse && (l & 1)) fpb[layout].push_back(make_int2(s, l));
+                else vpb[l & 1][layout].push_back(make_int2(s, l));
             }
     }
     if (ctx->n_len_waves < 0) ctx->n_len_waves = (int)waves.size();
@@ -457,7 +463,7 @@ int rebuild_tables(tdse_ctx* ctx) {
             Bucket b;
             b.M = kv.first.first;
             b.P = kv.first.second % 4096;
-            b.imag = (kv.first.second % 8192) >= 4096;
+            b.imag = b.vel = (kv.first.second % 8192) >= 4096;
             b.method = kv.first.second / 8192;
             int r = devvec_upload(ctx, b.lines, kv.second);
             if (r) return r;
@@ -471,11 +477,13 @@ int rebuild_tables(tdse_ctx* ctx) {
     if ((rc = fill(ctx->sh_adi_lbuckets, alb))) return rc;
     if ((rc = devvec_upload(ctx, ctx->adi_waves, adw))) return rc;
     for (auto& b : ctx->sh_buckets) {
+        if (!b.vel) continue;
+        const std::pair<int, int> layout{b.M, b.P + 4096};
         for (int par = 0; par < 2; ++par) {
-            auto it = vpb[par].find({b.M, b.P});
+            auto it = vpb[par].find(layout);
             if (it != vpb[par].end() && (rc = devvec_upload(ctx, b.vpairs[par], it->second))) return rc;
         }
-        auto it = fpb.find({b.M, b.P});
+        auto it = fpb.find(layout);
         if (it != fpb.end() && (rc = devvec_upload(ctx, b.fpairs, it->second))) return rc;
     }
     if ((rc = build_any(ctx, shb, vpb, fpb, adb, alb))) return rc;
@@ -496,7 +504,7 @@ int rebuild_tables(tdse_ctx* ctx) {
             ids.push_back(make_int2(s, 0));
             one_layout = one_layout && S.m == first.m && S.P == first.P;
             b.P = std::max(b.P, S.P);
-            b.lds = std::max(b.lds, line_lds_bytes(S.m, S.P, !b.imag));
+            b.lds = std::max(b.lds, line_lds_bytes(S.P));
         }
         b.M = one_layout ? first.m : 0;
         if ((rc = devvec_upload(ctx, b.lines, ids))) return rc;
@@ -578,15 +586,13 @@ void launch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
     const size_t lds = cn_lds_bytes(M, b.P, form);
     const ShObs obs = obs_of(ctx, ctx->jobs, b.P, ride);
     const dim3 grid((unsigned)(b.lines.count + obs.blocks)), block(b.P);
-    if (form == CN_EXPLICIT)
-        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
-                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
-    else if (form == CN_CAYLEY_LDS)
-        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS)>), grid, block, lds,
-                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
-    else
-        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
-                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
+    auto launch = [&](auto length, auto velocity) {
+        hipLaunchKernelGGL(b.vel ? velocity : length, grid, block, lds, st, ctx->d_sh, b.lines.ptr, (int)b.lines.count,
+                           obs);
+    };
+    constexpr int kMem = M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM, kLds = M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS;
+    if (form == CN_CAYLEY_LDS) launch(k_sh_rphase<M, MAXT, WPE, kLds, false>, k_sh_rphase<M, MAXT, WPE, kLds, true>);
+    else launch(k_sh_rphase<M, MAXT, WPE, kMem, false>, k_sh_rphase<M, MAXT, WPE, kMem, true>);
 }
 
 void dispatch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
@@ -694,14 +700,14 @@ void dispatch_vphase(tdse_ctx* ctx, const Bucket& b, int par, hipStream_t st) {
     }
 }
 
-size_t line_lds_bytes(int M, int P, bool real_steps) {
-    return ((size_t)line_lds_rows(M, real_steps) * P + kRedScratch) * sizeof(double2) + 64 * sizeof(double);
+size_t line_lds_bytes(int P) {
+    return (3 * (size_t)P + kRedScratch) * sizeof(double2) + 64 * sizeof(double);
 }
 
 template <int M, bool IMAG, int METHOD>
 void launch_line(tdse_ctx* ctx, const Bucket& b, int n_steps, hipStream_t st) {
     hipLaunchKernelGGL((k_line_steps<M, 512, IMAG, METHOD>), dim3((unsigned)b.lines.count), dim3(b.P),
-                       line_lds_bytes(M, b.P, IMAG), st, ctx->d_line, b.lines.ptr, (int)b.lines.count, n_steps);
+                       line_lds_bytes(b.P), st, ctx->d_line, b.lines.ptr, (int)b.lines.count, n_steps);
 }
 
 // b.M == 0: lines of any layouts (k_line_steps_any), b.P the most threads and b.lds the most LDS of any of them
@@ -877,15 +883,15 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)ctx->any_pairs.count), dim3(ctx->any_pair_threads), 0,
                                    ctx->stream, ctx->d_sh, ctx->any_pairs.ptr, (int)ctx->any_pairs.count, ctx->d_cl);
             };
-            const ShObs obs = obs_of(ctx, ctx->jobs, ctx->any_threads, ride);
-            auto solve = [&](auto kernel) {
-                hipLaunchKernelGGL(kernel, dim3((unsigned)(ctx->any_lines.count + obs.blocks)), dim3(ctx->any_threads),
-                                   ctx->any_lds, ctx->stream, ctx->d_sh, ctx->any_lines.ptr,
-                                   (int)ctx->any_lines.count, ctx->d_cl, obs);
+            auto solve = [&](auto kernel, const DevVec<int2>& lines, int threads, size_t lds, bool jobs) {
+                if (!lines.count) return;
+                const ShObs obs = obs_of(ctx, ctx->jobs, threads, jobs);
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(lines.count + obs.blocks)), dim3(threads), lds, ctx->stream,
+                                   ctx->d_sh, lines.ptr, (int)lines.count, ctx->d_cl, obs);
             };
+            solve(k_sh_solve_any<false>, ctx->any_lines, ctx->any_threads, ctx->any_lds, ride);
             vphase(k_sh_vphase_any<false>);
-            if (ctx->any_has_pairs) solve(k_sh_solve_any<true>);
-            else solve(k_sh_solve_any<false>);
+            solve(k_sh_solve_any<true>, ctx->any_vlines, ctx->any_vthreads, ctx->any_vlds, ride && !ctx->any_lines.count);
             vphase(k_sh_vphase_any<true>);
         } else if (ctx->profiling || ctx->sh_buckets.size() < 2) {
             observe(ctx->stream);
@@ -1233,7 +1239,7 @@ int tdse_ctx_destroy(tdse_ctx* ctx) {
     if (ctx->adi_waves.ptr) (void)hipFree(ctx->adi_waves.ptr);
     if (ctx->cyl_jobs.ptr) (void)hipFree(ctx->cyl_jobs.ptr);
     if (ctx->cyl_count_jobs.ptr) (void)hipFree(ctx->cyl_count_jobs.ptr);
-    for (auto* v : {&ctx->adi_jobs, &ctx->any_lines, &ctx->any_pairs, &ctx->any_adi_lines, &ctx->any_adi_groups})
+    for (auto* v : {&ctx->adi_jobs, &ctx->any_lines, &ctx->any_vlines, &ctx->any_pairs, &ctx->any_adi_lines, &ctx->any_adi_groups})
         if (v->ptr) (void)hipFree(v->ptr);
     if (ctx->d_cyl) (void)hipFree(ctx->d_cyl);
     if (ctx->waves.ptr) (void)hipFree(ctx->waves.ptr);
@@ -1650,20 +1656,16 @@ int tdse_cyl_add(tdse_ctx* ctx, const tdse_cyl_desc* desc, const double* zt, con
     H.n_data = n_data_points(S.N, S.store_every);
     const size_t pts = (size_t)S.nrpad * S.npz;
     double2 *g, *oip, *bas = nullptr;
-    double *dzt, *drtab, *dfs, *dts, *part, *on;
-    std::vector<double> rtab(2 * (size_t)S.nrpad, 0.0);  // couplings, then ratios, in the rho-sweep's order
-    double before = 0.0;  // the kernels use the uniform grid and rp of the descriptor, not rt and roff
-    for (int j = 0; j < S.nr; ++j) {
-        const double m = std::min(j + 1, S.nr - 1), o = (m * (1.0 / std::sqrt(m * m - 0.25))) * S.rp;
-        const size_t at = (size_t)(j % Mr) * Cr + j / Mr;
-        rtab[at] = o;
-        rtab[S.nrpad + at] = o != 0.0 ? before / o : 0.0;
-        before = o;
+    double *dzt, *droff, *dfs, *dts, *part, *on;
+    std::vector<double> coupling((size_t)S.nrpad, 0.0);  // in the rho-sweep's order, from the descriptor (not rt and roff)
+    for (int j = 0; j + 1 < S.nr; ++j) {
+        const double m = j + 1;
+        coupling[(size_t)(j % Mr) * Cr + j / Mr] = (m * (1.0 / std::sqrt(m * m - 0.25))) * S.rp;
     }
     int rc = 0;
     if ((rc = copy_to_device(ctx, H.blocks, reinterpret_cast<const double2*>(g0), pts, &g)) ||
         (rc = copy_to_device(ctx, H.blocks, zt, (size_t)S.npz, &dzt)) ||
-        (rc = copy_to_device(ctx, H.blocks, rtab.data(), rtab.size(), &drtab)) ||
+        (rc = copy_to_device(ctx, H.blocks, coupling.data(), coupling.size(), &droff)) ||
         (rc = copy_to_device(ctx, H.blocks, fs, (size_t)S.N, &dfs)) ||
         (rc = copy_to_device(ctx, H.blocks, ts, (size_t)S.N, &dts)) ||
         (rc = copy_to_device<double>(ctx, H.blocks, nullptr, (size_t)S.n_groups * (1 + 2 * S.n_basis), &part)) ||
@@ -1677,7 +1679,7 @@ int tdse_cyl_add(tdse_ctx* ctx, const tdse_cyl_desc* desc, const double* zt, con
     }
     S.g = g;
     S.zt = dzt;
-    S.rtab = drtab;
+    S.roff = droff;
     S.fs = dfs;
     S.ts = dts;
     S.part = part;

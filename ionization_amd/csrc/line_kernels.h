@@ -163,18 +163,12 @@ __device__ __forceinline__ void line_observe(LineSim& S, const double2 (&x)[M], 
     }
 }
 
-// From 10 rows per thread the real-time solve keeps alpha_i in LDS (cn_implicit_lowreg's
-// ALPHA_LDS form): with pass 2 gone the deep tiles no longer spill registers.
-constexpr bool line_alpha_lds(int M) { return M >= 10; }
-// LDS rows of P double2 that the solver uses (the reduction scratch follows them)
-constexpr int line_lds_rows(int M, bool IMAG) { return (IMAG && line_alpha_lds(M)) ? 3 + M - 2 : 3; }
-
 // m == M; the P threads of the line call this together, one line per workgroup.
 // IMAG: every w_n is purely imaginary (real time steps), which halves the
 // coefficient arithmetic; imaginary-time relaxation uses the general path.
 // METHOD: the step of every simulation of the launch (LINE_ADI, LINE_SIO_LEN,
 // LINE_SIO_VEL; the split operator only with IMAG).
-// lds: the solver's line_lds_rows(M, IMAG) * P + kRedScratch double2, then 64 doubles of reduction scratch.
+// lds: the solver's 3 * P + kRedScratch double2, then 64 doubles of reduction scratch.
 template <int M, bool IMAG, int METHOD>
 __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double2* __restrict__ lds) {
     if (!S.active) return;
@@ -183,7 +177,7 @@ __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double
     if (n > N) return;
     const int P = S.P, npad = S.npad;
     const int k = threadIdx.x;
-    double* red = reinterpret_cast<double*>(lds + line_lds_rows(M, IMAG) * P + kRedScratch);
+    double* red = reinterpret_cast<double*>(lds + 3 * P + kRedScratch);
     double2* __restrict__ g = S.g + k;
     const double* __restrict__ H = S.tab + LN_H * npad + k;
     const double* __restrict__ AP = S.tab + LN_AP * npad + k;
@@ -224,28 +218,14 @@ __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double
             asm volatile("" : "+v"(H1), "+v"(zq0), "+v"(dzq));  // and the z coupling per row
             const double so = sw * S.off;
             const int nz = S.n;
-            auto coef = [&](int i, double& hm, double& h, double& hp) {
+            auto coef = [&](int i, double& h, double& o) {
                 const int j = k * M + i;
                 const double zq = (j < nz) ? fma((double)j, dzq, zq0) : 0.0;
                 h = sw * fma(f, zq, ld1(H1, i * P));
-                hm = (j >= 1 && j < nz) ? so : 0.0;
-                hp = (j < nz) ? so : 0.0;  // row nz - 1 too: its neighbour is a zero padding row
+                o = (j + 1 < nz) ? so : 0.0;
             };
-            auto coef2 = [&](int i, double& hm, double& h) {
-                const double* H2 = H;
-                asm volatile("" : "+v"(H2));
-                const int j = k * M + i;
-                const double zq = (j < nz) ? fma((double)j, dzq, zq0) : 0.0;
-                h = sw * fma(f, zq, ld1(H2, i * P));
-                hm = (j >= 1 && j < nz) ? so : 0.0;
-            };
-            // equal off-diagonals: pass 2 reuses the stored pivots (hm / hp = 1 from row 1 to nz - 1)
-            auto ratio = [&](int i) {
-                const int j = k * M + i;
-                return (j >= 1 && j < nz) ? 1.0 : 0.0;
-            };
-            cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, 1, decltype(ratio), line_alpha_lds(M)>(
-                x, k, P, coef, coef2, lds, xl, xr, 0, ratio);
+            auto off = [&](int i) { return (k * M + i + 1 < nz) ? so : 0.0; };
+            cn_symmetric<M, true, 1>(x, k, P, (k > 0 && k * M < nz) ? so : 0.0, coef, off, lds, xl, xr);
             if constexpr (METHOD == LINE_SIO_LEN) line_phase<M>(x, k, sw * fs, S.zq0, S.dzq);
             if constexpr (METHOD == LINE_SIO_VEL) line_vel_pairs<M>(x, k, P, lds, sw * fs * S.vq, nz, true);
         } else {
@@ -295,7 +275,7 @@ __global__ void __launch_bounds__(MAXT) k_line_steps(LineSim* __restrict__ sims,
 // latency of its own chain of steps, so lines of different layouts gain nothing from launches of their
 // own, one after another. The workgroup has the longest line's threads; the whole waves past a line's P leave
 // before any barrier (s_barrier waits for the surviving waves only). 24 lines of 800 to 8192 points, velocity
-// gauge: 108.9 us per step as a launch for each layout, 16.3 with this one.
+// gauge: 108.9 us per step as a launch for each layout, 16.3 with this one (11.7 with cn_symmetric).
 template <int MAXT, bool IMAG, int METHOD>
 __global__ void __launch_bounds__(MAXT) k_line_steps_any(LineSim* __restrict__ sims, const int2* __restrict__ ids,
                                                          int n_ids, int n_steps) {

@@ -492,23 +492,21 @@ __global__ void __launch_bounds__(256) k_sh_observe(ShObs obs) { sh_observe_bloc
 enum { CN_CAYLEY_MEM = 0, CN_CAYLEY_LDS = 1, CN_EXPLICIT = 2 };
 
 // Shared tail of the CN line kernels: x holds the thread's M rows of the line
-// at gl (row i at gl[i * stride]; stride P by default); solves and stores
-// y = (1 + i H~)^-1 (1 - i H~) x. Ratio: optional pass-2 pivot ratios
-// (cn_implicit_lowreg). LANES / ln: LANES lines per workgroup, interleaved in LDS.
+// at gl (row i at gl[i * stride]); solves and stores y = (1 + i H~)^-1 (1 - i H~) x.
+// solve(explicit, xl, xr): the implicit solve of x in place (explicit: std::true_type for EXPLICIT).
+// LANES / ln: LANES lines per workgroup, interleaved in LDS.
 // store = false: the thread solves but writes nothing (rows that are all padding).
-template <int M, int FORM, class Coef, class Coef2, class Ratio = NoRatio, int LANES = 1>
+template <int M, int FORM, int LANES, class Solve>
 __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restrict__ gl, const int k, const int P,
-                                               Coef coef, Coef2 coef2, double2* __restrict__ lds,
-                                               Ratio ratio = Ratio{}, const int ln = 0, const int stride = -1, const bool store = true,
-                                               const bool pcr = true) {
-    const size_t st = stride < 0 ? (size_t)P : (size_t)stride;
+                                               double2* __restrict__ lds, Solve solve, const int ln, const size_t stride,
+                                               const bool store) {
     if constexpr (FORM == CN_EXPLICIT) {
         double2 xl, xr;
         chunk_neighbours<M, LANES>(x, k, P, lds, xl, xr, false, ln);
-        cn_implicit_lowreg<M, Coef, Coef2, true, LANES, Ratio>(x, k, P, coef, coef2, lds, xl, xr, ln, ratio, pcr);
+        solve(std::true_type{}, xl, xr);
         if (store) {
 #pragma unroll
-            for (int i = 0; i < M; ++i) st2s(gl, (size_t)i * st, x[i]);
+            for (int i = 0; i < M; ++i) st2s(gl, (size_t)i * stride, x[i]);
         }
     } else {
         double2* keep = lds + 3 * P * LANES + kRedScratch;  // CN_CAYLEY_LDS: this thread's own rows only
@@ -516,13 +514,12 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 #pragma unroll
             for (int i = 0; i < M; ++i) keep[(i * P + k) * LANES + ln] = x[i];
         }
-        cn_implicit_lowreg<M, Coef, Coef2, false, LANES, Ratio>(x, k, P, coef, coef2, lds, cmk(0.0, 0.0),
-                                                                cmk(0.0, 0.0), ln, ratio, pcr);
+        solve(std::false_type{}, cmk(0.0, 0.0), cmk(0.0, 0.0));
         if (!store) return;
 #pragma unroll
         for (int i = 0; i < M; ++i) {
-            const double2 x0 = (FORM == CN_CAYLEY_LDS) ? keep[(i * P + k) * LANES + ln] : ld2(gl, (size_t)i * st);
-            st2s(gl, (size_t)i * st, cmk(fma(2.0, x[i].x, -x0.x), fma(2.0, x[i].y, -x0.y)));
+            const double2 x0 = (FORM == CN_CAYLEY_LDS) ? keep[(i * P + k) * LANES + ln] : ld2(gl, (size_t)i * stride);
+            st2s(gl, (size_t)i * stride, cmk(fma(2.0, x[i].x, -x0.x), fma(2.0, x[i].y, -x0.y)));
         }
     }
 }
@@ -531,7 +528,7 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 // symmetric tridiagonal: diagonal s_n (T_j + l(l+1) U_j [+ corr0 at l = 0,
 // j = 0]), off-diagonals s_n A_{j-1}, s_n A_j (mesh_operators.py:889-928,
 // 244-269). One workgroup of P threads per line, M (= m) rows per thread,
-// solved by cn_implicit_lowreg, which keeps two complex values per row between
+// solved by cn_symmetric (velocity gauge: cn_implicit_lowreg), which keeps two complex values per row between
 // its passes and re-reads the (L2-resident) coefficient tables instead of
 // holding them, so WPE waves fit per SIMD; that occupancy hides the HBM
 // latency of the line loads. Two algebraically equal forms:
@@ -544,7 +541,9 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 //    from memory at the end (CN_CAYLEY_MEM).
 
 // lds: 3 * P + kRedScratch double2, then M * P for CN_CAYLEY_LDS. n: the step under way.
-template <int M, int FORM>
+// VEL: a velocity-gauge line. A template parameter, not S.vel: with both solvers in one kernel m = 8 spilled 56
+// registers at 4 waves per SIMD and m = 16 kept 326, one wave per SIMD.
+template <int M, int FORM, bool VEL>
 __device__ __forceinline__ void sh_rphase_line(const ShSim& S, const int n, const int l, double2* __restrict__ lds) {
     const int P = S.P, npad = S.npad;
     const int k = threadIdx.x;
@@ -578,32 +577,50 @@ __device__ __forceinline__ void sh_rphase_line(const ShSim& S, const int n, cons
         const double U = (j < nr) ? cu * tdse_rcp(r * r) : 0.0;
         return sn * (fma(ll1, U, T) + (i == 0 ? c0 : 0.0));
     };
-    double carry = a_left;  // A_{j-1} of the next row (pass 1 visits rows in order)
-    auto coef = [&](int i, double& hm, double& h, double& hp) {
-        const double2 tv = ld2(TA, (size_t)i * P);
-        h = diag(i, tv.x, k);
-        hm = sn * carry;
-        hp = sn * tv.y;
-        carry = tv.y;
+    auto general = [&](auto expl, const double2 xl, const double2 xr) {
+        double carry = a_left;  // A_{j-1} of the next row (pass 1 visits rows in order)
+        auto coef = [&](int i, double& hm, double& h, double& hp) {
+            const double2 tv = ld2(TA, (size_t)i * P);
+            h = diag(i, tv.x, k);
+            hm = sn * carry;
+            hp = sn * tv.y;
+            carry = tv.y;
+        };
+        // Second read of the same coefficients (pass 2, rows in order). The empty
+        // asm makes the pointer and the chunk opaque so the compiler reloads (and forms
+        // r_j again) instead of keeping the first pass's values live across the
+        // solver's barriers.
+        double carry2 = a_left;
+        auto coef2 = [&](int i, double& hm, double& h) {
+            const double2* TA2 = TA;
+            int k2 = k;
+            asm volatile("" : "+v"(TA2), "+v"(k2));
+            const double2 tv = ld2(TA2, (size_t)i * P);
+            h = diag(i, tv.x, k2);
+            hm = sn * carry2;
+            carry2 = tv.y;
+        };
+        cn_implicit_lowreg<M, decltype(coef), decltype(coef2), decltype(expl)::value>(x, k, P, coef, coef2, lds, xl, xr);
     };
-    // Second read of the same coefficients (pass 2, rows in order). The empty
-    // asm makes the pointer and the chunk opaque so the compiler reloads (and forms
-    // r_j again) instead of keeping the first pass's values live across the
-    // solver's barriers.
-    double carry2 = a_left;
-    auto coef2 = [&](int i, double& hm, double& h) {
-        const double2* TA2 = TA;
-        int k2 = k;
-        asm volatile("" : "+v"(TA2), "+v"(k2));
-        const double2 tv = ld2(TA2, (size_t)i * P);
-        h = diag(i, tv.x, k2);
-        hm = sn * carry2;
-        carry2 = tv.y;
+    auto symmetric = [&](auto expl, const double2 xl, const double2 xr) {
+        auto coef = [&](int i, double& h, double& o) {
+            const double2 tv = ld2(TA, (size_t)i * P);
+            h = diag(i, tv.x, k);
+            o = sn * tv.y;
+        };
+        const double* AN = S.tab + SH_AN * npad + k;
+        auto off = [&](int i) {
+            const double* A2 = AN;
+            asm volatile("" : "+v"(A2));  // read again, as above
+            return sn * ld1(A2, (size_t)i * P);
+        };
+        cn_symmetric<M, decltype(expl)::value, 1>(x, k, P, sn * a_left, coef, off, lds, xl, xr);
     };
-    cn_line_finish<M, FORM>(x, gl, k, P, coef, coef2, lds, NoRatio{}, 0, -1, !pad, !S.vel);
+    if constexpr (VEL) cn_line_finish<M, FORM, 1>(x, gl, k, P, lds, general, 0, P, !pad);
+    else cn_line_finish<M, FORM, 1>(x, gl, k, P, lds, symmetric, 0, P, !pad);
 }
 
-template <int M, int MAXT, int WPE, int FORM>
+template <int M, int MAXT, int WPE, int FORM, bool VEL>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, ShObs obs) {
     extern __shared__ double2 lds[];
@@ -618,7 +635,7 @@ k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_line
     const ShSim& S = sims[lt.x];
     const int n = S.rstep;
     if (!S.active || n >= S.N) return;  // uniform across the block
-    sh_rphase_line<M, FORM>(S, n, lt.y, lds);
+    sh_rphase_line<M, FORM, VEL>(S, n, lt.y, lds);
 }
 
 // ------------------------------------------------------------------ velocity gauge: h2
@@ -906,8 +923,7 @@ __device__ __forceinline__ void sh_vpair_lines(const ShSim& S, const int n, cons
     };
     double2 xl, xr;
     chunk_neighbours<M, 2>(x, k, P, lds, xl, xr, true, ln);
-    cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, 2, NoRatio, true>(x, k, P, coef, coef2, lds, xl, xr, ln,
-                                                                                     NoRatio{}, false);
+    cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, 2, true>(x, k, P, coef, coef2, lds, xl, xr, ln);
     if (fh != 0.0) sh_vpair_factors<M>(x, k, P, ln, lds, av, fp, true);
     if (pad) return;
 #pragma unroll
@@ -1021,8 +1037,7 @@ __device__ __forceinline__ void sh_adi_r_line(const ShSim& S, const int n, const
             hm = sn * carry2;
             carry2 = tv.y;
         };
-        cn_implicit_lowreg<M, decltype(coef), decltype(coef2), false, 1>(x, k, P, coef, coef2, lds, cmk(0.0, 0.0),
-                                                                         cmk(0.0, 0.0), 0, NoRatio{}, false);
+        cn_implicit_lowreg<M, decltype(coef), decltype(coef2)>(x, k, P, coef, coef2, lds);
         if (sh_adi_ahead(S, n, *ctl)) {  // uniform across the block
             const double* mk = S.tab + (size_t)SH_MASK * npad + k;
             asm volatile("" : "+v"(mk));  // loaded after the solve, not hoisted into it
@@ -1156,7 +1171,7 @@ __device__ __forceinline__ void sh_adi_lp_group(const ShSim& S, const int n, con
     double2 xl, xr;
     chunk_neighbours<M, LANES>(x, c, kAdiChunks, lds, xl, xr, false, ln);
     cn_implicit_lowreg<M, decltype(coef), decltype(coef2), true, LANES>(x, c, kAdiChunks, coef, coef2, lds, xl, xr,
-                                                                        ln, NoRatio{}, false);
+                                                                        ln);
 #pragma unroll
     for (int i = 0; i < M; ++i) {
         const int l = c * M + i;
@@ -1207,9 +1222,9 @@ __device__ __forceinline__ void sh_by_rows(const int m, F&& f) {
     }
 }
 
-// The Crank-Nicolson solves of a split-operator step: single lines and, with PAIRS, velocity-gauge odd l-pairs.
-template <bool PAIRS>
-__global__ void __launch_bounds__(PAIRS ? 2 * kAnyP : kAnyP)
+// The Crank-Nicolson solves of a split-operator step of one gauge: single lines and, with VEL, odd l-pairs.
+template <bool VEL>
+__global__ void __launch_bounds__(VEL ? 2 * kAnyP : kAnyP)
 k_sh_solve_any(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const double* __restrict__ cl,
                ShObs obs) {
     extern __shared__ double2 lds[];
@@ -1223,14 +1238,14 @@ k_sh_solve_any(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_l
     const ShSim& S = sims[lt.x];
     const int n = S.rstep;
     if (!S.active || n >= S.N) return;
-    if (PAIRS && (lt.y & kAnyPair)) {
+    if (VEL && (lt.y & kAnyPair)) {
         if ((int)threadIdx.x >= 2 * S.P) return;
         sh_by_rows(S.m, [&](auto m) { sh_vpair_lines<decltype(m)::value>(S, n, lt.y & (kAnyPair - 1), cl, lds); });
     } else {
         if ((int)threadIdx.x >= S.P) return;
         sh_by_rows(S.m, [&](auto m) {
             constexpr int M = decltype(m)::value;
-            sh_rphase_line<M, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS)>(S, n, lt.y, lds);
+            sh_rphase_line<M, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS), VEL>(S, n, lt.y, lds);
         });
     }
 }
