@@ -171,15 +171,18 @@ int sh_parts(int L) { return (L + kShPartRows - 1) / kShPartRows; }
 // Rows of an L-phase wave's l-segment: the most (up to kShSegRows) that still give the batch
 // kMinLWaves waves, about four for each SIMD. A wave walks its rows one pair after another, so a
 // small batch's L-phase takes as long as one segment: 64-row segments left one 250 x 100 mesh with
-// 8 waves (38.0 us per step, 28 us of it the L-phase; 8-row segments 19.9), one 200 x 1000 mesh with
-// 64 (51.3 -> 30.7). Long segments re-read fewer halo rows (7 per segment); on 32 simulations of
-// 15 M points 8 / 16 / 32 / 64 rows measured 270 / 260 / 267 / 267 us per step.
+// 8 waves (38.0 us per step, 28 us of it the L-phase; 8-row segments 14.2, 4-row segments 12.9), one 200 x 1000 mesh
+// with 64 (51.3 -> 20.8 -> 19.3). Long segments re-read fewer halo rows (7 per segment); on 32 simulations of
+// 15 M points 8 / 16 / 32 / 64 rows measured 270 / 260 / 267 / 267 us per step. Segments of 4 rows walk 11
+// rows where those of 8 walk 15, but twice as many of them: only where 8 rows leave fewer waves than there are
+// SIMDs (1 / 2 / 3 / 4 meshes of 200 x 1000, 400 waves each: 8 rows 19.2 / 21.1 / 22.1 / 24.2 us, 4 rows 18.3 / 20.6 /
+// 22.0 / 29.1).
 // `columns` counts, for every live simulation, its 64-position columns times its partials along l.
-constexpr int64_t kMinLWaves = 4096;
+constexpr int64_t kMinLWaves = 4096, kMinLWaves8 = 1024;
 int sh_segment_rows(int64_t columns) {
     int rows = kShSegRows;
-    while (rows > kShPartRows && columns * kShPartRows / rows < kMinLWaves) rows /= 2;
-    return rows;
+    while (rows > 8 && columns * kShPartRows / rows < kMinLWaves) rows /= 2;
+    return rows == 8 && columns * kShPartRows / 8 < kMinLWaves8 ? kShPartRows : rows;
 }
 
 int n_data_points(int N, int every) {
@@ -1447,11 +1450,11 @@ int tdse_sh_add(tdse_ctx* ctx, const tdse_sh_desc* desc, const double* tables, c
     int* bl = nullptr;
     int rc = 0;
     std::vector<double2> ta_host(npad);  // (T_j, A_j) interleaved for the R-phase
-    for (size_t p = 0; p < npad; ++p) ta_host[p] = make_double2(tables[SH_T * npad + p], tables[SH_AN * npad + p]);
+    for (size_t p = 0; p < npad; ++p) ta_host[p] = make_double2(tables[SH_IN_T * npad + p], tables[SH_IN_AN * npad + p]);
     if ((rc = copy_to_device(ctx, H.blocks, reinterpret_cast<const double2*>(g0), (size_t)S.L * npad, &g)) ||
         (rc = copy_to_device(ctx, H.blocks, ta_host.data(), npad, &ta)) ||
         (rc = copy_to_device<double2>(ctx, H.blocks, nullptr, (size_t)S.L * npad, &g2)) ||
-        (rc = copy_to_device(ctx, H.blocks, tables, (SH_NTAB + (H.vel ? 1 : 0)) * npad, &tab)) ||
+        (rc = copy_to_device(ctx, H.blocks, tables + SH_IN_AN * npad, (SH_NTAB - SH_IN_AN + (H.vel ? 1 : 0)) * npad, &tab)) ||
         // ADI: the L-phase sees a zero field (it only masks and observes); the field goes to fa
         (rc = copy_to_device(ctx, H.blocks, H.adi ? nullptr : fs, (size_t)S.N, &dfs)) ||
         (H.adi && (rc = copy_to_device(ctx, H.blocks, fs, (size_t)S.N, &dfa))) ||

@@ -30,7 +30,7 @@
 struct ShSim {
     double2* g;            // [L][npad] state before even steps (step counter n even)
     double2* g2;           // [L][npad] state before odd steps
-    const double* tab;     // [SH_NTAB][npad] radial tables in position order
+    const double* tab;     // [SH_MASK + 1, or SH_AV + 1 in the velocity gauge][npad] radial tables in position order
     const double* fs;      // [N] field times tau ratio per step: E(t_{n+1}+dt/2) * tau_n / tau0
     const double* ts;      // [N] tau_n / tau0
     double2* snap;         // [LB][npad] rows l < LB captured at data steps
@@ -63,11 +63,13 @@ struct ShSim {
 constexpr int kShSegRows = 64;  // most rows of one L-phase wave (its l-segment)
 // Rows of one norm partial. Segments are whole numbers of these, so the partials, and with them
 // the stored norms, do not depend on how many rows the L-phase gives a wave in a given batch.
-constexpr int kShPartRows = 8;
+constexpr int kShPartRows = 4;
 
-enum { SH_T = 0, SH_U = 1, SH_AP = 2, SH_AN = 3, SH_RQ = 4, SH_MASK = 5, SH_NTAB = 6 };
-// velocity-gauge simulations carry one more row: tau0 hbar q / (2 m dr) alpha_j, zero for j >= n - 1
-enum { SH_AV = 6 };
+// Rows of a simulation's radial tables as the caller gives them, and of those on the device: T is interleaved with AN
+// in `ta`, U and AP are formed from the grid and from AN. AV, velocity gauge only: tau0 hbar q / (2 m dr) alpha_j,
+// zero for j >= n - 1.
+enum { SH_IN_T = 0, SH_IN_AN = 3, SH_NTAB = 6 };
+enum { SH_AN = 0, SH_RQ = 1, SH_MASK = 2, SH_AV = 3 };
 
 // The wavefunction ping-pongs between two buffers: the state with step
 // counter n lives in sh_state(S, n). The L-phase of a step reads

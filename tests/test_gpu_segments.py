@@ -1,7 +1,7 @@
 """
-The L-phase gives a wave as many l-rows as the batch can afford (8 rows in a small batch, up to 64 in a large one).
+The L-phase gives a wave as many l-rows as the batch can afford (4 rows in a small batch, up to 64 in a large one).
 A simulation's wavefunction, norms, largest-l norms, norms by l and inner products must be the same bits either way:
-the same simulation alone (8-row segments) and beside fillers that push the batch to the longest segments.
+the same simulation alone (4-row segments) and beside fillers that push the batch to the longest segments.
 """
 
 import numpy as np
