@@ -456,13 +456,23 @@ def choose_cyl_layout(z_points: int, rho_points: int, z_rows: Optional[int] = No
     (Pz, Mz, Cr, Mr, lanes) for a cylindrical mesh: the z-sweep layout as for an
     SH radial line, and a rho-sweep shape of Cr chunks of Mr rows with `lanes`
     z-lines per workgroup (Cr * lanes a multiple of 64, Cr within the shape's
-    limit); least rho padding first, then the order of CYL_RHO_SHAPES ((8, 4)
-    ahead of (4, 4): a shorter reduced system, 1.02 -> 0.99 ms per rho-sweep of
-    the 32-simulation 2000 x 1000 workload).
+    limit). Up to 320 rho points (4, 4): more workgroups and shorter chains, faster
+    alone and in batches whatever its padding (one / 16 simulations of 400 x 200:
+    15.8 / 42.5 us per step, (8, 4) 18.6 / 43.4, (4, 8) with less padding 17.2 / 43.9;
+    120 x 60: 12.1 / 14.5, 15.7 / 18.1, 13.3 / 14.7). Above, least rho padding, then
+    the order of CYL_RHO_SHAPES ((8, 4) ahead of (4, 4): a shorter reduced system,
+    four simulations of 2000 x 1000 131 us per step against 164; 1024 x 512 alone / 16:
+    27.8 / 119 against 25.8 / 131), without (4, 8): 800 x 400 as 416 rows 25.1 / 125,
+    (4, 4) as 448 rows 22.5 / 112.
     """
     Pz, Mz = choose_layout(z_points, "cylz", z_rows)
     best = None
-    shapes = [tuple(rho_shape)] if rho_shape is not None else list(CYL_RHO_SHAPES)
+    if rho_shape is not None:
+        shapes = [tuple(rho_shape)]
+    elif rho_points <= 320:
+        shapes = [(4, 4)]
+    else:
+        shapes = [shape for shape in CYL_RHO_SHAPES if shape != (4, 8)]
     for pref, (mr, lanes) in enumerate(shapes):
         if (mr, lanes) not in CYL_RHO_SHAPES:
             raise DeviceError(f"unsupported rho-sweep shape {(mr, lanes)}")
