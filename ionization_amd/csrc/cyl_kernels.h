@@ -212,15 +212,16 @@ k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, 
 #pragma unroll
     for (int i = 0; i < M; ++i) x[i] = ld2(gl, (size_t)i * P * 2);
     // coefficients from the grid, no table reads
-    auto off = [&](int i) { return (k * M + i + 1 < nz) ? tzp : 0.0; };
+    auto off = [&](int) { return tzp; };
     auto coef = [&](int i, double& h, double& o) {
-        const int j = k * M + i;
-        const double z = fma((double)j, dz, z0);
-        h = j < nz ? fma(tau, cyl_half_potential(S, z, rho, E), tdiag) : 0.0;
-        o = off(i);
+        const double z = fma((double)(k * M + i), dz, z0);
+        h = fma(tau, cyl_half_potential(S, z, rho, E), tdiag);
+        o = tzp;
     };
+    const int rows = nz - k * M;  // of this chunk that are no padding
+    auto live = [&](int i) { return i < rows; };
     auto solve = [&](auto expl, const double2 xl, const double2 xr) {
-        cn_symmetric<M, decltype(expl)::value, 2>(x, k, P, (k > 0 && k * M < nz) ? tzp : 0.0, coef, off, lds, xl, xr, ln);
+        cn_symmetric<M, decltype(expl)::value, 2>(x, k, P, k > 0 ? tzp : 0.0, coef, off, lds, xl, xr, ln, live);
     };
     cn_line_finish<M, FORM, 2>(x, gl, k, P, lds, solve, ln, 2 * P, true);
 }

@@ -218,14 +218,18 @@ __device__ __forceinline__ void line_steps(LineSim& S, const int n_steps, double
             asm volatile("" : "+v"(H1), "+v"(zq0), "+v"(dzq));  // and the z coupling per row
             const double so = sw * S.off;
             const int nz = S.n;
+            const double j0 = (double)(k * M);
             auto coef = [&](int i, double& h, double& o) {
-                const int j = k * M + i;
-                const double zq = (j < nz) ? fma((double)j, dzq, zq0) : 0.0;
-                h = sw * fma(f, zq, ld1(H1, i * P));
-                o = (j + 1 < nz) ? so : 0.0;
+                // z per row from the grid: stepped along the thread's rows, sw f zq + i (sw f dzq) is one
+                // operation shorter, but its rounding is the same at every step and adds up (2e-12 after 4000 steps)
+                const double Hi = ld1(H1, i * P);
+                h = sw * (METHOD == LINE_ADI ? fma(f, fma(j0 + (double)i, dzq, zq0), Hi) : Hi);
+                o = so;
             };
-            auto off = [&](int i) { return (k * M + i + 1 < nz) ? so : 0.0; };
-            cn_symmetric<M, true, 1>(x, k, P, (k > 0 && k * M < nz) ? so : 0.0, coef, off, lds, xl, xr);
+            auto off = [&](int) { return so; };
+            const int rows = nz - k * M;  // of this chunk that are no padding
+            auto live = [&](int i) { return i < rows; };
+            cn_symmetric<M, true, 1>(x, k, P, k > 0 ? so : 0.0, coef, off, lds, xl, xr, 0, live);
             if constexpr (METHOD == LINE_SIO_LEN) line_phase<M>(x, k, sw * fs, S.zq0, S.dzq);
             if constexpr (METHOD == LINE_SIO_VEL) line_vel_pairs<M>(x, k, P, lds, sw * fs * S.vq, nz, true);
         } else {
@@ -275,7 +279,7 @@ __global__ void __launch_bounds__(MAXT) k_line_steps(LineSim* __restrict__ sims,
 // latency of its own chain of steps, so lines of different layouts gain nothing from launches of their
 // own, one after another. The workgroup has the longest line's threads; the whole waves past a line's P leave
 // before any barrier (s_barrier waits for the surviving waves only). 24 lines of 800 to 8192 points, velocity
-// gauge: 108.9 us per step as a launch for each layout, 16.3 with this one (11.7 with cn_symmetric).
+// gauge: 108.9 us per step as a launch for each layout, 16.3 with this one (10.7 with cn_symmetric).
 template <int MAXT, bool IMAG, int METHOD>
 __global__ void __launch_bounds__(MAXT) k_line_steps_any(LineSim* __restrict__ sims, const int2* __restrict__ ids,
                                                          int n_ids, int n_steps) {

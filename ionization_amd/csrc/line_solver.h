@@ -499,12 +499,26 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
 //
 // coef(i, h, o): row i's diagonal h_i and its coupling o_i to row i + 1, rows in order; off(i): o_i again in
 // passes 2 and 3 (in order forwards, then backwards; to be read again, not held across the reduced solve);
-// o_left: the coupling of row 0 to the previous chunk's last row. Couplings past the line's last row are 0.
+// o_left: the coupling of row 0 to the previous chunk's last row. Couplings past the line's last row are 0, or,
+// with live(i) (row i is no padding), anything: a padding row's r_i is made 0, and with it all that could pass through
+// the row, its own z_i included. One selection per row instead of one for each use of o_i and for h_i (an 8192-point
+// line 8.9 -> 8.1 us per step, 24 lines 11.7 -> 10.7). Padding rows hold zeros.
 // EXPLICIT, xl, xr, LANES, ln: as for cn_implicit_lowreg. lds: 3 P LANES + kRedScratch double2.
-template <int M, bool EXPLICIT, int LANES, class Coef, class Off>
+struct AllLive {};
+
+template <int M, bool EXPLICIT, int LANES, class Coef, class Off, class Live = AllLive>
 __device__ __forceinline__ void cn_symmetric(double2 (&x)[M], const int k, const int P, const double o_left, Coef coef,
                                              Off off, double2* __restrict__ lds, const double2 xl, const double2 xr,
-                                             const int ln = 0) {
+                                             const int ln = 0, Live live = Live{}) {
+    constexpr bool kSelect = !std::is_same_v<Live, AllLive>;
+    auto pivot = [&](int i, const double2 den) {
+        if constexpr (kSelect) {
+            const double inv = live(i) ? tdse_rcp(cabs2(den)) : 0.0;
+            return cmk(den.x * inv, -den.y * inv);
+        } else {
+            return crecip(den);
+        }
+    };
     double2 r[M - 1], u[M - 1];
     double2 p = cmk(1.0, 0.0), q = p, sa = p, sd = p, flast = p;
     double ob = o_left, hlast = 0.0, olast = 0.0;  // ob: o_{i-1}
@@ -512,6 +526,9 @@ __device__ __forceinline__ void cn_symmetric(double2 (&x)[M], const int k, const
     for (int i = 0; i < M; ++i) {
         double h, o;
         coef(i, h, o);
+        if constexpr (kSelect) {
+            if (i == M - 1) ob = live(i) ? ob : 0.0;  // the last row has no r_i
+        }
         double2 f = x[i];
         if constexpr (EXPLICIT) {
             // (1 - i H) x on row i: x_i - i (o_{i-1} x_{i-1} + h x_i + o_i x_{i+1})
@@ -521,7 +538,7 @@ __device__ __forceinline__ void cn_symmetric(double2 (&x)[M], const int k, const
         }
         if (i < M - 1) {
             if (i == 0) {
-                r[0] = crecip(cmk(1.0, h));
+                r[0] = pivot(0, cmk(1.0, h));
                 q = r[0];
                 u[0] = cmul(q, f);
                 sa = q;
@@ -529,7 +546,7 @@ __device__ __forceinline__ void cn_symmetric(double2 (&x)[M], const int k, const
             } else {
                 const double2 rb = r[i > 0 ? i - 1 : 0], ub = u[i > 0 ? i - 1 : 0];
                 const double c = ob * ob;
-                const double2 ri = crecip(cmk(fma(c, rb.x, 1.0), fma(c, rb.y, h)));
+                const double2 ri = pivot(i, cmk(fma(c, rb.x, 1.0), fma(c, rb.y, h)));
                 const double2 ui = cmul(ri, cmk(fma(ob, ub.y, f.x), fma(-ob, ub.x, f.y)));
                 q = cmul(ri, p);
                 sa = cmla(sa, p, q);
