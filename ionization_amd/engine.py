@@ -109,19 +109,6 @@ def choose_layout(n: int, kind: str = "sh", rows: Optional[int] = None) -> Tuple
     return best[1], best[2]
 
 
-def choose_sh_layout(n: int, gauge: str, method: str, rows: Optional[int] = None) -> Tuple[int, int]:
-    """
-    choose_layout of an SH simulation's radial lines. In the length gauge's split operator, where the rule takes 16 rows
-    per thread and at most 128 threads, the same padding with 8 rows and twice the threads: the symmetric solver's
-    shorter chains win where a line is one or two waves (1000 points: 16.4 -> 15.3 us per step alone, 52.1 -> 49.4 for
-    24 simulations; 2000: 18.1 -> 17.3, 82.2 -> 80.8; 4000 points as 512 x 8: 145.7 -> 158.2).
-    """
-    P, m = choose_layout(n, "sh", rows)
-    if (gauge, method, m) == ("length", "sio", 16) and P <= 128 and rows is None and sh_size_class(n) not in _SH_TUNED:
-        return 2 * P, 8
-    return P, m
-
-
 def position_index(n: int, P: int, m: int) -> np.ndarray:
     """j for every position p (j >= n marks padding)."""
     p = np.arange(P * m)
@@ -315,7 +302,7 @@ def compile_sh(*, r_bound, r_points, l_bound, potential, field: Callable, mask, 
         P, m = int(layout[0]), int(layout[1])
         check_layout(r_points, P, m, "sh")
     else:
-        P, m = choose_sh_layout(r_points, gauge, method, rows)
+        P, m = choose_layout(r_points, "sh", rows)
     tables, corr0, delta_r, _, centrifugal = sh_radial_tables(
         r_bound=r_bound, r_points=r_points, potential=potential, mask=mask, time_step=time_step,
         test_charge=test_charge, hydrogen_correction=hydrogen_correction, P=P, m=m,
@@ -354,7 +341,7 @@ def compile_sh(*, r_bound, r_points, l_bound, potential, field: Callable, mask, 
 def relayout_sh(c: CompiledSH, layout: Optional[Tuple[int, int]] = None) -> CompiledSH:
     """The same simulation under another device layout (the tuned or rule one when None):
     position-ordered arrays are permuted, nothing is recomputed."""
-    P, m = layout if layout is not None else choose_sh_layout(c.r_points, c.gauge, c.method)
+    P, m = layout if layout is not None else choose_layout(c.r_points, "sh")
     check_layout(c.r_points, P, m, "sh")
     if (P, m) == (c.P, c.m):
         return c
