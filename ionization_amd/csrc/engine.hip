@@ -146,7 +146,6 @@ struct Bucket {
     int M = 0;  // exact rows per chunk-thread
     int P = 0;
     bool imag = false;  // Line: complex time steps (imaginary-time relaxation)
-    bool vel = false;   // SH: velocity gauge
     int method = 0;     // Line: LINE_ADI, LINE_SIO_LEN or LINE_SIO_VEL
     size_t lds = 0;     // Line, M == 0 (any layouts): dynamic LDS of the launch
     int Mr = 0, Cr = 0, lanes = 1;  // cylindrical rho-sweep: rows per thread, chunks, lines per workgroup
@@ -171,8 +170,8 @@ int sh_parts(int L) { return (L + kShPartRows - 1) / kShPartRows; }
 // Rows of an L-phase wave's l-segment: the most (up to kShSegRows) that still give the batch
 // kMinLWaves waves, about four for each SIMD. A wave walks its rows one pair after another, so a
 // small batch's L-phase takes as long as one segment: 64-row segments left one 250 x 100 mesh with
-// 8 waves (38.0 us per step, 28 us of it the L-phase; 8-row segments 14.2, 4-row segments 12.9), one 200 x 1000 mesh
-// with 64 (51.3 -> 20.8 -> 19.3). Long segments re-read fewer halo rows (7 per segment); on 32 simulations of
+// 8 waves (38.0 us per step, 28 us of it the L-phase; 8-row segments 15.6, 4-row segments 14.3), one 200 x 1000 mesh
+// with 64 (51.3 -> 23.3 -> 21.8). Long segments re-read fewer halo rows (7 per segment); on 32 simulations of
 // 15 M points 8 / 16 / 32 / 64 rows measured 270 / 260 / 267 / 267 us per step. Segments of 4 rows walk 11
 // rows where those of 8 walk 15, but twice as many of them: only where 8 rows leave fewer waves than there are
 // SIMDs (1 / 2 / 3 / 4 meshes of 200 x 1000, 400 waves each: 8 rows 19.2 / 21.1 / 22.1 / 24.2 us, 4 rows 18.3 / 20.6 /
@@ -223,10 +222,10 @@ struct tdse_ctx {
     hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
     // every layout in one launch for each sweep (any_layouts): the buckets' lines, longest first
     bool any_sh = false, any_adi = false;
-    // (any_lines: length gauge; any_vlines: velocity gauge, its odd l-pairs marked kAnyPair; any_pairs: its even ones)
-    DevVec<int2> any_lines, any_vlines, any_pairs, any_adi_lines, any_adi_groups;
-    int any_threads = 0, any_vthreads = 0, any_pair_threads = 0, any_adi_threads = 0;
-    size_t any_lds = 0, any_vlds = 0, any_adi_lds = 0;
+    DevVec<int2> any_lines, any_pairs, any_adi_lines, any_adi_groups;
+    int any_threads = 0, any_pair_threads = 0, any_adi_threads = 0;
+    size_t any_lds = 0, any_adi_lds = 0;
+    bool any_has_pairs = false;  // some entries of any_lines are velocity odd l-pairs
     std::vector<Bucket> line_buckets;
     bool dirty = true;
     bool sh_norm_by_l = false;   // some live SH simulation reduces the norm in every l (L-phase instance)
@@ -297,8 +296,8 @@ size_t adi_lds_bytes(int P);
 // Whether the layouts of a set of lines share one launch per sweep: more than one of them, none past kAnyP threads,
 // and a batch small enough that the launches and their forks and joins cost more than the deepest tile's
 // occupancy does. Measured (us per step, one launch / a launch for each layout): 32 length-gauge simulations of 15 M
-// points 228 / 239, the 256 of 111 M 1689 / 1579; velocity gauge 4.7 M 194 / 275, 111 M 4334 / 3500; ADI 4.2 M
-// 104 / 143, 111 M 2441 / 2024. Between them the gain falls linearly with the points: the lines below are near zero.
+// points 228 / 239, the 256 of 111 M 1689 / 1579; velocity gauge 4.7 M 194 / 275, 111 M 4334 / 3500;
+// ADI 4.2 M 109 / 143, 111 M 2441 / 2024. Between them the gain falls linearly with the points: the lines below are near zero.
 using Layouts = std::map<std::pair<int, int>, std::vector<int2>>;  // (rows, chunks) -> lines
 constexpr int64_t kAnyPoints = int64_t(24) << 20;       // single lines only
 constexpr int64_t kAnyPointsMore = int64_t(12) << 20;   // with velocity-gauge pairs, or ADI's three sweeps
@@ -306,9 +305,8 @@ bool any_layouts(const Layouts& lines, const Layouts& pairs, int64_t limit) {
     int64_t points = 0;
     for (const Layouts* m : {&lines, &pairs})
         for (auto& kv : *m) {
-            const int P = kv.first.second % 4096;
-            if (P > kAnyP) return false;
-            points += (int64_t)kv.second.size() * kv.first.first * P;
+            if (kv.first.second > kAnyP) return false;
+            points += (int64_t)kv.second.size() * kv.first.first * kv.first.second;
         }
     return lines.size() + pairs.size() > 1 && points <= limit;
 }
@@ -316,34 +314,32 @@ bool any_layouts(const Layouts& lines, const Layouts& pairs, int64_t limit) {
 // The single-launch tables of the split-operator and ADI simulations (longest lines first).
 int build_any(tdse_ctx* ctx, const Layouts& lines, const Layouts (&vpairs)[2], const Layouts& fpairs,
               const Layouts& adi, const Layouts& adi_groups) {
-    std::vector<int2> solve, vsolve, pairs, al, ag;
+    std::vector<int2> solve, pairs, al, ag;
     int rc;
     // pairs count half their points (one entry for two rows)
     ctx->any_sh = any_layouts(lines, fpairs, fpairs.empty() ? kAnyPoints : kAnyPointsMore / 2);
     ctx->any_adi = any_layouts(adi, adi_groups, kAnyPointsMore) && ctx->adi_waves.count == 0;
-    ctx->any_threads = ctx->any_vthreads = ctx->any_pair_threads = ctx->any_adi_threads = 0;
-    ctx->any_lds = ctx->any_vlds = ctx->any_adi_lds = 0;
+    ctx->any_threads = ctx->any_pair_threads = ctx->any_adi_threads = 0;
+    ctx->any_lds = ctx->any_adi_lds = 0;
+    ctx->any_has_pairs = false;
     if (ctx->any_sh) {
         for (auto it = fpairs.rbegin(); it != fpairs.rend(); ++it) {
-            const int M = it->first.first, P = it->first.second % 4096;
-            for (const int2& e : it->second) vsolve.push_back(make_int2(e.x, e.y | kAnyPair));
-            ctx->any_vthreads = std::max(ctx->any_vthreads, 2 * P);
-            ctx->any_vlds = std::max(ctx->any_vlds, vpair_lds_bytes(M, P));
+            const int M = it->first.first, P = it->first.second;
+            for (const int2& e : it->second) solve.push_back(make_int2(e.x, e.y | kAnyPair));
+            ctx->any_has_pairs = true;
+            ctx->any_threads = std::max(ctx->any_threads, 2 * P);
+            ctx->any_lds = std::max(ctx->any_lds, vpair_lds_bytes(M, P));
         }
         for (auto it = lines.rbegin(); it != lines.rend(); ++it) {
-            const int M = it->first.first, P = it->first.second % 4096;
-            const bool vel = it->first.second >= 4096;
-            auto& list = vel ? vsolve : solve;
-            list.insert(list.end(), it->second.begin(), it->second.end());
-            int& threads = vel ? ctx->any_vthreads : ctx->any_threads;
-            size_t& lds = vel ? ctx->any_vlds : ctx->any_lds;
-            threads = std::max(threads, P);
-            lds = std::max(lds, cn_lds_bytes(M, P, cn_form(M, P)));
+            const int M = it->first.first, P = it->first.second;
+            solve.insert(solve.end(), it->second.begin(), it->second.end());
+            ctx->any_threads = std::max(ctx->any_threads, P);
+            ctx->any_lds = std::max(ctx->any_lds, cn_lds_bytes(M, P, cn_form(M, P)));
         }
         // up to kAnyP threads the odd l-pairs are solved with the lines: only the even ones are left
         for (auto it = vpairs[0].rbegin(); it != vpairs[0].rend(); ++it) {
             pairs.insert(pairs.end(), it->second.begin(), it->second.end());
-            ctx->any_pair_threads = std::max(ctx->any_pair_threads, sh_vel_split(it->first.first) * (it->first.second % 4096));
+            ctx->any_pair_threads = std::max(ctx->any_pair_threads, sh_vel_split(it->first.first) * it->first.second);
         }
     }
     if (ctx->any_adi) {
@@ -355,8 +351,7 @@ int build_any(tdse_ctx* ctx, const Layouts& lines, const Layouts (&vpairs)[2], c
         for (auto it = adi_groups.rbegin(); it != adi_groups.rend(); ++it)
             ag.insert(ag.end(), it->second.begin(), it->second.end());
     }
-    if ((rc = devvec_upload(ctx, ctx->any_lines, solve)) || (rc = devvec_upload(ctx, ctx->any_vlines, vsolve)) ||
-        (rc = devvec_upload(ctx, ctx->any_pairs, pairs)) ||
+    if ((rc = devvec_upload(ctx, ctx->any_lines, solve)) || (rc = devvec_upload(ctx, ctx->any_pairs, pairs)) ||
         (rc = devvec_upload(ctx, ctx->any_adi_lines, al)) || (rc = devvec_upload(ctx, ctx->any_adi_groups, ag)))
         return rc;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // the host vectors end here
@@ -368,7 +363,7 @@ int rebuild_tables(tdse_ctx* ctx) {
     std::vector<ShWave> waves;
     std::vector<int2> jobs, ajobs;
     ctx->n_len_waves = -1;
-    std::map<std::pair<int, int>, std::vector<int2>> shb, lnb;  // (rows, chunks [+ 4096 if velocity gauge / complex steps])
+    std::map<std::pair<int, int>, std::vector<int2>> shb, lnb;  // (rows, chunks [+ 4096 if complex steps])
     std::map<std::pair<bool, int>, std::vector<int>> lna;       // lines of any layout, (complex steps, method)
     std::map<std::pair<int, int>, std::vector<int2>> vpb[2];    // velocity l-pairs by parity, (rows, chunks)
     std::map<std::pair<int, int>, std::vector<int2>> fpb;       // velocity odd l-pairs solved in one workgroup
@@ -413,8 +408,7 @@ int rebuild_tables(tdse_ctx* ctx) {
             }
             continue;
         }
-        const std::pair<int, int> layout{h.dev.m, h.dev.P + (h.vel ? 4096 : 0)};
-        auto& v = shb[layout];
+        auto& v = shb[{h.dev.m, h.dev.P}];
         // velocity gauge: where two lines fit one workgroup (2 P <= 512) the odd l-pairs are
         // solved together with their h2 factors; the rows outside them stay single lines
         const bool fuse = h.vel && 2 * h.dev.P <= kMaxPairThreads;
@@ -424,8 +418,8 @@ int rebuild_tables(tdse_ctx* ctx) {
         }
         if (h.vel)
             for (int l = 0; l + 1 < h.dev.L; ++l) {
-                if (fuse && (l & 1)) fpb[layout].push_back(make_int2(s, l));
-                else vpb[l & 1][layout].push_back(make_int2(s, l));
+                if (fuse && (l & 1)) fpb[{h.dev.m, h.dev.P}].push_back(make_int2(s, l));
+                else vpb[l & 1][{h.dev.m, h.dev.P}].push_back(make_int2(s, l));
             }
     }
     if (ctx->n_len_waves < 0) ctx->n_len_waves = (int)waves.size();
@@ -466,7 +460,7 @@ int rebuild_tables(tdse_ctx* ctx) {
             Bucket b;
             b.M = kv.first.first;
             b.P = kv.first.second % 4096;
-            b.imag = b.vel = (kv.first.second % 8192) >= 4096;
+            b.imag = (kv.first.second % 8192) >= 4096;
             b.method = kv.first.second / 8192;
             int r = devvec_upload(ctx, b.lines, kv.second);
             if (r) return r;
@@ -480,13 +474,11 @@ int rebuild_tables(tdse_ctx* ctx) {
     if ((rc = fill(ctx->sh_adi_lbuckets, alb))) return rc;
     if ((rc = devvec_upload(ctx, ctx->adi_waves, adw))) return rc;
     for (auto& b : ctx->sh_buckets) {
-        if (!b.vel) continue;
-        const std::pair<int, int> layout{b.M, b.P + 4096};
         for (int par = 0; par < 2; ++par) {
-            auto it = vpb[par].find(layout);
+            auto it = vpb[par].find({b.M, b.P});
             if (it != vpb[par].end() && (rc = devvec_upload(ctx, b.vpairs[par], it->second))) return rc;
         }
-        auto it = fpb.find(layout);
+        auto it = fpb.find({b.M, b.P});
         if (it != fpb.end() && (rc = devvec_upload(ctx, b.fpairs, it->second))) return rc;
     }
     if ((rc = build_any(ctx, shb, vpb, fpb, adb, alb))) return rc;
@@ -589,13 +581,15 @@ void launch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
     const size_t lds = cn_lds_bytes(M, b.P, form);
     const ShObs obs = obs_of(ctx, ctx->jobs, b.P, ride);
     const dim3 grid((unsigned)(b.lines.count + obs.blocks)), block(b.P);
-    auto launch = [&](auto length, auto velocity) {
-        hipLaunchKernelGGL(b.vel ? velocity : length, grid, block, lds, st, ctx->d_sh, b.lines.ptr, (int)b.lines.count,
-                           obs);
-    };
-    constexpr int kMem = M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM, kLds = M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS;
-    if (form == CN_CAYLEY_LDS) launch(k_sh_rphase<M, MAXT, WPE, kLds, false>, k_sh_rphase<M, MAXT, WPE, kLds, true>);
-    else launch(k_sh_rphase<M, MAXT, WPE, kMem, false>, k_sh_rphase<M, MAXT, WPE, kMem, true>);
+    if (form == CN_EXPLICIT)
+        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
+                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
+    else if (form == CN_CAYLEY_LDS)
+        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS)>), grid, block, lds,
+                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
+    else
+        hipLaunchKernelGGL((k_sh_rphase<M, MAXT, WPE, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_MEM)>), grid, block, lds,
+                           st, ctx->d_sh, b.lines.ptr, (int)b.lines.count, obs);
 }
 
 void dispatch_rphase(tdse_ctx* ctx, const Bucket& b, hipStream_t st, bool ride) {
@@ -886,15 +880,15 @@ int launch_step(tdse_ctx* ctx, bool cyl_pre) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)ctx->any_pairs.count), dim3(ctx->any_pair_threads), 0,
                                    ctx->stream, ctx->d_sh, ctx->any_pairs.ptr, (int)ctx->any_pairs.count, ctx->d_cl);
             };
-            auto solve = [&](auto kernel, const DevVec<int2>& lines, int threads, size_t lds, bool jobs) {
-                if (!lines.count) return;
-                const ShObs obs = obs_of(ctx, ctx->jobs, threads, jobs);
-                hipLaunchKernelGGL(kernel, dim3((unsigned)(lines.count + obs.blocks)), dim3(threads), lds, ctx->stream,
-                                   ctx->d_sh, lines.ptr, (int)lines.count, ctx->d_cl, obs);
+            const ShObs obs = obs_of(ctx, ctx->jobs, ctx->any_threads, ride);
+            auto solve = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(ctx->any_lines.count + obs.blocks)), dim3(ctx->any_threads),
+                                   ctx->any_lds, ctx->stream, ctx->d_sh, ctx->any_lines.ptr,
+                                   (int)ctx->any_lines.count, ctx->d_cl, obs);
             };
-            solve(k_sh_solve_any<false>, ctx->any_lines, ctx->any_threads, ctx->any_lds, ride);
             vphase(k_sh_vphase_any<false>);
-            solve(k_sh_solve_any<true>, ctx->any_vlines, ctx->any_vthreads, ctx->any_vlds, ride && !ctx->any_lines.count);
+            if (ctx->any_has_pairs) solve(k_sh_solve_any<true>);
+            else solve(k_sh_solve_any<false>);
             vphase(k_sh_vphase_any<true>);
         } else if (ctx->profiling || ctx->sh_buckets.size() < 2) {
             observe(ctx->stream);
@@ -1242,7 +1236,7 @@ int tdse_ctx_destroy(tdse_ctx* ctx) {
     if (ctx->adi_waves.ptr) (void)hipFree(ctx->adi_waves.ptr);
     if (ctx->cyl_jobs.ptr) (void)hipFree(ctx->cyl_jobs.ptr);
     if (ctx->cyl_count_jobs.ptr) (void)hipFree(ctx->cyl_count_jobs.ptr);
-    for (auto* v : {&ctx->adi_jobs, &ctx->any_lines, &ctx->any_vlines, &ctx->any_pairs, &ctx->any_adi_lines, &ctx->any_adi_groups})
+    for (auto* v : {&ctx->adi_jobs, &ctx->any_lines, &ctx->any_pairs, &ctx->any_adi_lines, &ctx->any_adi_groups})
         if (v->ptr) (void)hipFree(v->ptr);
     if (ctx->d_cyl) (void)hipFree(ctx->d_cyl);
     if (ctx->waves.ptr) (void)hipFree(ctx->waves.ptr);

@@ -48,13 +48,12 @@ __device__ __forceinline__ double2 wmul(double2 w, double2 v) {
 //  * pcr: parallel cyclic reduction, log2 levels in which every lane updates its own
 //    equation, where cyclic reduction takes as many levels up and again down at the same
 //    issue cost (a wave's instruction costs the same with one lane active);
-//  * otherwise cyclic reduction, the same products as the block-wide levels form. The
-//    velocity gauge and the l-sweep of ADI add and subtract rows of very different size,
-//    so their smallest rows carry the rounding of their largest: there the bits of a solve
-//    show in stored values (the norm in the largest l) that a change in rounding would move.
+//  * otherwise cyclic reduction, the same products as the block-wide levels form. SH
+//    simulations mix rows of very different size, and what a pulse leaves in the largest l is
+//    the rounding of amplitudes that cancel: there the bits of a solve show in a stored value
+//    (the norm in the largest l), which any change in rounding would move.
 // Against cyclic reduction behind block barriers throughout, us per step: one 8192-point
-// line (P = 512) 12.2 -> 10.5, 250 x 100 SH (P = 64) 17.2 -> 16.1, 250 x 100 cylinder
-// 20.2 -> 18.4 (pcr); R-phase of the 256-simulation scan 0.98 -> 0.92 ms (serial).
+// line (P = 512) 12.2 -> 10.5, 250 x 100 cylinder 20.2 -> 18.4 (pcr).
 //
 // LANES > 1: LANES independent lines share the block, thread k LANES + ln on equation
 // k of line ln, which sits at LDS index k * LANES + ln (each array of 3 holds P * LANES
@@ -480,8 +479,7 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
     }
 }
 
-// Implicit solve (1 + i H) z = x for real symmetric H, the solver of every line but those whose results
-// are rounding noise and have to stay as they are (velocity gauge, AlternatingDirectionImplicit:
+// Implicit solve (1 + i H) z = x for real symmetric H: Line and the cylinder (the SH meshes keep
 // cn_implicit_lowreg). Symmetry leaves one real coupling o_i = H_{i,i+1} per row, and per row the solver keeps the
 // reciprocal pivot r_i and the eliminated right-hand side u_i (4 doubles):
 //
@@ -493,9 +491,9 @@ __device__ __forceinline__ void cn_implicit_lowreg(double2 (&x)[M], const int k,
 //  pass 3 (backward): z_{m-1} = Y_k, z_i = u_i - r_i (i o_i z_{i+1}).
 // Every real factor (i o) stays apart from the complex ones, pass 2 needs neither the pivots' reciprocals nor the
 // diagonal again, and sums are fused (cmla): about 62 FP64 operations per row where the general form
-// takes 92. Per step, general -> this: an 8192-point line 10.5 -> 8.9 us, 24 velocity-gauge lines 15.6 -> 11.7, the
-// R-phases of 32 SH simulations of 13.2 M points 118 -> 109, a 250 x 100 cylinder 16.2 -> 16.0, four of 2000 x 1000
-// 137 -> 133, 256 SH simulations of 111 M points 1.549 -> 1.483 ms (whole step).
+// takes 92. Per step, general -> this: an 8192-point line 10.5 -> 8.9 us, 24 velocity-gauge lines 15.6 -> 11.7,
+// a 250 x 100 cylinder 16.2 -> 16.0, four of 2000 x 1000
+// 137 -> 133. The SH lines would gain too (256 simulations 1.55 -> 1.48 ms per step), but keep their bits (reduced_cr).
 //
 // coef(i, h, o): row i's diagonal h_i and its coupling o_i to row i + 1, rows in order; off(i): o_i again in
 // passes 2 and 3 (in order forwards, then backwards; to be read again, not held across the reduced solve);

@@ -140,52 +140,6 @@ __device__ __forceinline__ void sh_rotate(double a, double2& x0, double2& x1) {
     sh_turn<VEL>(s, c, x0, x1);
 }
 
-// The angles of one half step at a lane's radial position: theta times the coupling of the pair.
-//
-// Length gauge: the coupling c_l = (l + 1) / sqrt((2 l + 1)(2 l + 3)) lies just above 1/2 (0.577 at
-// l = 0, 1/2 + 1/(16 (l + 1)^2) far out), so the sine and cosine of theta / 2 are taken once per wave and
-// each pair adds delta = theta (c_l - 1/2) to that angle by its addition theorem. Where |delta| <= 1/256 the
-// series of delta end at delta^5 and delta^4 (the first omitted terms are below 6e-18): 11 operations and no
-// branch on the lanes' angles against 14 (|a| <= 1/8) or 45 and two tests for a sine and cosine of its own.
-// From l + 1 >= sqrt(256 |theta| / 12) on that holds (c_l - 1/2 <= 1 / (12 (l + 1)^2)): sh_short_rows.
-template <bool VEL>
-struct ShAngle {
-    double theta, half, s0, c0;
-    __device__ __forceinline__ explicit ShAngle(double th) : theta(th), half(0.5 * th), s0(0.0), c0(1.0) {
-        if constexpr (!VEL) {
-            if (__all(fabs(half) <= kSmallAngle)) tdse_sincos_small(half, &s0, &c0);
-            else tdse_sincos(half, &s0, &c0);
-        }
-    }
-    // the sum of two angles
-    __device__ __forceinline__ ShAngle(const ShAngle& a, const ShAngle& b)
-        : theta(a.theta + b.theta), half(0.5 * theta), s0(fma(a.s0, b.c0, a.c0 * b.s0)),
-          c0(fma(a.c0, b.c0, -(a.s0 * b.s0))) {}
-    // c: the pair's coupling, uniform (0 where there is no such pair: the identity); is_short: its row is past
-    // sh_short_rows and the pair exists
-    __device__ __forceinline__ void rotate(double c, bool is_short, double2& x0, double2& x1) const {
-        if (!VEL && is_short) {
-            const double d = fma(theta, c, -half);
-            const double d2 = d * d;
-            const double sd = fma(fma(d2, 0.008333333333333333, -0.16666666666666666) * d2, d, d);
-            const double cd = fma(fma(d2, 0.041666666666666664, -0.5), d2, 1.0);
-            sh_turn<VEL>(fma(s0, cd, c0 * sd), fma(c0, cd, -(s0 * sd)), x0, x1);
-        } else {
-            sh_rotate<VEL>(theta * c, x0, x1);
-        }
-    }
-};
-
-// First row l whose pairs may take the short form in every lane of the wave.
-template <bool VEL>
-__device__ __forceinline__ int sh_short_rows(const ShAngle<VEL>& a, const ShAngle<VEL>& b, const ShAngle<VEL>& c) {
-    if constexpr (VEL) return 0;
-    const double most = fmax(fabs(a.theta), fmax(fabs(b.theta), fabs(c.theta)));
-    // rounded up generously; a huge or non-finite angle never takes the short form
-    int rows = most <= 1e6 ? (int)(sqrtf((float)most * (256.0f / 12.0f)) + 1.01f) : (1 << 28);
-    return wave_max(rows);
-}
-
 // ------------------------------------------------------------------ L-phase
 //
 // A wave covers 64 consecutive positions of one simulation and one segment
@@ -218,10 +172,11 @@ struct ShWave {
 // What bounds it: HBM in large batches (256 simulations: 0.73 ms for 3.56 GB algorithmic, 3.8 GB real = 5.2 TB/s against
 // 6.1 for a copy), its own instructions and the chain table entry -> simulation -> rows in small ones. The row
 // control is scalar, loads take any row (clamped) instead of testing each lane, the ring's slots keep
-// their registers and most rotations take the short sines (ShAngle): about 110 vector instructions per two rows
-// instead of 330. us per step: 250 x 100 16.1 -> 14.5, 200 x 1000 with data every step 24.4 -> 22.2; 256-simulation
-// L-phase 0.748 -> 0.730 ms, with data every step the whole step 1.739 -> 1.687. 4 waves per SIMD (128 VGPRs,
-// 4 spilled): 0.761.
+// their registers. 3 waves per SIMD: the fourth, which 119 VGPRs would allow, takes cache lines from the halo
+// rows (256 simulations: L-phase 0.760 ms with 4, 0.742 with 3; 5 iterations of prefetch 0.744). Every pair takes a
+// sine and cosine of its own: the addition theorem from those of theta / 2 was faster (0.730 ms; 250 x 100 12.9
+// us per step instead of 14.3) but rounds differently, and the norm in the largest l after a pulse is what rounding
+// leaves of amplitudes that cancel (values of 1e-49 moved by 1e-3).
 //
 // BY_L: the instance that can also reduce the norm in every l (launched only
 // while some simulation asks for it: the reductions cost registers).
@@ -232,7 +187,8 @@ struct ShWave {
 // rotation is the real one.
 // counters: the simulations again, for the step counter's store (a pointer of its own as in ShObs).
 template <bool BY_L, bool VEL>
-__global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, const ShWave* __restrict__ waves,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_sh_lphase(ShSim* __restrict__ sims, const ShWave* __restrict__ waves,
                                                    int n_waves, const double* __restrict__ cl, int end_only,
                                                    ShSim* counters) {
     constexpr int PF = 4;  // prefetch depth in iterations (2 rows each), and the unrolling of the row loop
@@ -272,12 +228,9 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
     const int q = __builtin_amdgcn_readfirstlane((j & 1) & (L & 1));
     const double rq = ld1(S.tab, SH_RQ * npad + p);
     const double mk = ld1(S.tab, SH_MASK * npad + p);
-    const ShAngle<VEL> a_end(do_end ? ld1(S.fs, n - 1) * rq : 0.0);
-    const ShAngle<VEL> a_start(do_start ? ld1(S.fs, n) * rq : 0.0);
-    const ShAngle<VEL> a_sum(a_end, a_start);
-    // rows from which every lane of the wave may take the short form of the sines
-    const int l_short = sh_short_rows<VEL>(a_end, a_start, a_sum);
-    auto is_short = [=](int l) { return l >= l_short && l + 1 < L; };
+    const double f_end = do_end ? ld1(S.fs, n - 1) * rq : 0.0;
+    const double f_start = do_start ? ld1(S.fs, n) * rq : 0.0;
+    const double f_sum = f_end + f_start;
     const double2* __restrict__ const gin = sh_state(S, n);
     double2* __restrict__ const gout = sh_state(S, n + 1);
     // Output row r depends on input rows up to r + 3, so rows from hi + 3 on (which the prefetch ring would
@@ -319,12 +272,12 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
 
         // stage 1: O_end on (v0-1, v0)
         double2 s1m = carry_u, s10 = u0;
-        if (do_end) a_end.rotate(c_m1, is_short(le + 1), s1m, s10);
+        if (do_end) sh_rotate<VEL>(f_end * c_m1, s1m, s10);
         // stage 2: E_end on (v0-2, v0-1), mask; stage 3: E_start on the same pair
         double2 s2a = carry_s1, s2b = s1m;
         if (both && !observe) {
             // E_end and E_start as one rotation (the mask, a function of r only, commutes with both)
-            a_sum.rotate(c_m2, is_short(le), s2a, s2b);
+            sh_rotate<VEL>(f_sum * c_m2, s2a, s2b);
             s2a = cscale(mk, s2a);
             s2b = cscale(mk, s2b);
         } else {
@@ -336,15 +289,15 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
             double2 oa = s2a, ob = s2b;  // the observed rows: g after step n
             if (both) {
                 if (by_l || per_row) {
-                    a_end.rotate(c_m2, is_short(le), oa, ob);
+                    sh_rotate<VEL>(f_end * c_m2, oa, ob);
                     oa = cscale(mk, oa);
                     ob = cscale(mk, ob);
                 }
-                a_sum.rotate(c_m2, is_short(le), s2a, s2b);
+                sh_rotate<VEL>(f_sum * c_m2, s2a, s2b);
                 s2a = cscale(mk, s2a);
                 s2b = cscale(mk, s2b);
             } else if (do_end) {
-                a_end.rotate(c_m2, is_short(le), s2a, s2b);
+                sh_rotate<VEL>(f_end * c_m2, s2a, s2b);
                 s2a = cscale(mk, s2a);
                 s2b = cscale(mk, s2b);
                 oa = s2a;
@@ -383,11 +336,11 @@ __global__ void __launch_bounds__(256) k_sh_lphase(ShSim* __restrict__ sims, con
                     if (le + 1 >= lo && le + 1 < hi) part_l[(size_t)(le + 1) * wpl + wcol] = rb;
                 }
             }
-            if (!both && do_start) a_start.rotate(c_m2, is_short(le), s2a, s2b);
+            if (!both && do_start) sh_rotate<VEL>(f_start * c_m2, s2a, s2b);
         }
         // stage 4: O_start on (v0-3, v0-2)
         double2 o_a = carry_s3, o_b = s2a;
-        if (do_start) a_start.rotate(c_m3, is_short(le - 1), o_a, o_b);
+        if (do_start) sh_rotate<VEL>(f_start * c_m3, o_a, o_b);
         const int lo_row = le - 1;
         if (live) {
             if (lo_row >= lo && lo_row < hi) st2s(gout + (size_t)lo_row * npad, (unsigned)p, o_a);
@@ -530,7 +483,7 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 // symmetric tridiagonal: diagonal s_n (T_j + l(l+1) U_j [+ corr0 at l = 0,
 // j = 0]), off-diagonals s_n A_{j-1}, s_n A_j (mesh_operators.py:889-928,
 // 244-269). One workgroup of P threads per line, M (= m) rows per thread,
-// solved by cn_symmetric (velocity gauge: cn_implicit_lowreg), which keeps two complex values per row between
+// solved by cn_implicit_lowreg, which keeps two complex values per row between
 // its passes and re-reads the (L2-resident) coefficient tables instead of
 // holding them, so WPE waves fit per SIMD; that occupancy hides the HBM
 // latency of the line loads. Two algebraically equal forms:
@@ -543,9 +496,7 @@ __device__ __forceinline__ void cn_line_finish(double2 (&x)[M], double2* __restr
 //    from memory at the end (CN_CAYLEY_MEM).
 
 // lds: 3 * P + kRedScratch double2, then M * P for CN_CAYLEY_LDS. n: the step under way.
-// VEL: a velocity-gauge line. A template parameter, not S.vel: with both solvers in one kernel m = 8 spilled 56
-// registers at 4 waves per SIMD and m = 16 kept 326, one wave per SIMD.
-template <int M, int FORM, bool VEL>
+template <int M, int FORM>
 __device__ __forceinline__ void sh_rphase_line(const ShSim& S, const int n, const int l, double2* __restrict__ lds) {
     const int P = S.P, npad = S.npad;
     const int k = threadIdx.x;
@@ -579,7 +530,7 @@ __device__ __forceinline__ void sh_rphase_line(const ShSim& S, const int n, cons
         const double U = (j < nr) ? cu * tdse_rcp(r * r) : 0.0;
         return sn * (fma(ll1, U, T) + (i == 0 ? c0 : 0.0));
     };
-    auto general = [&](auto expl, const double2 xl, const double2 xr) {
+    auto solve = [&](auto expl, const double2 xl, const double2 xr) {
         double carry = a_left;  // A_{j-1} of the next row (pass 1 visits rows in order)
         auto coef = [&](int i, double& hm, double& h, double& hp) {
             const double2 tv = ld2(TA, (size_t)i * P);
@@ -604,25 +555,10 @@ __device__ __forceinline__ void sh_rphase_line(const ShSim& S, const int n, cons
         };
         cn_implicit_lowreg<M, decltype(coef), decltype(coef2), decltype(expl)::value>(x, k, P, coef, coef2, lds, xl, xr);
     };
-    auto symmetric = [&](auto expl, const double2 xl, const double2 xr) {
-        auto coef = [&](int i, double& h, double& o) {
-            const double2 tv = ld2(TA, (size_t)i * P);
-            h = diag(i, tv.x, k);
-            o = sn * tv.y;
-        };
-        const double* AN = S.tab + SH_AN * npad + k;
-        auto off = [&](int i) {
-            const double* A2 = AN;
-            asm volatile("" : "+v"(A2));  // read again, as above
-            return sn * ld1(A2, (size_t)i * P);
-        };
-        cn_symmetric<M, decltype(expl)::value, 1>(x, k, P, sn * a_left, coef, off, lds, xl, xr);
-    };
-    if constexpr (VEL) cn_line_finish<M, FORM, 1>(x, gl, k, P, lds, general, 0, P, !pad);
-    else cn_line_finish<M, FORM, 1>(x, gl, k, P, lds, symmetric, 0, P, !pad);
+    cn_line_finish<M, FORM, 1>(x, gl, k, P, lds, solve, 0, P, !pad);
 }
 
-template <int M, int MAXT, int WPE, int FORM, bool VEL>
+template <int M, int MAXT, int WPE, int FORM>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
 k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, ShObs obs) {
     extern __shared__ double2 lds[];
@@ -637,7 +573,7 @@ k_sh_rphase(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_line
     const ShSim& S = sims[lt.x];
     const int n = S.rstep;
     if (!S.active || n >= S.N) return;  // uniform across the block
-    sh_rphase_line<M, FORM, VEL>(S, n, lt.y, lds);
+    sh_rphase_line<M, FORM>(S, n, lt.y, lds);
 }
 
 // ------------------------------------------------------------------ velocity gauge: h2
@@ -1224,9 +1160,9 @@ __device__ __forceinline__ void sh_by_rows(const int m, F&& f) {
     }
 }
 
-// The Crank-Nicolson solves of a split-operator step of one gauge: single lines and, with VEL, odd l-pairs.
-template <bool VEL>
-__global__ void __launch_bounds__(VEL ? 2 * kAnyP : kAnyP)
+// The Crank-Nicolson solves of a split-operator step: single lines and, with PAIRS, velocity-gauge odd l-pairs.
+template <bool PAIRS>
+__global__ void __launch_bounds__(PAIRS ? 2 * kAnyP : kAnyP)
 k_sh_solve_any(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_lines, const double* __restrict__ cl,
                ShObs obs) {
     extern __shared__ double2 lds[];
@@ -1240,14 +1176,14 @@ k_sh_solve_any(ShSim* __restrict__ sims, const int2* __restrict__ lines, int n_l
     const ShSim& S = sims[lt.x];
     const int n = S.rstep;
     if (!S.active || n >= S.N) return;
-    if (VEL && (lt.y & kAnyPair)) {
+    if (PAIRS && (lt.y & kAnyPair)) {
         if ((int)threadIdx.x >= 2 * S.P) return;
         sh_by_rows(S.m, [&](auto m) { sh_vpair_lines<decltype(m)::value>(S, n, lt.y & (kAnyPair - 1), cl, lds); });
     } else {
         if ((int)threadIdx.x >= S.P) return;
         sh_by_rows(S.m, [&](auto m) {
             constexpr int M = decltype(m)::value;
-            sh_rphase_line<M, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS), VEL>(S, n, lt.y, lds);
+            sh_rphase_line<M, (M >= 10 ? CN_EXPLICIT : CN_CAYLEY_LDS)>(S, n, lt.y, lds);
         });
     }
 }

@@ -1,6 +1,6 @@
 """
-The Crank-Nicolson solver of symmetric lines against the oracle for every rows-per-thread instance, in the length gauge
-(SH) and on a Line: with the last row at each place it can have in its thread (first, last but one, last), and with no
+The Crank-Nicolson solvers against the oracle for every rows-per-thread instance, on the radial lines of the length
+gauge (SH) and on a Line: with the last row at each place it can have in its thread (first, last but one, last), and with no
 padding row at all.
 """
 import pytest
