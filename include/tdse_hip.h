@@ -254,7 +254,7 @@ int tdse_download(tdse_ctx *ctx, int32_t kind, int32_t slot, double *g, double *
  * The wavefunction in the reference's own order, reordered on the device: SH
  * l_bound * r_points, Line z_points, Cyl z_points * rho_points complex doubles.
  * tdse_download_g copies it to the host; tdse_upload_g is tdse_upload_state for
- * that order (padding positions keep their zeros). Replaces reading and
+ * that order, with zeros at the padding positions. Replaces reading and
  * assigning sim.mesh.g (sims.py:255-346).
  */
 int tdse_download_g(tdse_ctx *ctx, int32_t kind, int32_t slot, double *g);

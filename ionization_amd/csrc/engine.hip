@@ -1080,20 +1080,46 @@ hipError_t launch_tdma(tdse_ctx* ctx, const double2* a, const double2* b, const 
 // row, chunk layout P x m), or (jz, r) of a cylinder (cyl_at), rows row0 .. row0 + rows - 1. One thread per
 // natural element, the natural side unit-stride. The host's own reordering (a NumPy gather and scatter over the padded
 // copy) took 0.2 s for 15 M points, more than a third of a 2000-step run of them.
+// After them, one thread per padding position of `pads` (null: none) writes its zero: the zero couplings of
+// padding rows keep zeros, but not against a state that held a NaN or an infinity (0 * NaN), which
+// the solves carry into every padding row that shares a line with it.
 struct NaturalMap {
     int n, P, m, npad;  // points per natural row; chunk layout and padded length of the permuted index
-    int cyl;            // the row index (z), not the column (rho), is the permuted one
+    int rows;           // natural rows
+    int rpad;           // cylinder: padded rho rows; else 0. The row index (z), not the column (rho), is then permuted
+    __device__ int position(int j) const { return (j % m) * P + j / m; }
+    __host__ __device__ int64_t padding() const {
+        return rpad ? (int64_t)rpad * npad - (int64_t)rows * n : (int64_t)rows * (npad - n);
+    }
+    // Device element of padding position q < padding(): the indices past the end of the permuted index, then a
+    // cylinder's rho rows past the last for the rest.
+    __device__ size_t padding_at(int64_t q) const {
+        const int over = npad - (rpad ? rows : n);
+        if (!rpad) return (size_t)(q / over) * npad + position(n + (int)(q % over));
+        const int64_t first = (int64_t)rpad * over;
+        if (q < first) return cyl_at((int)(q / over), position(rows + (int)(q % over)), npad);
+        return cyl_at(n + (int)((q - first) / rows), position((int)((q - first) % rows)), npad);
+    }
+};
+struct PaddedStates {
+    double2 *a = nullptr, *b = nullptr;
 };
 template <bool TO_NATURAL>
 __global__ void __launch_bounds__(256) k_natural(double2* __restrict__ g, double2* __restrict__ nat, NaturalMap map,
-                                                 int64_t row0, int64_t rows) {
+                                                 int64_t row0, int64_t rows, PaddedStates pads) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * map.n) return;
+    if (i >= rows * map.n) {
+        const int64_t q = i - rows * map.n;
+        if (TO_NATURAL || q >= map.padding()) return;
+        const size_t at = map.padding_at(q);
+        if (pads.a) st2(pads.a, at, cmk(0.0, 0.0));
+        if (pads.b) st2(pads.b, at, cmk(0.0, 0.0));
+        return;
+    }
     const int64_t row = row0 + i / map.n;
     const int col = (int)(i % map.n);
-    const int j = map.cyl ? (int)row : col;
-    const int p = (j % map.m) * map.P + j / map.m;
-    const size_t at = map.cyl ? cyl_at(col, p, map.npad) : (size_t)row * map.npad + p;
+    const int p = map.position(map.rpad ? (int)row : col);
+    const size_t at = map.rpad ? cyl_at(col, p, map.npad) : (size_t)row * map.npad + p;
     if (TO_NATURAL) st2(nat, (size_t)i, ld2(g, at));
     else st2(g, at, ld2(nat, (size_t)i));
 }
@@ -1102,7 +1128,8 @@ __global__ void __launch_bounds__(256) k_natural(double2* __restrict__ g, double
 // all rows at once, or as many as the free pool holds; a full pool takes them through a block of the
 // runtime's own.
 template <bool TO_HOST>
-int move_natural(tdse_ctx* ctx, double2* g, const NaturalMap& map, int64_t rows, double2* host) {
+int move_natural(tdse_ctx* ctx, double2* g, const NaturalMap& map, double2* host, const PaddedStates pads = {}) {
+    const int64_t rows = map.rows;
     const size_t row_bytes = (size_t)map.n * sizeof(double2);
     int64_t chunk = rows;
     void* stage = nullptr;
@@ -1113,11 +1140,12 @@ int move_natural(tdse_ctx* ctx, double2* g, const NaturalMap& map, int64_t rows,
     hipError_t e = hipSuccess;
     for (int64_t r = 0; r < rows && e == hipSuccess; r += chunk) {
         const int64_t k = std::min(chunk, rows - r), count = k * map.n;
-        const dim3 grid((unsigned)((count + 255) / 256));
+        const PaddedStates clear = r + k == rows ? pads : PaddedStates{};  // with the last rows
+        const dim3 grid((unsigned)((count + (clear.a ? map.padding() : 0) + 255) / 256));
         if (!TO_HOST)
             e = hipMemcpyAsync(nat, host + r * map.n, (size_t)k * row_bytes, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_natural<TO_HOST>, grid, dim3(256), 0, ctx->stream, g, nat, map, r, k);
+            hipLaunchKernelGGL(k_natural<TO_HOST>, grid, dim3(256), 0, ctx->stream, g, nat, map, r, k, clear);
             e = hipGetLastError();
         }
         if (TO_HOST && e == hipSuccess)
@@ -1131,25 +1159,22 @@ int move_natural(tdse_ctx* ctx, double2* g, const NaturalMap& map, int64_t rows,
     return e == hipSuccess ? TDSE_OK : fail(ctx, TDSE_ERR_HIP, std::string("wavefunction copy: ") + hipGetErrorString(e));
 }
 
-// The live simulation's map and natural rows; false for a bad kind or slot.
-bool natural_of(const tdse_ctx* ctx, int32_t kind, int32_t slot, NaturalMap* map, int64_t* rows) {
+// The live simulation's map; false for a bad kind or slot.
+bool natural_of(const tdse_ctx* ctx, int32_t kind, int32_t slot, NaturalMap* map) {
     if (slot < 0) return false;
     if (kind == 0 && slot < (int)ctx->sh.size() && ctx->sh[slot].live) {
         const ShSim& S = ctx->sh[slot].dev;
-        *map = NaturalMap{S.n, S.P, S.m, S.npad, 0};
-        *rows = S.L;
+        *map = NaturalMap{S.n, S.P, S.m, S.npad, S.L, 0};
         return true;
     }
     if (kind == 1 && slot < (int)ctx->line.size() && ctx->line[slot].live) {
         const LineSim& S = ctx->line[slot].dev;
-        *map = NaturalMap{S.n, S.P, S.m, S.npad, 0};
-        *rows = 1;
+        *map = NaturalMap{S.n, S.P, S.m, S.npad, 1, 0};
         return true;
     }
     if (kind == 2 && slot < (int)ctx->cyl.size() && ctx->cyl[slot].live) {
         const CylSim& S = ctx->cyl[slot].dev;
-        *map = NaturalMap{S.nr, S.Pz, S.Mz, S.npz, 1};
-        *rows = S.nz;
+        *map = NaturalMap{S.nr, S.Pz, S.Mz, S.npz, S.nz, S.nrpad};
         return true;
     }
     return false;
@@ -1860,8 +1885,7 @@ int tdse_download_g(tdse_ctx* ctx, int32_t kind, int32_t slot, double* g) {
     if (!ctx) return fail(nullptr, TDSE_ERR_ARG, "ctx is NULL");
     if (!g) return fail(ctx, TDSE_ERR_ARG, "g is NULL");
     NaturalMap map;
-    int64_t rows;
-    if (!natural_of(ctx, kind, slot, &map, &rows)) return fail(ctx, TDSE_ERR_ARG, "bad simulation kind or slot");
+    if (!natural_of(ctx, kind, slot, &map)) return fail(ctx, TDSE_ERR_ARG, "bad simulation kind or slot");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     double2* dev = kind == 1 ? ctx->line[slot].dev.g : kind == 2 ? ctx->cyl[slot].dev.g : nullptr;
@@ -1871,7 +1895,7 @@ int tdse_download_g(tdse_ctx* ctx, int32_t kind, int32_t slot, double* g) {
                                hipMemcpyDeviceToHost));
         dev = sh_state(ctx->sh[slot].dev, st);
     }
-    return move_natural<true>(ctx, dev, map, rows, reinterpret_cast<double2*>(g));
+    return move_natural<true>(ctx, dev, map, reinterpret_cast<double2*>(g));
 }
 
 int tdse_download_norm_by_l(tdse_ctx* ctx, int32_t slot, double* out) {
@@ -1890,12 +1914,19 @@ static int upload_state(tdse_ctx* ctx, int32_t kind, int32_t slot, const double*
     if (!ctx) return fail(nullptr, TDSE_ERR_ARG, "ctx is NULL");
     if (!g) return fail(ctx, TDSE_ERR_ARG, "g is NULL");
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    auto copy = [&](double2* dev, size_t count) -> int {
+    // other: the SH mesh's second buffer, whose padding the sweeps read and write as they do dev's
+    auto copy = [&](double2* dev, size_t count, double2* other = nullptr) -> int {
         NaturalMap map;
-        int64_t rows;
-        if (natural && natural_of(ctx, kind, slot, &map, &rows))
-            return move_natural<false>(ctx, dev, map, rows, const_cast<double2*>(reinterpret_cast<const double2*>(g)));
+        if (!natural_of(ctx, kind, slot, &map)) return fail(ctx, TDSE_ERR_ARG, "bad simulation kind or slot");
+        if (natural)
+            return move_natural<false>(ctx, dev, map, const_cast<double2*>(reinterpret_cast<const double2*>(g)),
+                                       PaddedStates{dev, other});
         HIP_TRY(ctx, hipMemcpy(dev, g, count * sizeof(double2), hipMemcpyHostToDevice));
+        if (other && map.padding()) {
+            hipLaunchKernelGGL(k_natural<false>, dim3((unsigned)((map.padding() + 255) / 256)), dim3(256), 0, ctx->stream,
+                               dev, dev, map, int64_t(0), int64_t(0), PaddedStates{other, nullptr});
+            HIP_TRY(ctx, hipGetLastError());
+        }
         return TDSE_OK;
     };
     int rc;
@@ -1903,7 +1934,7 @@ static int upload_state(tdse_ctx* ctx, int32_t kind, int32_t slot, const double*
         if (slot < 0 || slot >= (int)ctx->sh.size() || !ctx->sh[slot].live) return fail(ctx, TDSE_ERR_ARG, "bad SH slot");
         const ShSim& S = ctx->sh[slot].dev;
         if (step < 0 || step > S.N + 1) return fail(ctx, TDSE_ERR_ARG, "step out of range");
-        if ((rc = copy(sh_state(S, step), (size_t)S.L * S.npad))) return rc;
+        if ((rc = copy(sh_state(S, step), (size_t)S.L * S.npad, sh_state(S, step + 1)))) return rc;
         const int st[2] = {step, 1};  // the uploaded g is the reference g after `step` steps
         HIP_TRY(ctx, hipMemcpy(reinterpret_cast<char*>(ctx->d_sh + slot) + offsetof(ShSim, step), &st[0], sizeof(int),
                                hipMemcpyHostToDevice));
