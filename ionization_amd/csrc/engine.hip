@@ -1050,7 +1050,8 @@ double2* device_scratch(int device, hipError_t* err) {
     return g_scratch_ptr[device];
 }
 
-// Thomas solves of n_systems lines (lengths on the host and, as len, on the device). A line gets one wave for
+// Thomas solves of n_systems lines (lengths on the host and, as len, on the device): by one thread each
+// (tdma_by_threads) or by waves. A line then gets one wave for
 // every kTdmaSpan rows, of which those find work whose rows hold a restart (k_tdma_lines); the span
 // grows where that would be more than kTdmaWaves workgroups. A second launch redoes every line as one run if
 // a split line met a value that is not finite.
@@ -1058,8 +1059,16 @@ constexpr int64_t kTdmaSpan = 64, kTdmaWaves = int64_t(1) << 20;
 hipError_t launch_tdma(tdse_ctx* ctx, const double2* a, const double2* b, const double2* c, const double2* d,
                        double2* x, double2* cp, const int64_t* off, const int64_t* len, const int64_t* lengths,
                        int64_t n_systems) {
-    int64_t longest = 1;
-    for (int64_t i = 0; i < n_systems; ++i) longest = std::max(longest, lengths[i]);
+    int64_t longest = 1, rows = 0;
+    for (int64_t i = 0; i < n_systems; ++i) {
+        longest = std::max(longest, lengths[i]);
+        rows += lengths[i];
+    }
+    if (tdma_by_threads(n_systems, rows, longest)) {
+        hipLaunchKernelGGL(k_tdma_threads, dim3((unsigned)((n_systems + TDSE_WAVE - 1) / TDSE_WAVE)), dim3(TDSE_WAVE), 0,
+                           ctx->stream, a, b, c, d, x, cp, off, len, n_systems);
+        return hipGetLastError();
+    }
     const int64_t most = std::max<int64_t>(1, kTdmaWaves / n_systems);  // waves per line
     const int64_t span = std::max(kTdmaSpan, (longest + most - 1) / most);
     const int64_t per_line = (longest + span - 1) / span;

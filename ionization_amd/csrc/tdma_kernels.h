@@ -26,6 +26,9 @@
 //
 // 100 lines of 250 rows flattened to one call (25 000 unknowns), whole call on host arrays: 13.4 ms ->
 // 0.20 ms; the same length without a restart: 5.3 ms.
+//
+// A wave's instruction costs the same for one row as for 64 lines' rows, so lines that fill the chip by
+// themselves are faster with one thread each (k_tdma_threads; tdma_by_threads has the line between the two).
 constexpr int kTdmaTile = TDSE_WAVE;
 
 __device__ __forceinline__ bool tdma_zero(double2 v) { return v.x == 0.0 && v.y == 0.0; }
@@ -50,8 +53,10 @@ __global__ void __launch_bounds__(TDSE_WAVE) k_tdma_lines(
     const double2* __restrict__ d, double2* __restrict__ x, double2* __restrict__ cp,
     const int64_t* __restrict__ off, const int64_t* __restrict__ len, int64_t n_lines, int64_t span,
     int64_t waves_per_line, int redo_pass, int* __restrict__ redo) {
-    const int64_t line = blockIdx.x / waves_per_line, w = blockIdx.x % waves_per_line;
-    if (line >= n_lines || (redo_pass && *redo == 0)) return;
+    // the lines' first waves first, then their second ones: with a line's waves side by side, 8 or 16 of them put all the
+    // first waves, which have the whole line to do where it does not split, on one XCD
+    const int64_t line = blockIdx.x % (unsigned)n_lines, w = blockIdx.x / (unsigned)n_lines;
+    if (w >= waves_per_line || (redo_pass && *redo == 0)) return;
     const int64_t o = off[line], n = len[line];
     if (w * span >= n) return;
     a += o, b += o, c += o, d += o, x += o, cp += o;
@@ -134,4 +139,44 @@ __global__ void __launch_bounds__(TDSE_WAVE) k_tdma_lines(
         }
     }
     if (waves_per_line > 1 && !fine) *redo = 1;  // the same value from every wave
+}
+
+// One thread per line, the same recurrence and bits.
+__global__ void __launch_bounds__(TDSE_WAVE) k_tdma_threads(
+    const double2* __restrict__ a, const double2* __restrict__ b, const double2* __restrict__ c,
+    const double2* __restrict__ d, double2* __restrict__ x, double2* __restrict__ cp,
+    const int64_t* __restrict__ off, const int64_t* __restrict__ len, int64_t n_lines) {
+    const int64_t line = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (line >= n_lines) return;
+    const int64_t o = off[line], n = len[line];
+    double2 cprev = cmk(0.0, 0.0), dprev = cmk(0.0, 0.0);
+    for (int64_t t = 0; t < n; ++t) {
+        const double2 at = t > 0 ? a[o + t] : cmk(0.0, 0.0);
+        const double2 ct = t + 1 < n ? c[o + t] : cmk(0.0, 0.0);
+        const double2 r = crecip(csub(b[o + t], cmul(at, cprev)));
+        dprev = cmul(csub(d[o + t], cmul(at, dprev)), r);
+        cprev = cmul(ct, r);
+        x[o + t] = dprev;
+        cp[o + t] = cprev;
+    }
+    double2 xn = dprev;
+    for (int64_t t = n - 2; t >= 0; --t) {
+        xn = csub(x[o + t], cmul(cp[o + t], xn));
+        x[o + t] = xn;
+    }
+}
+
+// Whether lines are solved by one thread each: when a wave for every line would take longer to issue (about 1.1 ns
+// for its workgroup and 0.092 ns for each row, over the whole chip) than the longest line takes as one thread's
+// chain (850 ns a row). Past 64 K lines the threads' rows no longer stay in the L2s (each keeps a 128 B line
+// of five arrays in use), and waves are faster again from 16 rows on. Device us, threads / waves:
+//   lines x rows    1024 x 4    4096 x 8    4096 x 16    8192 x 32   8192 x 250   32768 x 32   65536 x 8   65536 x 32
+//                  4.6 / 5.5   8.2 / 9.2  14.4 / 12.6    28 / 32     236 / 230     96 / 102     50 / 79    226 / 201
+//   lines x rows   1024 x 100  4096 x 100  16384 x 100  16384 x 1000  65536 x 1   262144 x 4  262144 x 64
+//                   67 / 26     84 / 57     100 / 168   1075 / 1550    3.5 / 77    61 / 289   2177 / 1460
+// A launch holds fewer than 2^32 threads: past 2^25 lines it is always threads.
+inline bool tdma_by_threads(int64_t n_lines, int64_t rows, int64_t longest) {
+    if (n_lines >= int64_t(1) << 25) return true;
+    if (n_lines >= int64_t(1) << 16 && rows >= 16 * n_lines) return false;
+    return 850.0 * (double)longest <= 1.1 * (double)n_lines + 0.092 * (double)rows;
 }
