@@ -293,14 +293,25 @@ int cn_form(int M, int P);
 size_t vpair_lds_bytes(int M, int P);
 size_t adi_lds_bytes(int P);
 
-// Whether the layouts of a set of lines share one launch per sweep: more than one of them, none past kAnyP threads,
-// and a batch small enough that the launches and their forks and joins cost more than the deepest tile's
-// occupancy does. Measured (us per step, one launch / a launch for each layout): 32 length-gauge simulations of 15 M
-// points 228 / 239, the 256 of 111 M 1689 / 1579; velocity gauge 4.7 M 194 / 275, 111 M 4334 / 3500;
-// ADI 4.2 M 109 / 143, 111 M 2441 / 2024. Between them the gain falls linearly with the points: the lines below are near zero.
+// Whether the layouts of a set of lines share one launch per sweep (any_layouts): none past kAnyP threads, a batch of
+// at most 24 M points (12 M with velocity-gauge pairs, counted as half their points, or ADI's three sweeps), and
+// workgroups that lose little by it. What a shared launch saves are the other launches with their forks and joins, 10
+// to 50 us a step; what it costs is occupancy: every workgroup takes the threads and the LDS of the deepest
+// line, and the registers of 2 waves per SIMD. AnyCost adds up, over the workgroups, the share of a CU that each takes there
+// beyond its share in its layout's own launch: CU-rounds lost. In the length gauge the waves past a line's threads
+// leave at once and count half. One launch against a launch for each layout was faster in 170 batches while
+// the loss was below about 3 rounds (length gauge), 0.4 per layout and 0.4 more (velocity gauge, whose chains have more
+// launches each) and 13.5 (ADI, r-lines and l-groups together); a rule by points alone took the slower one by up to a
+// factor of 2.5. us per step, one launch / one for each layout, and the rounds lost:
+//   length-gauge simulations of 500 to 4000 radial points    4 M points   86 / 106 (0.8)    16 M  298 / 279 (4.5)
+//   velocity-gauge ones                                      4 M         206 / 256 (2.7)     9 M  443 / 375 (8)
+//   a 4000 x 50 mesh beside 250 x 50 ones, length gauge     50 of them    35 /  41 (2.4)    200    94 /  77 (9.8)
+//   the same, velocity gauge                                10            58 /  76 (0.9)    200   303 / 144 (18)
+//   the same, ADI                                           50            59 /  72 (6.4)    200   157 / 105 (24)
 using Layouts = std::map<std::pair<int, int>, std::vector<int2>>;  // (rows, chunks) -> lines
 constexpr int64_t kAnyPoints = int64_t(24) << 20;       // single lines only
 constexpr int64_t kAnyPointsMore = int64_t(12) << 20;   // with velocity-gauge pairs, or ADI's three sweeps
+constexpr double kAnyLost = 3.0, kAnyLostPairs = 0.4, kAnyLostAdi = 13.2;
 bool any_layouts(const Layouts& lines, const Layouts& pairs, int64_t limit) {
     int64_t points = 0;
     for (const Layouts* m : {&lines, &pairs})
@@ -308,34 +319,76 @@ bool any_layouts(const Layouts& lines, const Layouts& pairs, int64_t limit) {
             if (kv.first.second > kAnyP) return false;
             points += (int64_t)kv.second.size() * kv.first.first * kv.first.second;
         }
-    return lines.size() + pairs.size() > 1 && points <= limit;
+    return points <= limit;
 }
+struct AnyCost {
+    size_t lds;     // of the shared launch
+    double waves;   // of its workgroups
+    double lost = 0.0;
+    static double share(size_t lds, double waves, int per_simd) {
+        return std::max((double)lds / (160 << 10), waves / (4 * per_simd));
+    }
+    // count workgroups of a layout whose own launch has own_lds, own_waves and rows per thread M;
+    // early: the part of the surplus waves' share that they give back by leaving
+    void add(size_t count, size_t own_lds, double own_waves, int M, double early = 0.0) {
+        const int per_simd = M <= 8 ? 4 : M == 10 ? 3 : 2;  // as launched (launch_rphase, launch_adi_lp)
+        lost += (double)count * (share(lds, waves - early * (waves - own_waves), 2) - share(own_lds, own_waves, per_simd));
+    }
+};
 
 // The single-launch tables of the split-operator and ADI simulations (longest lines first).
 int build_any(tdse_ctx* ctx, const Layouts& lines, const Layouts (&vpairs)[2], const Layouts& fpairs,
               const Layouts& adi, const Layouts& adi_groups) {
     std::vector<int2> solve, pairs, al, ag;
     int rc;
-    // pairs count half their points (one entry for two rows)
-    ctx->any_sh = any_layouts(lines, fpairs, fpairs.empty() ? kAnyPoints : kAnyPointsMore / 2);
-    ctx->any_adi = any_layouts(adi, adi_groups, kAnyPointsMore) && ctx->adi_waves.count == 0;
+    ctx->any_sh = lines.size() + fpairs.size() > 1 &&
+                  any_layouts(lines, fpairs, fpairs.empty() ? kAnyPoints : kAnyPointsMore / 2);
+    // one layout in each of ADI's sweeps: nothing to share
+    ctx->any_adi = (adi.size() > 1 || adi_groups.size() > 1) && any_layouts(adi, adi_groups, kAnyPointsMore) &&
+                   ctx->adi_waves.count == 0;
     ctx->any_threads = ctx->any_pair_threads = ctx->any_adi_threads = 0;
     ctx->any_lds = ctx->any_adi_lds = 0;
     ctx->any_has_pairs = false;
+    for (auto& kv : fpairs) {
+        ctx->any_threads = std::max(ctx->any_threads, 2 * kv.first.second);
+        ctx->any_lds = std::max(ctx->any_lds, vpair_lds_bytes(kv.first.first, kv.first.second));
+    }
+    for (auto& kv : lines) {
+        const int M = kv.first.first, P = kv.first.second;
+        ctx->any_threads = std::max(ctx->any_threads, P);
+        ctx->any_lds = std::max(ctx->any_lds, cn_lds_bytes(M, P, cn_form(M, P)));
+    }
+    if (ctx->any_sh) {
+        AnyCost cost{ctx->any_lds, (double)ctx->any_threads / TDSE_WAVE};
+        for (auto& kv : fpairs) {
+            const int M = kv.first.first, P = kv.first.second;
+            cost.add(kv.second.size(), vpair_lds_bytes(M, P), 2.0 * P / TDSE_WAVE, M);
+        }
+        for (auto& kv : lines) {
+            const int M = kv.first.first, P = kv.first.second;
+            cost.add(kv.second.size(), cn_lds_bytes(M, P, cn_form(M, P)), (double)P / TDSE_WAVE, M, fpairs.empty() ? 0.5 : 0.0);
+        }
+        const double most = fpairs.empty() ? kAnyLost : kAnyLostPairs * (1.0 + (double)lines.size());
+        ctx->any_sh = cost.lost <= most * ctx->cus;
+    }
+    for (auto& kv : adi) {
+        ctx->any_adi_threads = std::max(ctx->any_adi_threads, kv.first.second);
+        ctx->any_adi_lds = std::max(ctx->any_adi_lds, adi_lds_bytes(kv.first.second));
+    }
+    if (ctx->any_adi) {
+        AnyCost r{ctx->any_adi_lds, (double)ctx->any_adi_threads / TDSE_WAVE};
+        for (auto& kv : adi) r.add(kv.second.size(), adi_lds_bytes(kv.first.second), (double)kv.first.second / TDSE_WAVE, kv.first.first);
+        const size_t group_lds = adi_lds_bytes(kAdiChunks * kAdiLanes);
+        AnyCost l{group_lds, (double)(kAdiChunks * kAdiLanes) / TDSE_WAVE};
+        for (auto& kv : adi_groups) l.add(kv.second.size(), group_lds, l.waves, kv.first.first);
+        ctx->any_adi = r.lost + l.lost <= kAnyLostAdi * ctx->cus;
+    }
     if (ctx->any_sh) {
         for (auto it = fpairs.rbegin(); it != fpairs.rend(); ++it) {
-            const int M = it->first.first, P = it->first.second;
             for (const int2& e : it->second) solve.push_back(make_int2(e.x, e.y | kAnyPair));
             ctx->any_has_pairs = true;
-            ctx->any_threads = std::max(ctx->any_threads, 2 * P);
-            ctx->any_lds = std::max(ctx->any_lds, vpair_lds_bytes(M, P));
         }
-        for (auto it = lines.rbegin(); it != lines.rend(); ++it) {
-            const int M = it->first.first, P = it->first.second;
-            solve.insert(solve.end(), it->second.begin(), it->second.end());
-            ctx->any_threads = std::max(ctx->any_threads, P);
-            ctx->any_lds = std::max(ctx->any_lds, cn_lds_bytes(M, P, cn_form(M, P)));
-        }
+        for (auto it = lines.rbegin(); it != lines.rend(); ++it) solve.insert(solve.end(), it->second.begin(), it->second.end());
         // up to kAnyP threads the odd l-pairs are solved with the lines: only the even ones are left
         for (auto it = vpairs[0].rbegin(); it != vpairs[0].rend(); ++it) {
             pairs.insert(pairs.end(), it->second.begin(), it->second.end());
@@ -343,11 +396,7 @@ int build_any(tdse_ctx* ctx, const Layouts& lines, const Layouts (&vpairs)[2], c
         }
     }
     if (ctx->any_adi) {
-        for (auto it = adi.rbegin(); it != adi.rend(); ++it) {
-            al.insert(al.end(), it->second.begin(), it->second.end());
-            ctx->any_adi_threads = std::max(ctx->any_adi_threads, it->first.second);
-            ctx->any_adi_lds = std::max(ctx->any_adi_lds, adi_lds_bytes(it->first.second));
-        }
+        for (auto it = adi.rbegin(); it != adi.rend(); ++it) al.insert(al.end(), it->second.begin(), it->second.end());
         for (auto it = adi_groups.rbegin(); it != adi_groups.rend(); ++it)
             ag.insert(ag.end(), it->second.begin(), it->second.end());
     }
