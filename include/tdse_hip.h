@@ -82,7 +82,7 @@ int tdse_tdma_batched(tdse_ctx *ctx, const double *sub, const double *diag, cons
  * Allocation-free form of tdse_tdma_batched. No counterpart in the reference:
  * it is for callers that cannot allocate device memory (tight serving loops,
  * code that forbids hipMalloc). sub, diag, sup, d and x are DEVICE arrays of
- * `total` complex128 each, owned by the caller (x is written); offsets and
+ * `total` complex128 each, owned by the caller (x is written, and may be d); offsets and
  * lengths are host arrays of n_systems, every system inside [0, total). The
  * Thomas scratch (primed super-diagonal) and the staged offsets / lengths live
  * in a static device array of the library, one per GPU, so the call allocates

@@ -1103,11 +1103,12 @@ double2* device_scratch(int device, hipError_t* err) {
 // (tdma_by_threads) or by waves. A line then gets one wave for
 // every kTdmaSpan rows, of which those find work whose rows hold a restart (k_tdma_lines); the span
 // grows where that would be more than kTdmaWaves workgroups. A second launch redoes every line as one run if
-// a split line met a value that is not finite.
+// a split line met a value that is not finite. in_place: x overlaps an input, which a second launch would find
+// overwritten and another wave's search for restarts may: lines are then not split.
 constexpr int64_t kTdmaSpan = 64, kTdmaWaves = int64_t(1) << 20;
 hipError_t launch_tdma(tdse_ctx* ctx, const double2* a, const double2* b, const double2* c, const double2* d,
                        double2* x, double2* cp, const int64_t* off, const int64_t* len, const int64_t* lengths,
-                       int64_t n_systems) {
+                       int64_t n_systems, bool in_place) {
     int64_t longest = 1, rows = 0;
     for (int64_t i = 0; i < n_systems; ++i) {
         longest = std::max(longest, lengths[i]);
@@ -1119,7 +1120,7 @@ hipError_t launch_tdma(tdse_ctx* ctx, const double2* a, const double2* b, const 
         return hipGetLastError();
     }
     const int64_t most = std::max<int64_t>(1, kTdmaWaves / n_systems);  // waves per line
-    const int64_t span = std::max(kTdmaSpan, (longest + most - 1) / most);
+    const int64_t span = in_place ? longest : std::max(kTdmaSpan, (longest + most - 1) / most);
     const int64_t per_line = (longest + span - 1) / span;
     int* redo = ctx->d_ctl + 1;
     hipError_t e = hipSuccess;
@@ -1413,7 +1414,7 @@ int tdse_tdma_batched(tdse_ctx* ctx, const double* sub, const double* diag, cons
         free_blocks(ctx, blocks);
         return rc;
     }
-    hipError_t e = launch_tdma(ctx, da, db, dc, dd, dx, dcp, doff, dlen, lengths, n_systems);
+    hipError_t e = launch_tdma(ctx, da, db, dc, dd, dx, dcp, doff, dlen, lengths, n_systems, false);
     if (e == hipSuccess) e = hipMemcpyAsync(x, dx, n * sizeof(double2), hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->stream);
@@ -1456,9 +1457,11 @@ int tdse_tdma_batched_noalloc(tdse_ctx* ctx, const double* sub, const double* di
     const size_t nb = (size_t)n_systems * sizeof(int64_t);
     HIP_TRY(ctx, hipMemcpyAsync(doff, offsets, nb, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(dlen, lengths, nb, hipMemcpyHostToDevice, ctx->stream));
+    bool in_place = false;
+    for (const double* input : {sub, diag, sup, d}) in_place = in_place || (x < input + 2 * total && input < x + 2 * total);
     HIP_TRY(ctx, launch_tdma(ctx, reinterpret_cast<const double2*>(sub), reinterpret_cast<const double2*>(diag),
                              reinterpret_cast<const double2*>(sup), reinterpret_cast<const double2*>(d),
-                             reinterpret_cast<double2*>(x), cp, doff, dlen, lengths, n_systems));
+                             reinterpret_cast<double2*>(x), cp, doff, dlen, lengths, n_systems, in_place));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return TDSE_OK;
 }
