@@ -1361,6 +1361,7 @@ int tdse_copy_probe(tdse_ctx* ctx, size_t bytes, int launches, double* avg_ms) {
     if (!ctx) return fail(nullptr, TDSE_ERR_ARG, "ctx is NULL");
     if (bytes == 0 || bytes % sizeof(double2) != 0 || launches < 1)
         return fail(ctx, TDSE_ERR_ARG, "tdse_copy_probe: bytes must be a positive multiple of 16, launches >= 1");
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
     std::vector<void*> blocks;
     double2 *src, *dst;
     const size_t n = bytes / sizeof(double2);
@@ -1397,6 +1398,7 @@ int tdse_tdma_batched(tdse_ctx* ctx, const double* sub, const double* diag, cons
         if (lengths[i] < 1 || offsets[i] < 0) return fail(ctx, TDSE_ERR_ARG, "tdse_tdma_batched: bad system extent");
         total = std::max(total, offsets[i] + lengths[i]);
     }
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
     std::vector<void*> blocks;
     double2 *da, *db, *dc, *dd, *dx, *dcp;
     int64_t *doff, *dlen;
@@ -1974,6 +1976,7 @@ int tdse_download_norm_by_l(tdse_ctx* ctx, int32_t slot, double* out) {
 static int upload_state(tdse_ctx* ctx, int32_t kind, int32_t slot, const double* g, int32_t step, bool natural) {
     if (!ctx) return fail(nullptr, TDSE_ERR_ARG, "ctx is NULL");
     if (!g) return fail(ctx, TDSE_ERR_ARG, "g is NULL");
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     // other: the SH mesh's second buffer, whose padding the sweeps read and write as they do dev's
     auto copy = [&](double2* dev, size_t count, double2* other = nullptr) -> int {
