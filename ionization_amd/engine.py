@@ -186,15 +186,18 @@ class CompiledSH:
 
     @property
     def footprint_bytes(self):
-        """Device bytes this simulation holds (two g buffers, tables, snapshots, basis, data)."""
+        """Device bytes this simulation holds (two g buffers, tables, snapshots, norm partials, basis, data)."""
         nd = data_count(self.n_steps, self.store_every)
+        # one partial for every 4 rows (kShPartRows) of 64 positions and one for the last row; each row's own by l
+        partials = self.npad // 64 * (-(-self.l_bound // 4) + 1 + (self.l_bound if self.norm_by_l else 0))
         return int(
             2 * 16 * self.l_bound * self.npad
             + 8 * len(self.tables) * self.npad
-            + 16 * self.n_steps
+            + (24 if self.method == "adi" else 16) * self.n_steps
             + 16 * self.lb * self.npad
-            + 8 * len(self.basis_l) * self.npad
-            + nd * (16 + 16 * max(1, len(self.basis_l)))
+            + 8 * partials
+            + (8 * self.npad + 4) * len(self.basis_l)
+            + nd * (16 + 16 * max(1, len(self.basis_l)) + (8 * self.l_bound if self.norm_by_l else 0))
         )
 
 
