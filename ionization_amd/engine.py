@@ -134,6 +134,16 @@ def from_positions(a: np.ndarray, n: int, P: int, m: int) -> np.ndarray:
     return out
 
 
+def mesh_state(g: np.ndarray, shape: Tuple[int, ...]) -> np.ndarray:
+    """g as a contiguous complex128 array of the mesh's shape; a state of fewer points is extended by zeros."""
+    g = np.asarray(g, dtype=np.complex128)
+    if g.shape != shape and g.ndim == len(shape) and all(have <= want for have, want in zip(g.shape, shape)):
+        out = np.zeros(shape, dtype=np.complex128)
+        out[tuple(slice(0, have) for have in g.shape)] = g
+        return out
+    return np.ascontiguousarray(g).reshape(shape)
+
+
 def data_count(n_steps: int, store_every: int) -> int:
     if store_every >= 1:
         return n_steps // store_every + 1 + (1 if n_steps % store_every else 0)
@@ -813,7 +823,7 @@ class DeviceContext:
         else:
             c = self._sh[slot] if kind == KIND_SH else self._line[slot]
             shape = (c.l_bound, c.r_points) if kind == KIND_SH else (c.z_points,)
-        g = np.ascontiguousarray(g_natural, dtype=np.complex128).reshape(shape)
+        g = mesh_state(g_natural, shape)
         self._check(self._lib.tdse_upload_g(self._ctx, kind, slot, _lib.dptr(g), int(step)))
 
     def materialize(self, kind: int, slot: int):
