@@ -472,7 +472,9 @@ def choose_cyl_layout(z_points: int, rho_points: int, z_rows: Optional[int] = No
     limit). Up to 320 rho points (4, 4): more workgroups and shorter chains, faster
     alone and in batches whatever its padding (one / 16 simulations of 400 x 200:
     15.8 / 42.5 us per step, (8, 4) 18.6 / 43.4, (4, 8) with less padding 17.2 / 43.9;
-    120 x 60: 12.1 / 14.5, 15.7 / 18.1, 13.3 / 14.7). Above, least rho padding, then
+    120 x 60: 12.1 / 14.5, 15.7 / 18.1, 13.3 / 14.7), but (4, 8) up to 32, which it pads to
+    32 where (4, 4) needs 64 (one / 128 / 512 simulations of 300 x 30: 10.7 / 32.9 / 89.7 us,
+    (4, 4) 10.8 / 41.9 / 130.4; meshes of up to 64 z points keep (4, 4)). Above 320, least rho padding, then
     the order of CYL_RHO_SHAPES ((8, 4) ahead of (4, 4): a shorter reduced system,
     four simulations of 2000 x 1000 131 us per step against 164; 1024 x 512 alone / 16:
     27.8 / 119 against 25.8 / 131), without (4, 8): 800 x 400 as 416 rows 25.1 / 125,
@@ -483,7 +485,7 @@ def choose_cyl_layout(z_points: int, rho_points: int, z_rows: Optional[int] = No
     if rho_shape is not None:
         shapes = [tuple(rho_shape)]
     elif rho_points <= 320:
-        shapes = [(4, 4)]
+        shapes = [(4, 8) if rho_points <= 32 and z_points > 64 else (4, 4)]
     else:
         shapes = [shape for shape in CYL_RHO_SHAPES if shape != (4, 8)]
     for pref, (mr, lanes) in enumerate(shapes):
