@@ -111,19 +111,6 @@ __device__ __forceinline__ double wave_sum_last(double v) {
     return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
 
-// Largest of the wave's values (all >= 0), uniform.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp_max(int v) { return max(v, __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, true)); }
-__device__ __forceinline__ int wave_max(int v) {
-    v = dpp_max<0x111, 0xf>(v);
-    v = dpp_max<0x112, 0xf>(v);
-    v = dpp_max<0x114, 0xf>(v);
-    v = dpp_max<0x118, 0xf>(v);
-    v = dpp_max<0x142, 0xa>(v);
-    v = dpp_max<0x143, 0xc>(v);
-    return __builtin_amdgcn_readlane(v, TDSE_WAVE - 1);
-}
-
 // Sum over the 64 lanes of a wave; every lane gets the total.
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll

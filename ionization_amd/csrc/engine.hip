@@ -1588,7 +1588,6 @@ int tdse_sh_add(tdse_ctx* ctx, const tdse_sh_desc* desc, const double* tables, c
     S.out_nl = onl;
     S.fa = dfa;
     S.adi = H.adi ? 1 : 0;
-    S.vel = H.vel ? 1 : 0;
     HIP_TRY(ctx, hipMemcpyAsync(ctx->d_sh + s, &S, sizeof(ShSim), hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // host buffers may be released after return
     H.live = true;

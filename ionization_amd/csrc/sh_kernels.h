@@ -52,7 +52,6 @@ struct ShSim {
     int active;
     int phase;             // 0: g is mid-step (after the R-phase); 1: g is the reference g after `step` steps
     int norm_by_l;         // 1: also reduce the norm of every l at data times
-    int vel;               // 1: velocity gauge (its line solves keep cyclic reduction, reduced_cr)
     int adi;               // 1: AlternatingDirectionImplicit (fs is then zero: the L-phase only masks and observes)
     const double* fa;      // ADI: [N] field times tau ratio per step, E(t_{n+1} + dt/2) tau_n / tau0
     int flags;             // health flags (norm_health), device-updated at data times
