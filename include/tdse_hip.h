@@ -206,7 +206,8 @@ typedef struct {
  * Add one cylindrical simulation. zt: npz doubles (z of every position, 0 for
  * padding); rt: nrpad doubles (rho, 0 for padding); roff: nrpad doubles
  * (rho_prefactor * c(j + 1) between rho j and j + 1, 0 past the line,
- * mesh_operators.py:582-592); fs: N doubles E(t_{n+1}); ts: N doubles
+ * mesh_operators.py:582-592); neither may be NULL, but both are left unread: the
+ * grid and the couplings are formed from the descriptor; fs: N doubles E(t_{n+1}); ts: N doubles
  * tau_n = (t_{n+1} - t_n) / (2 hbar); g0 and basis: nrpad * npz complex each.
  * Replaces MeshSpecification.to_sim() + the first
  * AlternatingDirectionImplicit.evolve (sims.py:46-118, evolution_methods.py:48-77).

@@ -236,7 +236,7 @@ k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, 
 //
 // What bounds it: FP64 issue at 4 waves per SIMD (128 VGPRs). The couplings come from the simulation's table,
 // staged in LDS once per workgroup: formed from m each time, they were a reciprocal square root three times per row
-// and a reciprocal for their ratio, and kept registers busy over the solve. With half the potential in LDS too, the
+// and kept registers busy over the solve. With half the potential in LDS too, the
 // explicit half gained nothing (139.6 us against 140.1 per step of four 2000 x 1000 simulations), so it is formed
 // again. A wave whose points all lie inside the mask's ramp skips it. Padding rows hold zeros, so nothing selects on
 // them. Per step, before and after (with cn_symmetric): one 250 x 100 simulation 18.4 -> 16.0 us, four of 2000 x 1000
@@ -248,7 +248,7 @@ k_cyl_z(CylSim* __restrict__ sims, const int2* __restrict__ pairs, int n_pairs, 
 // PRE (phase 1 only): observables of g at step 0, explicit half of step n.
 enum { CYL_PRE = 0, CYL_MAIN = 1 };
 
-// LDS of the rho-sweep: the solver's rows, the couplings and their ratios, reduction scratch.
+// LDS of the rho-sweep: the solver's rows, the couplings, reduction scratch.
 constexpr size_t cyl_rho_lds_bytes(int M, int LANES, int P) {
     return ((size_t)3 * P * LANES + kRedScratch) * sizeof(double2) +
            ((size_t)M * P + 16) * sizeof(double);

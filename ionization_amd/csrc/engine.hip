@@ -174,15 +174,15 @@ void free_bucket(Bucket& b) {
 // Norm partials along l of one simulation (kShPartRows rows each).
 int sh_parts(int L) { return (L + kShPartRows - 1) / kShPartRows; }
 
-// Rows of an L-phase wave's l-segment: the most (up to kShSegRows) that still give the batch
-// kMinLWaves waves, about four for each SIMD. A wave walks its rows one pair after another, so a
-// small batch's L-phase takes as long as one segment: 64-row segments left one 250 x 100 mesh with
-// 8 waves (38.0 us per step, 28 us of it the L-phase; 8-row segments 15.6, 4-row segments 14.3), one 200 x 1000 mesh
-// with 64 (51.3 -> 23.3 -> 21.8). Long segments re-read fewer halo rows (7 per segment); on 32 simulations of
-// 15 M points 8 / 16 / 32 / 64 rows measured 270 / 260 / 267 / 267 us per step. Segments of 4 rows walk 11
-// rows where those of 8 walk 15, but twice as many of them: only where 8 rows leave fewer waves than there are
-// SIMDs (1 / 2 / 3 / 4 meshes of 200 x 1000, 400 waves each: 8 rows 19.2 / 21.1 / 22.1 / 24.2 us, 4 rows 18.3 / 20.6 /
-// 22.0 / 29.1).
+// Rows of an L-phase wave's l-segment: the most (up to kShSegRows) that still give the batch kMinLWaves waves.
+// A wave walks its rows one pair after another, so a small batch's L-phase takes as long as one segment; long
+// segments re-read fewer halo rows (7 per segment). Segments of 4 rows walk 11 rows where those of 8 walk 15, but
+// twice as many of them: only where 8 rows leave fewer waves than there are SIMDs (1 / 2 / 3 / 4 meshes of 200 x 1000,
+// 400 waves each: 8 rows 19.2 / 21.1 / 22.1 / 24.2 us, 4 rows 18.3 / 20.6 / 22.0 / 29.1). us per step with 4 / 8 / 16 / 32 / 64
+// rows: 250 x 100 14.4 / 15.9 / 18.8 / 23.9 / 30.8, 1000 x 200 21.1 / 22.2 / 24.7 / 30.9 / 38.4; with 8 / 16 / 32 / 64,
+// simulations of 500 to 4000 radial points: 4 M points 95 / 92 / 92 / 99, 13 M 246 / 234 / 237 / 246, 48 M 762 / 697 /
+// 705 / 724. The rule dates from a kernel of 4 waves per SIMD (the present one has 3): from about 4 M points on 16
+// rows would be up to 4 % faster than its choice.
 // `columns` counts, for every live simulation, its 64-position columns times its partials along l.
 constexpr int64_t kMinLWaves = 4096, kMinLWaves8 = 1024;
 int sh_segment_rows(int64_t columns) {
@@ -1757,7 +1757,10 @@ int tdse_cyl_add(tdse_ctx* ctx, const tdse_cyl_desc* desc, const double* zt, con
     const size_t pts = (size_t)S.nrpad * S.npz;
     double2 *g, *oip, *bas = nullptr;
     double *dzt, *droff, *dfs, *dts, *part, *on;
-    std::vector<double> coupling((size_t)S.nrpad, 0.0);  // in the rho-sweep's order, from the descriptor (not rt and roff)
+    // rp c(j + 1) in the rho-sweep's order, from the descriptor (not rt and roff); rounded three times. The same at every
+    // step, a rounding adds up as a phase: after 1000 steps of 250 x 100 the wavefunction is 2.4e-13 from one in long
+    // double with the same prefactors (2.4e-13 too with one rounding; 6.1e-13 when the kernels formed the couplings).
+    std::vector<double> coupling((size_t)S.nrpad, 0.0);
     for (int j = 0; j + 1 < S.nr; ++j) {
         const double m = j + 1;
         coupling[(size_t)(j % Mr) * Cr + j / Mr] = (m * (1.0 / std::sqrt(m * m - 0.25))) * S.rp;

@@ -1138,7 +1138,8 @@ __global__ void __launch_bounds__(kAdiLanes * kAdiChunks) k_sh_adi_lp(ShSim* __r
 // lines of every layout (P <= kAnyP) in one launch: the workgroup has the threads of the longest line in the
 // batch, whole waves past a line's threads leave before any barrier (s_barrier waits for the surviving waves
 // only), and the rows per thread are chosen by a branch. They hold the registers of the deepest
-// tile, 2 waves per SIMD, which is why a large batch keeps a launch for each layout (any_layouts, engine.hip).
+// tile, 2 waves per SIMD (k_sh_adi_lp_any, built for 16 rows, also spills 20 VGPRs), and their workgroups the LDS of the deepest
+// line, which is why large batches and those of many shallow lines keep a launch for each layout (AnyCost, engine.hip).
 // Each line's arithmetic is the layout launch's own. us per step: those 12 velocity-gauge simulations 277 -> 194,
 // 12 ADI ones of 4.2 M points 140 -> 106, three small velocity-gauge meshes 47 -> 31, 32 length-gauge ones of
 // 15 M points 240 -> 228.

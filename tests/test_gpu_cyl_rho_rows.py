@@ -1,8 +1,8 @@
 """
-Where the last row of a cylindrical line can sit, on the device: its coupling to the next row is
-stored like any other (pass 2 of the solver divides by it), so it has to meet a zero row, whether
-that is a padding row of the same thread, of the next one, or none at all. The sizes put it at each
-of these, in the rho- and in the z-sweep; the mask's ramp crosses every one of them.
+Where the last row of a cylindrical line can sit, on the device: followed by a padding row of the same
+thread, of the next one, or by none at all. In the rho-sweep its coupling to the next row is zero; in the
+z-sweep, whose couplings are all alike, the padding rows' pivots are made zero. The sizes put it at each of
+these, in both sweeps; the mask's ramp crosses every one of them.
 """
 import numpy as np
 import pytest
